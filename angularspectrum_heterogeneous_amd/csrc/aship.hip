@@ -17,7 +17,7 @@
 
 #include "../../include/aship.h"
 #include "kernels.h"
-#include "generic.h"
+#include "generic_launch.h"
 #include "learned.h"
 
 using namespace ash;
@@ -74,8 +74,8 @@ int caught_exception() noexcept {
 // Sizes of the FFT kernels; every other size runs the general-size kernels (generic.h).
 bool line_supported(int n) { return n == 64 || n == 128 || n == 192 || n == 256 || n == 384; }
 bool col_supported(int m) { return m == 128 || m == 256 || m == 512 || m == 1024; }
-constexpr int GEN_MAX_LINE = GEN_MAXL;  // general-size line kernels: 2 .. 1024
-constexpr int GEN_MAX_NT = 2048;         // general-length column kernel: 4 .. 2048
+constexpr int GEN_MAX_LINE = 1024;  // general-size line kernels: 2 .. 1024
+constexpr int GEN_MAX_NT = 2048;    // general-length column kernel: 4 .. 2048
 
 // Python's round(): half to even
 long py_round(double v) {
@@ -372,9 +372,23 @@ int build_tables(ash_plan* p) {
   }
   if ((rc = upload(p, twiddles(nX), &p->T.twx))) return rc;
   if ((rc = upload(p, twiddles(nY), &p->T.twy))) return rc;
-  p->T.twgx = p->T.twx;  // the same full-length tables serve the general-size kernels
-  p->T.twgy = p->T.twy;
   if ((rc = upload(p, twiddles(nT), &p->T.twgt))) return rc;
+  // DFT matrices of the axes outside the FFT set, filled on the device
+  auto matrix = [p](int n, const float2* tw, DftMat* m) -> int {
+    *m = dft_matrix_shape(n);
+    const size_t bytes = dft_matrix_bytes(*m);
+    void* a = nullptr;
+    p->allocs.reserve(p->allocs.size() + 1);
+    HIP_TRY(hipMalloc(&a, bytes));
+    p->allocs.push_back(a);
+    p->ws_bytes += (int64_t)bytes;
+    m->A = (const float4*)a;
+    dft_matrix_fill(*m, tw, (float4*)a, nullptr);
+    return ASH_OK;
+  };
+  if (p->gen_x && (rc = matrix(nX, p->T.twx, &p->T.dmx))) return rc;
+  if (p->gen_y && (rc = matrix(nY, p->T.twy, &p->T.dmy))) return rc;
+  if (p->gen_t && (rc = matrix(nT, p->T.twgt, &p->T.dmt))) return rc;
   if (!p->gen_t) {
     // pass-major twiddles of the column transform, [r * Ns + k] = W_{Ns R}^{k r}
     auto radices = [&](bool inv) {
@@ -550,12 +564,10 @@ void launch_col_M(ash_plan* p, const ColDesc& cd, hipStream_t s) {
     default: break;                            \
   }
 
-dim3 gen_grid(const ash_plan* p, int n_line, int n_other) { return dim3(n_other * (p->g.MP / gen_lines(n_line))); }
-
 void xfwd(ash_plan* p, hipStream_t s) {
   ProfScope ps(p, ASH_K_XFWD, s);
   if (p->gen_x) {
-    hipLaunchKernelGGL(k_gx_fwd, gen_grid(p, p->g.nX, p->g.nY), dim3(GNT), 0, s, p->spec, p->T, p->g);
+    gen_xfwd(p->spec, p->T, p->g, s);
     return;
   }
   DISPATCH_L(p->g.nX, launch_xfwd_L<L>(p, s));
@@ -563,7 +575,7 @@ void xfwd(ash_plan* p, hipStream_t s) {
 void ypass(ash_plan* p, const OpDesc& op, hipStream_t s) {
   ProfScope ps(p, ASH_K_YPASS, s);
   if (p->gen_y) {
-    hipLaunchKernelGGL(k_gy_pass, gen_grid(p, p->g.nY, p->g.nX), dim3(GNT), 0, s, p->spec, p->T, p->g, op);
+    gen_ypass(p->spec, p->T, p->g, op, s);
     return;
   }
   DISPATCH_L(p->g.nY, launch_ypass_L<L>(p, op, s));
@@ -571,10 +583,7 @@ void ypass(ash_plan* p, const OpDesc& op, hipStream_t s) {
 void xinv(ash_plan* p, int epi, const EpiDesc& e, hipStream_t s) {
   ProfScope ps(p, ASH_K_XINV, s);
   if (p->gen_x) {
-    const dim3 grid = gen_grid(p, p->g.nX, p->g.nY);
-    if (epi == 0) hipLaunchKernelGGL(k_gx_inv<0>, grid, dim3(GNT), 0, s, p->spec, p->T, p->g, e);
-    else if (epi == 1) hipLaunchKernelGGL(k_gx_inv<1>, grid, dim3(GNT), 0, s, p->spec, p->T, p->g, e);
-    else hipLaunchKernelGGL(k_gx_inv<2>, grid, dim3(GNT), 0, s, p->spec, p->T, p->g, e);
+    gen_xinv(epi, p->spec, p->T, p->g, e, s);
     return;
   }
   if (epi == 0) { DISPATCH_L(p->g.nX, (launch_xinv_L<L, 0>(p, e, s))); }
@@ -590,7 +599,7 @@ void launch_ypower_L(ash_plan* p, hipStream_t s) {
 void ypower(ash_plan* p, hipStream_t s) {
   ProfScope ps(p, ASH_K_YPASS, s);
   if (p->gen_y) {
-    hipLaunchKernelGGL(k_gy_power, gen_grid(p, p->g.nY, p->g.nX), dim3(GNT), 0, s, p->spec, p->T, p->g, p->obl_acc);
+    gen_ypower(p->spec, p->T, p->g, p->obl_acc, s);
     return;
   }
   DISPATCH_L(p->g.nY, launch_ypower_L<L>(p, s));
@@ -598,47 +607,10 @@ void ypower(ash_plan* p, hipStream_t s) {
 void ysa(ash_plan* p, const ScreenDesc& sd, hipStream_t s) {
   ProfScope ps(p, ASH_K_YSA, s);
   if (p->gen_y) {
-    hipLaunchKernelGGL(k_gy_sa, gen_grid(p, p->g.nY, p->g.nX), dim3(GNT), 0, s, p->spec, p->T, p->g, sd);
+    gen_ysa(p->spec, p->T, p->g, sd, s);
     return;
   }
   DISPATCH_L(p->g.nY, launch_ysa_L<L>(p, sd, s));
-}
-
-// General-length column kernel: S real samples per lane, 64 S >= nT.
-int gen_col_samples(int nT) { return nT <= 128 ? 2 : nT <= 256 ? 4 : nT <= 512 ? 8 : nT <= 1024 ? 16 : 32; }
-template <int S, int MODE, int NLK>
-void launch_gcol_SMN(ash_plan* p, const ColDesc& cd, hipStream_t s) {
-  const int ncols = p->g.nX * p->g.nY;
-  const int blocks = std::min((ncols + GC_WPB - 1) / GC_WPB, p->col_grid);
-  hipLaunchKernelGGL((k_gcolumn<S, MODE, NLK>), dim3(blocks), dim3(256), 0, s, p->spec, p->T, p->g, cd);
-}
-template <int S, int MODE>
-void launch_gcol_SM(ash_plan* p, const ColDesc& cd, hipStream_t s) {
-  switch (cd.nl) {
-    case NL_KT: launch_gcol_SMN<S, MODE, NL_KT>(p, cd, s); break;
-    case NL_KT_MINMOD: launch_gcol_SMN<S, MODE, NL_KT_MINMOD>(p, cd, s); break;
-    case NL_RUSANOV: launch_gcol_SMN<S, MODE, NL_RUSANOV>(p, cd, s); break;
-    case NL_TVD: launch_gcol_SMN<S, MODE, NL_TVD>(p, cd, s); break;
-    default: launch_gcol_SMN<S, MODE, NL_NONE>(p, cd, s); break;
-  }
-}
-template <int S>
-void launch_gcol_S(ash_plan* p, const ColDesc& cd, hipStream_t s) {
-  switch (cd.mode) {
-    case COL_LOAD: launch_gcol_SMN<S, COL_LOAD, NL_NONE>(p, cd, s); break;
-    case COL_NL: launch_gcol_SM<S, COL_NL>(p, cd, s); break;
-    case COL_TAPER: launch_gcol_SMN<S, COL_TAPER, NL_NONE>(p, cd, s); break;
-    case COL_FINAL:
-      if (cd.n_src > 0 || cd.smask) launch_gcol_SMN<S, COL_FINAL_SRC, NL_NONE>(p, cd, s);
-      else launch_gcol_SMN<S, COL_FINAL, NL_NONE>(p, cd, s);
-      break;
-    case COL_STORE: launch_gcol_SMN<S, COL_STORE, NL_NONE>(p, cd, s); break;
-    case COL_RAWNL: launch_gcol_SM<S, COL_RAWNL>(p, cd, s); break;
-    case COL_TOREAL: launch_gcol_SMN<S, COL_TOREAL, NL_NONE>(p, cd, s); break;
-    case COL_MAXABS: launch_gcol_SMN<S, COL_MAXABS, NL_NONE>(p, cd, s); break;
-    case COL_TOF: launch_gcol_SMN<S, COL_TOF, NL_NONE>(p, cd, s); break;
-    default: break;
-  }
 }
 
 // Blocks of the final column pass: one resident round (CUs x blocks per CU).
@@ -666,13 +638,7 @@ void column(ash_plan* p, const ColDesc& cd, hipStream_t s) {
                  : cd.mode == COL_FINAL ? ASH_K_COL_FINAL : ASH_K_COL_OTHER;
   ProfScope ps(p, kind, s);
   if (p->gen_t) {
-    switch (gen_col_samples(p->g.nT)) {
-      case 2: launch_gcol_S<2>(p, cd, s); break;
-      case 4: launch_gcol_S<4>(p, cd, s); break;
-      case 8: launch_gcol_S<8>(p, cd, s); break;
-      case 16: launch_gcol_S<16>(p, cd, s); break;
-      default: launch_gcol_S<32>(p, cd, s); break;
-    }
+    gen_column(p->spec, p->T, p->g, cd, s);
     return;
   }
   switch (p->g.M) {
@@ -706,7 +672,7 @@ int nl_kind(const ash_plan* p) {
 bool is_kt(int nl) { return nl == NL_KT || nl == NL_KT_MINMOD; }
 
 int col_blocks(const ash_plan* p, int M) {
-  if (p->gen_t) return std::min((p->g.nX * p->g.nY + GC_WPB - 1) / GC_WPB, p->col_grid);
+  if (p->gen_t) return gen_column_blocks(p->g.nX * p->g.nY);
   const int per_block = M == 128 ? ColCfg<128>::WPB * ColCfg<128>::CPW
                       : M == 256 ? ColCfg<256>::WPB * ColCfg<256>::CPW
                       : M == 512 ? ColCfg<512>::WPB * ColCfg<512>::CPW

@@ -1,268 +1,450 @@
-// General-size kernels: the same sweeps as kernels.h / column.h for grid
-// sizes outside the FFT kernels' set (any line length 2..1024, any nT 4..2048),
-// e.g. the odd and prime grids of the reference's validation scripts.
+// General-size kernels: the same sweeps as kernels.h / column.h for grid sizes
+// outside the FFT kernels' set (any line length 2..1024, any nT 4..2048), e.g.
+// the odd and prime grids of the reference's validation scripts.
 //
-// The transforms are direct DFTs through LDS, O(n^2) per line, with a
-// full-length twiddle table exp(-2 pi i k / n) (FP64-accurate, rounded once)
-// indexed by (j k) mod n, so every twiddle is exact to one rounding.  Each
-// sweep reads and writes the spectrum once, like its FFT counterpart; these
-// kernels trade arithmetic for generality and are not the fast path.
+// The transforms are direct DFTs on the matrix cores (v_mfma_f32_16x16x4_f32:
+// float32 operands and accumulation).  With e_j = x_j + x_{n-j} and
+// o_j = x_j - x_{n-j} (0 <= j <= n/2) a length-n DFT is two real matrix products
+//   C_k = sum_j cos(2 pi j k / n) e_j,   S_k = sum_j sin(2 pi j k / n) o_j,
+//   X_k = C_k - i S_k,   X_{n-k} = C_k + i S_k,
+// a quarter of the direct sum's products.  For even n = 2h the sums over even and
+// odd j are kept apart: position h - k has the same terms with the signs
+// (-1)^j and -(-1)^j, so the rows k <= h/2 give all four positions k, h - k,
+// h + k and n - k, another half.  The matrices come from the full-length twiddle
+// table exp(-2 pi i k / n) at (j k) mod n, so every entry is exact to one rounding,
+// and lie in memory in the order in which the lanes load them (k_dft_matrix).
+//
+// Per element of a complex line that is 2n flops (odd n) or n (even n): at
+// 365x365x425 an x sweep does 20.7 GFLOP over 454 MB, so the matrix cores bound it
+// above n of about 200 and memory below.  There, against the direct sums through LDS
+// (a vector fma and two LDS reads per term): x sweep 2217 -> 293 us, y pass 5145 ->
+// 541 us, KT column pass 5736 -> 743 us; at 193x193x1201 the KT column pass 17.7 ->
+// 2.4 ms.
 #pragma once
 #include "column.h"
 
 namespace ash {
 
-constexpr int GNT = 256;  // threads per general-size line block
+constexpr int GEN_MAXL = 1024;  // general-size line kernels: 2 .. 1024
 
-// f bins per general-size line tile: the tile (two n x lines complex buffers)
-// stays within 32 KB of LDS
-__host__ __device__ constexpr int gen_lines(int n) { return n <= 128 ? 16 : n <= 256 ? 8 : n <= 512 ? 4 : 2; }
-constexpr int GEN_MAXL = 1024;
-constexpr int GEN_TILE = 2048;  // n * lines <= 2048 for every n <= 1024
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-// out[k][l] = sum_j in[j][l] W^(j k), W = exp(-+2 pi i / n); [pos][line] layout, line fastest.
-template <bool INV>
-__device__ __forceinline__ void tile_dft(const float2* in, float2* out, const float2* tw, int n, int lines,
-                                         int tid) {
-  const int tot = n * lines;
-  for (int e = tid; e < tot; e += GNT) {
-    const int l = e % lines, k = e / lines;
-    float ax = 0.f, ay = 0.f;
-    int idx = 0;
-    for (int j = 0; j < n; ++j) {
-      const float2 x = in[j * lines + l];
-      float2 w = tw[idx];
-      if (INV) w.y = -w.y;
-      ax = fmaf(x.x, w.x, fmaf(-x.y, w.y, ax));
-      ay = fmaf(x.x, w.y, fmaf(x.y, w.x, ay));
-      idx += k;
-      if (idx >= n) idx -= n;
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// Input position of matrix column r: natural order for odd n, the even positions
+// and then (from column Ke on) the odd ones for even n.
+template <bool EVEN>
+__device__ __forceinline__ int hm_pos(const DftMat& d, int r) {
+  if constexpr (EVEN) return r < d.Ke ? 2 * r : 2 * (r - d.Ke) + 1;
+  else return r;
+}
+// and the column of input position j
+template <bool EVEN>
+__device__ __forceinline__ int hm_col(const DftMat& d, int j) {
+  if constexpr (EVEN) return (j & 1) ? d.Ke + (j >> 1) : (j >> 1);
+  else return j;
+}
+
+// Fills the matrix of one axis: entry [rt][g][lane] holds (cos, sin) at matrix row
+// 16 rt + lane % 16 and columns 8 g + lane / 16 and 8 g + 4 + lane / 16, the A
+// operands of two matrix-core products of four columns each; zero outside.
+template <bool EVEN>
+__global__ __launch_bounds__(256) void k_dft_matrix(DftMat d, const float2* __restrict__ tw, float4* __restrict__ out) {
+  const int G = d.Kp / 8;
+  const long tot = (long)d.R * G * 64;
+  for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < tot; e += (long)gridDim.x * 256) {
+    const int lane = (int)(e % 64);
+    const long rg = e / 64;
+    const int g = (int)(rg % G), rt = (int)(rg / G);
+    const int k = 16 * rt + (lane & 15);
+    float v[4];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int j = hm_pos<EVEN>(d, 8 * g + 4 * q + (lane >> 4));
+      float2 w = make_float2(0.f, 0.f);
+      if (k < d.rows && j <= d.h) w = tw[(int)(((long)j * k) % d.n)];
+      v[2 * q] = w.x;
+      v[2 * q + 1] = -w.y;
     }
-    out[e] = make_float2(ax, ay);
+    out[e] = make_float4(v[0], v[1], v[2], v[3]);
   }
 }
 
-// x-sweep, forward DFT along x.  Tile = (y, block of `lines` f bins).
-__global__ __launch_bounds__(GNT) void k_gx_fwd(float2* __restrict__ spec, Tables T, Geom g) {
-  __shared__ float2 tw[GEN_MAXL];
-  __shared__ float2 a[GEN_TILE], b[GEN_TILE];
-  const int n = g.nX, lines = gen_lines(n), nfb = g.MP / lines;
-  const int tid = threadIdx.x;
-  const int y = blockIdx.x / nfb, f0 = (blockIdx.x % nfb) * lines;
-  const long sx = (long)g.nY * g.MP;
-  float2* base = spec + (long)y * g.MP + f0;
-  const int nvalid = min(lines, g.M + 1 - f0);
-  for (int i = tid; i < n; i += GNT) tw[i] = T.twgx[i];
-  for (int e = tid; e < n * lines; e += GNT) {
-    const int l = e % lines, j = e / lines;
-    a[e] = l < nvalid ? base[j * sx + l] : make_float2(0.f, 0.f);
-  }
-  __syncthreads();
-  tile_dft<false>(a, b, tw, n, lines, tid);
-  __syncthreads();
-  for (int e = tid; e < n * lines; e += GNT) {
-    const int l = e % lines, k = e / lines;
-    if (l < nvalid) base[k * sx + l] = b[e];
-  }
+// ---------------------------------------------------------------------------
+// Lines (x and y sweeps).  A tile is all n positions of 16 consecutive f bins
+// (128-byte segments), folded into LDS rows [column r][line] of (e.re, e.im,
+// o.re, o.im): lane l's B operands of four matrix columns are one 16-byte read at
+// 4 s + l/16 of line l%16, 1 KB in a row per wave.  Every matrix entry meets two
+// operands (re and im), so the matrix stream from L2 stays at 16 B per CU-cycle of
+// matrix-core time.  Waves take row tiles rt = wave, wave + W, ...
+// ---------------------------------------------------------------------------
+template <bool EVEN>
+struct LineAcc {
+  static constexpr int NP = EVEN ? 2 : 1;  // sums over even j and over odd j
+  f32x4 c[NP][2], s[NP][2];                // [parity][re, im]
+};
+
+template <bool EVEN>
+__device__ __forceinline__ void hm_line_tile(const float4* eo, const DftMat& d, int rt, int lane, LineAcc<EVEN>& a) {
+  const int G = d.Kp / 8;
+  const float4* ap = d.A + (long)rt * G * 64 + lane;
+  const float4* bp = eo + lane;
+#pragma unroll
+  for (int p = 0; p < LineAcc<EVEN>::NP; ++p)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) a.c[p][q] = a.s[p][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto run = [&](int g0, int g1, f32x4 (&c)[2], f32x4 (&s)[2]) {
+#pragma unroll 2
+    for (int g = g0; g < g1; ++g) {
+      const float4 w = ap[g * 64];
+      const float4 b0 = bp[g * 128], b1 = bp[g * 128 + 64];
+      c[0] = mfma4(w.x, b0.x, c[0]);
+      c[1] = mfma4(w.x, b0.y, c[1]);
+      s[0] = mfma4(w.y, b0.z, s[0]);
+      s[1] = mfma4(w.y, b0.w, s[1]);
+      c[0] = mfma4(w.z, b1.x, c[0]);
+      c[1] = mfma4(w.z, b1.y, c[1]);
+      s[0] = mfma4(w.w, b1.z, s[0]);
+      s[1] = mfma4(w.w, b1.w, s[1]);
+    }
+  };
+  run(0, d.Ke / 8, a.c[0], a.s[0]);
+  if constexpr (EVEN) run(d.Ke / 8, G, a.c[1], a.s[1]);
 }
 
-// x-sweep, inverse DFT along x + the epilogues of k_xfft_inv (EPI 0, 1, 2).
-template <int EPI>
-__global__ __launch_bounds__(GNT) void k_gx_inv(float2* __restrict__ spec, Tables T, Geom g, EpiDesc ep) {
-  __shared__ float2 tw[GEN_MAXL];
-  __shared__ float2 a[GEN_TILE], b[GEN_TILE];
-  const int n = g.nX, lines = gen_lines(n), nfb = g.MP / lines;
-  const int tid = threadIdx.x;
-  const int y = blockIdx.x / nfb, f0 = (blockIdx.x % nfb) * lines;
-  const long sx = (long)g.nY * g.MP;
-  float2* base = spec + (long)y * g.MP + f0;
-  const int nvalid = min(lines, g.M + 1 - f0);
-  for (int i = tid; i < n; i += GNT) tw[i] = T.twgx[i];
-  for (int e = tid; e < n * lines; e += GNT) {
-    const int l = e % lines, j = e / lines;
-    a[e] = l < nvalid ? base[j * sx + l] : make_float2(0.f, 0.f);
+// The transform's values at output row k = 16 rt + 4 (lane / 16) + i of line
+// lane % 16: P = C - i S belongs to position k of the forward transform and
+// Q = C + i S to position n - k (the inverse swaps them); for even n also P2, Q2 of
+// positions h - k and h + k.
+template <bool EVEN>
+__device__ __forceinline__ void hm_values(const LineAcc<EVEN>& a, int i, float2& P, float2& Q, float2& P2, float2& Q2) {
+  float cr = a.c[0][0][i], ci = a.c[0][1][i], sr = a.s[0][0][i], si = a.s[0][1][i];
+  if constexpr (EVEN) {
+    const float cr1 = a.c[1][0][i], ci1 = a.c[1][1][i], sr1 = a.s[1][0][i], si1 = a.s[1][1][i];
+    const float dcr = cr - cr1, dci = ci - ci1, dsr = sr1 - sr, dsi = si1 - si;
+    P2 = make_float2(dcr + dsi, dci - dsr);
+    Q2 = make_float2(dcr - dsi, dci + dsr);
+    cr += cr1; ci += ci1; sr += sr1; si += si1;
   }
-  __syncthreads();
-  tile_dft<true>(a, b, tw, n, lines, tid);
-  __syncthreads();
-  if constexpr (EPI == 0 || EPI == 1) {
-    float ty = 1.f;
-    const float* tx = nullptr;
-    if constexpr (EPI == 1) {
-      ty = ep.half ? T.tapy_h[y] : T.tapy_f[y];
-      tx = ep.half ? T.tapx_h : T.tapx_f;
-    }
-    for (int e = tid; e < n * lines; e += GNT) {
-      const int l = e % lines, k = e / lines;
-      float2 v = b[e];
-      if constexpr (EPI == 1) v = cscale(v, tx[k] * ty);
-      if (l < nvalid) base[k * sx + l] = v;
-    }
-  } else {
-    // scale, DC/Nyquist projection and frequency-weighted mask, then the SA x stencil
-    // on the masked values (as k_xfft_inv<., 2>)
-    const float lgy = T.lgy[y];
-    for (int e = tid; e < n * lines; e += GNT) {
-      const int l = e % lines, k = e / lines, m = f0 + l;
-      float2 v = cscale(b[e], ep.scale);
-      if (m == 0 || m == g.nyq) v.y = 0.f;
-      if (ep.fw) v = cscale(v, exp2f(T.fw_exp[min(m, g.MP - 1)] * (T.lgx[k] + lgy)));
-      b[e] = v;
-    }
-    __syncthreads();
-    for (int e = tid; e < n * lines; e += GNT) {
-      const int l = e % lines, k = e / lines, m = f0 + l;
-      float2 v = b[e];
-      if (ep.sa) {
-        const float w = T.sa_wx[k];
-        if (w != 0.f) {
-          float2 d;
-          if (k == 0) d = cscale(csub(b[lines + l], v), ep.invdx);
-          else if (k == n - 1) d = cscale(csub(v, b[(n - 2) * lines + l]), ep.invdx);
-          else d = cscale(csub(b[(k + 1) * lines + l], b[(k - 1) * lines + l]), ep.inv2dx);
-          const float cw = T.sa_cw[min(m, g.MP - 1)];
-          const float2 cd = make_float2(cw * d.y, -cw * d.x);
-          const float2 pin = k < n / 2 ? cscale(cadd(v, cd), 0.5f) : cscale(csub(v, cd), 0.5f);
-          v = csub(v, cscale(pin, ep.sa_strength * w));
+  P = make_float2(cr + si, ci - sr);
+  Q = make_float2(cr - si, ci + sr);
+}
+
+// f(position, value) for every output of this lane in one tile
+template <bool EVEN, bool INV, class F>
+__device__ __forceinline__ void hm_emit(const DftMat& d, const LineAcc<EVEN>& a, int rt, int lane, F f) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int k = 16 * rt + 4 * (lane >> 4) + i;
+    float2 P, Q, P2, Q2;
+    hm_values<EVEN>(a, i, P, Q, P2, Q2);
+    if (k < d.rows) {
+      f(k, INV ? Q : P);
+      if (k > 0) f(d.n - k, INV ? P : Q);
+      if constexpr (EVEN) {
+        const int k2 = d.h - k;
+        if (k2 != k) {
+          f(k2, INV ? Q2 : P2);
+          if (k > 0) f(d.h + k, INV ? P2 : Q2);
         }
       }
-      if (l < nvalid) base[k * sx + l] = v;
     }
   }
 }
 
-// y-pass: forward DFT along y, the visit operator, inverse DFT.  Tile = (x, f block).
-__global__ __launch_bounds__(GNT) void k_gy_pass(float2* __restrict__ spec, Tables T, Geom g, OpDesc op) {
-  __shared__ float2 tw[GEN_MAXL];
-  __shared__ float2 a[GEN_TILE], b[GEN_TILE];
-  __shared__ LineConst slc[16];
-  const int n = g.nY, lines = gen_lines(n), nfb = g.MP / lines;
-  const int tid = threadIdx.x;
-  const int x = blockIdx.x / nfb, f0 = (blockIdx.x % nfb) * lines;
+// Folds a line tile into LDS; ld(position, line) reads one element.  The loads of
+// four rows are issued before the first is used.
+template <bool EVEN, class Ld>
+__device__ __forceinline__ void hm_fold(float4* eo, const DftMat& d, int tid, int nthr, Ld ld) {
+  const int line = tid & 15, step = nthr >> 4;
+  for (int r0 = tid >> 4; r0 < d.Kp; r0 += 4 * step) {
+    float2 a[4], b[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int j = min(hm_pos<EVEN>(d, min(r0 + q * step, d.Kp - 1)), d.h);
+      a[q] = ld(j, line);
+      b[q] = ld(j == 0 ? 0 : d.n - j, line);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = r0 + q * step;
+      if (r >= d.Kp) break;
+      const int j = hm_pos<EVEN>(d, r);
+      const bool pair = j > 0 && 2 * j != d.n;  // positions 0 and n/2 have no partner
+      float4 v = make_float4(a[q].x, a[q].y, 0.f, 0.f);
+      if (pair) v = make_float4(a[q].x + b[q].x, a[q].y + b[q].y, a[q].x - b[q].x, a[q].y - b[q].y);
+      if (j > d.h) v = make_float4(0.f, 0.f, 0.f, 0.f);  // matrix padding
+      eo[r * 16 + line] = v;
+    }
+  }
+}
+
+// x-sweep, forward DFT along x.  Tile = (y, 16 f bins).  Padding lines past the last
+// bin are zero and stay zero, so no load or store is guarded.
+template <bool EVEN>
+__global__ __launch_bounds__(512) void k_gx_fwd(float2* __restrict__ spec, Tables T, Geom g) {
+  extern __shared__ float4 eo[];
+  const DftMat d = T.dmx;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
+  const int y = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
+  const uint32_t sxb = (uint32_t)g.nY * g.MP * 8u;
+  float2* base = spec + (long)y * g.MP + f0;
+  hm_fold<EVEN>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * sxb + line * 8u); });
+  __syncthreads();
+  const uint32_t lo = (lane & 15) * 8u;
+  for (int rt = wave; rt < d.R; rt += W) {
+    LineAcc<EVEN> a;
+    hm_line_tile<EVEN>(eo, d, rt, lane, a);
+    hm_emit<EVEN, false>(d, a, rt, lane, [&](int pos, float2 v) { gst(base, pos * sxb + lo, v); });
+  }
+}
+
+// x-sweep, inverse DFT along x + the epilogues 0 and 1 of k_xfft_inv.
+template <bool EVEN, int EPI>
+__global__ __launch_bounds__(512) void k_gx_inv(float2* __restrict__ spec, Tables T, Geom g, EpiDesc ep) {
+  extern __shared__ float4 eo[];
+  const DftMat d = T.dmx;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
+  const int y = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
+  const uint32_t sxb = (uint32_t)g.nY * g.MP * 8u;
+  float2* base = spec + (long)y * g.MP + f0;
+  hm_fold<EVEN>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * sxb + line * 8u); });
+  __syncthreads();
+  const uint32_t lo = (lane & 15) * 8u;
+  float ty = 1.f;
+  const float* tx = nullptr;
+  if constexpr (EPI == 1) {
+    ty = ep.half ? T.tapy_h[y] : T.tapy_f[y];
+    tx = ep.half ? T.tapx_h : T.tapx_f;
+  }
+  for (int rt = wave; rt < d.R; rt += W) {
+    LineAcc<EVEN> a;
+    hm_line_tile<EVEN>(eo, d, rt, lane, a);
+    hm_emit<EVEN, true>(d, a, rt, lane, [&](int pos, float2 v) {
+      if constexpr (EPI == 1) v = cscale(v, tx[pos] * ty);
+      gst(base, pos * sxb + lo, v);
+    });
+  }
+}
+
+// x-sweep, inverse DFT along x + epilogue 2 of k_xfft_inv: scale, DC/Nyquist
+// projection, frequency-weighted mask and the SA x stencil on the masked values,
+// which pass through the tile's LDS (n * 16 float2 fit the folded tile) once every
+// wave holds its T row tiles in registers.
+template <bool EVEN, int T_>
+__global__ __launch_bounds__(512) void k_gx_inv_sa(float2* __restrict__ spec, Tables T, Geom g, EpiDesc ep) {
+  extern __shared__ float4 eo[];
+  const DftMat d = T.dmx;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
+  const int y = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
+  const uint32_t sxb = (uint32_t)g.nY * g.MP * 8u;
+  float2* base = spec + (long)y * g.MP + f0;
+  hm_fold<EVEN>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * sxb + line * 8u); });
+  __syncthreads();
+  LineAcc<EVEN> a[T_];
+#pragma unroll
+  for (int i = 0; i < T_; ++i)
+    if (wave + W * i < d.R) hm_line_tile<EVEN>(eo, d, wave + W * i, lane, a[i]);
+  __syncthreads();
+  float2* b = reinterpret_cast<float2*>(eo);
+  const float lgy = T.lgy[y];
+  {
+    const int line = lane & 15, m = f0 + line;
+    const float fe = T.fw_exp[m];
+    const bool real = m == 0 || m == g.nyq;  // irfft/rfft round trip of the reference
+#pragma unroll
+    for (int i = 0; i < T_; ++i)
+      if (wave + W * i < d.R)
+        hm_emit<EVEN, true>(d, a[i], wave + W * i, lane, [&](int pos, float2 v) {
+          v = cscale(v, ep.scale);
+          if (real) v.y = 0.f;
+          if (ep.fw && m <= g.M) v = cscale(v, exp2f(fe * (T.lgx[pos] + lgy)));
+          b[pos * 16 + line] = v;
+        });
+  }
+  __syncthreads();
+  const int n = d.n, line = tid & 15;
+  const float cw = T.sa_cw[f0 + line];
+  for (int k = tid >> 4; k < n; k += blockDim.x >> 4) {
+    float2 v = b[k * 16 + line];
+    if (ep.sa) {
+      const float w = T.sa_wx[k];
+      if (w != 0.f) {
+        float2 dd;
+        if (k == 0) dd = cscale(csub(b[16 + line], v), ep.invdx);
+        else if (k == n - 1) dd = cscale(csub(v, b[(n - 2) * 16 + line]), ep.invdx);
+        else dd = cscale(csub(b[(k + 1) * 16 + line], b[(k - 1) * 16 + line]), ep.inv2dx);
+        const float2 cd = make_float2(cw * dd.y, -cw * dd.x);
+        const float2 pin = k < n / 2 ? cscale(cadd(v, cd), 0.5f) : cscale(csub(v, cd), 0.5f);
+        v = csub(v, cscale(pin, ep.sa_strength * w));
+      }
+    }
+    gst(base, k * sxb + line * 8u, v);
+  }
+}
+
+__device__ __forceinline__ LineConst line_const(const Tables& T, const OpDesc& op, int m) {
+  const double kt = T.kt[m], ka = T.ka[m];
+  LineConst lc;
+  lc.kt2 = kt * kt;
+  lc.ka2 = ka * ka;
+  lc.ktd = kt;
+  lc.kt = (float)kt;
+  lc.ka = (float)ka;
+  lc.ald = T.alpha[m] * op.dz_att;
+  lc.asd = T.astar[m] * op.dz_att;
+  lc.al = (float)lc.ald;
+  lc.as = (float)lc.asd;
+  lc.kept = kt > 0.0;
+  return lc;
+}
+
+// y-pass: forward DFT along y, the visit operator, inverse DFT.  Tile = (x, 16 f
+// bins).  A lane holds positions k and n - k (for even n also h - k and h + k) of its
+// line, which is the pair the inverse transform folds: the operator and the fold
+// happen in registers, and only the folded rows return to LDS.  The operator is
+// evaluated at every position's own wavenumber (the grids are mirror images only up
+// to rounding, and one ulp decides a mode at the evanescent cutoff).
+template <bool EVEN, int T_, bool PRECISE>
+__global__ __launch_bounds__(512) void k_gy_pass(float2* __restrict__ spec, Tables T, Geom g, OpDesc op) {
+  extern __shared__ float4 eo[];
+  const DftMat d = T.dmy;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
+  const int x = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
+  const uint32_t syb = (uint32_t)g.MP * 8u;
   float2* base = spec + (long)x * g.nY * g.MP + f0;
-  const int nvalid = min(lines, g.M + 1 - f0);
-  for (int i = tid; i < n; i += GNT) tw[i] = T.twgy[i];
-  if (tid < lines) {
-    const int m = min(f0 + tid, g.MP - 1);
-    const double kt = T.kt[m], ka = T.ka[m];
-    LineConst lc;
-    lc.kt2 = kt * kt;
-    lc.ka2 = ka * ka;
-    lc.ktd = kt;
-    lc.kt = (float)kt;
-    lc.ka = (float)ka;
-    lc.ald = T.alpha[m] * op.dz_att;
-    lc.asd = T.astar[m] * op.dz_att;
-    lc.al = (float)lc.ald;
-    lc.as = (float)lc.asd;
-    lc.kept = kt > 0.0;
-    slc[tid] = lc;
+  hm_fold<EVEN>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * syb + line * 8u); });
+  __syncthreads();
+  LineAcc<EVEN> a[T_];
+#pragma unroll
+  for (int i = 0; i < T_; ++i)
+    if (wave + W * i < d.R) hm_line_tile<EVEN>(eo, d, wave + W * i, lane, a[i]);
+  __syncthreads();
+  {
+    const int line = lane & 15, m = f0 + line;
+    const LineConst lc = line_const(T, op, m);
+    const double kx = T.kx[x];
+    auto apply = [&](int pos, float2 v) {
+      const double kk = kperp2(kx, T.ky[pos]);
+      float2 o;
+      if constexpr (PRECISE) o = visit_operator_fp64(op, kk, lc, m);
+      else o = visit_operator(op, kk, lc, m);
+      return cmul(v, o);
+    };
+    // folded row of position k from the values at k and n - k
+    auto put = [&](int k, float2 v, float2 vn, bool pair) {
+      v = apply(k, v);
+      float4 e = make_float4(v.x, v.y, 0.f, 0.f);
+      if (pair) {
+        vn = apply(d.n - k, vn);
+        e = make_float4(v.x + vn.x, v.y + vn.y, v.x - vn.x, v.y - vn.y);
+      }
+      eo[hm_col<EVEN>(d, k) * 16 + line] = e;
+    };
+#pragma unroll
+    for (int i = 0; i < T_; ++i) {
+      const int rt = wave + W * i;
+      if (rt < d.R) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int k = 16 * rt + 4 * (lane >> 4) + q;
+          float2 P, Q, P2, Q2;
+          hm_values<EVEN>(a[i], q, P, Q, P2, Q2);
+          if (k < d.rows) {
+            put(k, P, Q, k > 0);
+            if constexpr (EVEN) {
+              if (d.h - k != k) put(d.h - k, P2, Q2, k > 0);
+            }
+          }
+        }
+      }
+    }
   }
-  for (int e = tid; e < n * lines; e += GNT) {
-    const int l = e % lines, j = e / lines;
-    a[e] = l < nvalid ? base[(long)j * g.MP + l] : make_float2(0.f, 0.f);
-  }
   __syncthreads();
-  tile_dft<false>(a, b, tw, n, lines, tid);
-  __syncthreads();
-  const double kx = T.kx[x];
-  for (int e = tid; e < n * lines; e += GNT) {
-    const int l = e % lines, k = e / lines;
-    const double ky = T.ky[k];
-    const double kk = kperp2(kx, ky);
-    const float2 o = op.precise ? visit_operator_fp64(op, kk, slc[l], f0 + l) : visit_operator(op, kk, slc[l], f0 + l);
-    b[e] = cmul(b[e], o);
-  }
-  __syncthreads();
-  tile_dft<true>(b, a, tw, n, lines, tid);
-  __syncthreads();
-  for (int e = tid; e < n * lines; e += GNT) {
-    const int l = e % lines, k = e / lines;
-    if (l < nvalid) base[(long)k * g.MP + l] = a[e];
+  const uint32_t lo = (lane & 15) * 8u;
+  for (int rt = wave; rt < d.R; rt += W) {
+    LineAcc<EVEN> r;
+    hm_line_tile<EVEN>(eo, d, rt, lane, r);
+    hm_emit<EVEN, true>(d, r, rt, lane, [&](int pos, float2 v) { gst(base, pos * syb + lo, v); });
   }
 }
 
 // Power-weighted obliquity sums of a (kx row, f block) tile (as k_ypower): forward
 // DFT along y, then acc[0] += sum P k/k_z, acc[1] += sum P over propagating modes.
-__global__ __launch_bounds__(GNT) void k_gy_power(const float2* __restrict__ spec, Tables T, Geom g,
+template <bool EVEN>
+__global__ __launch_bounds__(512) void k_gy_power(const float2* __restrict__ spec, Tables T, Geom g,
                                                   double* __restrict__ acc) {
-  __shared__ float2 tw[GEN_MAXL];
-  __shared__ float2 a[GEN_TILE], b[GEN_TILE];
-  __shared__ double sred[2][GNT / 64];
-  const int n = g.nY, lines = gen_lines(n), nfb = g.MP / lines;
-  const int tid = threadIdx.x;
-  const int x = blockIdx.x / nfb, f0 = (blockIdx.x % nfb) * lines;
+  extern __shared__ float4 eo[];
+  __shared__ double sred[2][8];
+  const DftMat d = T.dmy;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
+  const int x = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
+  const uint32_t syb = (uint32_t)g.MP * 8u;
   const float2* base = spec + (long)x * g.nY * g.MP + f0;
-  const int nvalid = min(lines, g.M + 1 - f0);
-  for (int i = tid; i < n; i += GNT) tw[i] = T.twgy[i];
-  for (int e = tid; e < n * lines; e += GNT) {
-    const int l = e % lines, j = e / lines;
-    a[e] = l < nvalid ? base[(long)j * g.MP + l] : make_float2(0.f, 0.f);
-  }
+  hm_fold<EVEN>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * syb + line * 8u); });
   __syncthreads();
-  tile_dft<false>(a, b, tw, n, lines, tid);
-  __syncthreads();
+  const int m = f0 + (lane & 15);
+  const double km = m <= g.M ? T.ka[m] : 0.0;  // ka[0] = 0: the DC bin weighs nothing
   const double kx = T.kx[x];
   double num = 0.0, den = 0.0;
-  for (int e = tid; e < n * lines; e += GNT) {
-    const int l = e % lines, k = e / lines, m = f0 + l;
-    if (l >= nvalid || m == 0) continue;
-    const double km = T.ka[m];
-    const double ky = T.ky[k];
-    const double kz2 = kz2_of(km, kperp2(kx, ky));
-    if (kz2 > 0.0) {
-      const float2 v = b[e];
-      const double P = (double)v.x * v.x + (double)v.y * v.y;
-      num += P * km / fmax(sqrt(kz2), km * 1e-6);
-      den += P;
-    }
+  for (int rt = wave; rt < d.R; rt += W) {
+    LineAcc<EVEN> a;
+    hm_line_tile<EVEN>(eo, d, rt, lane, a);
+    hm_emit<EVEN, false>(d, a, rt, lane, [&](int pos, float2 v) {
+      const double ky = T.ky[pos];
+      const double kz2 = kz2_of(km, kperp2(kx, ky));
+      if (km > 0.0 && kz2 > 0.0) {
+        const double P = (double)v.x * v.x + (double)v.y * v.y;
+        num += P * km / fmax(sqrt(kz2), km * 1e-6);
+        den += P;
+      }
+    });
   }
   for (int o = 32; o > 0; o >>= 1) {
     num += __shfl_xor(num, o, 64);
     den += __shfl_xor(den, o, 64);
   }
-  if ((tid & 63) == 0) { sred[0][tid >> 6] = num; sred[1][tid >> 6] = den; }
+  if (lane == 0) { sred[0][wave] = num; sred[1][wave] = den; }
   __syncthreads();
   if (tid == 0) {
     double s0 = 0.0, s1 = 0.0;
-    for (int w = 0; w < GNT / 64; ++w) { s0 += sred[0][w]; s1 += sred[1][w]; }
+    for (int w = 0; w < W; ++w) { s0 += sred[0][w]; s1 += sred[1][w]; }
     atomicAdd(acc, s0);
     atomicAdd(acc + 1, s1);
   }
 }
 
 // y-sweep without a transform (as k_ysa) for any nY: super-absorbing y pass,
-// DC/Nyquist projection and an optional phase/amplitude screen.  Tile = (x, f block
-// of gen_lines(nY) bins); the rows handled (all with a screen, else the two boundary
-// bands) sit in LDS.
-__global__ __launch_bounds__(GNT) void k_gy_sa(float2* __restrict__ spec, Tables T, Geom g, ScreenDesc s) {
-  __shared__ float2 buf[GEN_TILE];
-  const int L = g.nY, lines = gen_lines(L), nfb = g.MP / lines;
-  const int tid = threadIdx.x;
-  const int x = blockIdx.x / nfb, f0 = (blockIdx.x % nfb) * lines;
+// DC/Nyquist projection and an optional phase/amplitude screen.  Tile = (x, 16 f
+// bins); the rows handled (all with a screen, else the two boundary bands) sit in
+// LDS, ysa_rows * 128 bytes of it.
+__global__ __launch_bounds__(256) void k_gy_sa(float2* __restrict__ spec, Tables T, Geom g, ScreenDesc s) {
+  extern __shared__ float2 sbuf[];
+  const int L = g.nY;
+  const int tid = threadIdx.x, l = tid & 15;
+  const int x = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
   float2* base = spec + (long)x * g.nY * g.MP + f0;
-  const int nvalid = min(lines, g.M + 1 - f0);
   const int nrows = ysa_rows(L, s.band, s.phase != nullptr);
   const bool band = nrows < L;
   auto row_of = [&](int i) { return (band && i > s.band) ? L - nrows + i : i; };
-  const int nel = nrows * lines;
-  for (int el = tid; el < nel; el += GNT) {
-    const int l = el % lines, i = el / lines;
-    buf[el] = l < nvalid ? base[(long)row_of(i) * g.MP + l] : make_float2(0.f, 0.f);
-  }
+#pragma unroll 4
+  for (int i = tid >> 4; i < nrows; i += 16) sbuf[i * 16 + l] = base[(long)row_of(i) * g.MP + l];
   __syncthreads();
-  for (int el = tid; el < nel; el += GNT) {
-    const int l = el % lines, i = el / lines;
-    const int pos = row_of(i), m = f0 + l;
-    float2 u = buf[el];
+  const int m = f0 + l;
+  const float cw = s.sa ? T.sa_cw[m] : 0.f;
+  const float fs = (float)m / s.f0b;
+  for (int i = tid >> 4; i < nrows; i += 16) {
+    const int pos = row_of(i);
+    float2 u = sbuf[i * 16 + l];
     if (s.sa) {
       const float w = T.sa_wy[pos];
       if (w != 0.f) {
         float2 d;
-        if (pos == 0) d = cscale(csub(buf[(i + 1) * lines + l], u), s.invdy);
-        else if (pos == L - 1) d = cscale(csub(u, buf[(i - 1) * lines + l]), s.invdy);
-        else d = cscale(csub(buf[(i + 1) * lines + l], buf[(i - 1) * lines + l]), s.inv2dy);
-        const float cw = T.sa_cw[min(m, g.MP - 1)];
+        if (pos == 0) d = cscale(csub(sbuf[(i + 1) * 16 + l], u), s.invdy);
+        else if (pos == L - 1) d = cscale(csub(u, sbuf[(i - 1) * 16 + l]), s.invdy);
+        else d = cscale(csub(sbuf[(i + 1) * 16 + l], sbuf[(i - 1) * 16 + l]), s.inv2dy);
         const float2 cd = make_float2(cw * d.y, -cw * d.x);
         const float2 pin = pos < L / 2 ? cscale(cadd(u, cd), 0.5f) : cscale(csub(u, cd), 0.5f);
         u = csub(u, cscale(pin, s.sa_strength * w));
@@ -271,7 +453,6 @@ __global__ __launch_bounds__(GNT) void k_gy_sa(float2* __restrict__ spec, Tables
     if (m == 0 || m == g.nyq) u.y = 0.f;
     if (s.phase) {
       const long idx = (long)x * g.nY + pos;
-      const float fs = (float)m / s.f0b;
       const float th = s.phase[idx] * fs;
       float sn, cs;
       sincosf(th, &sn, &cs);
@@ -282,42 +463,105 @@ __global__ __launch_bounds__(GNT) void k_gy_sa(float2* __restrict__ spec, Tables
       }
       if (m == 0 || m == g.nyq) u.y = 0.f;
     }
-    if (l < nvalid) base[(long)pos * g.MP + l] = u;
+    if (m <= g.M) base[(long)pos * g.MP + l] = u;
   }
 }
 
 // ---------------------------------------------------------------------------
-// General-length t-column kernel: one wave per column, lane ln holds the S
-// contiguous samples t = S ln .. S ln + S - 1 (padding beyond nT is zero).
-// irfft and rfft are direct real DFTs through the wave's LDS region; the
-// real-space stage is column_realspace, as in k_column.  Semantics of the
-// transforms (ASS:664, :685): the inverse ignores the imaginary parts of the DC
-// bin and, for even nT, of the Nyquist bin; the forward writes them as zero.
+// General-length t columns: one block takes 16 columns, the 16 output columns of
+// a matrix-core product.  irfft and rfft are the real halves of the folded DFT:
+//   inverse  C_t = sum_m a_m Re X_m cos, S_t = sum_m a_m Im X_m sin (a_0 = a_{nT/2}
+//            = 1, else 2), u_t = (C_t - S_t) / nT, u_{nT-t} = (C_t + S_t) / nT;
+//   forward  X_m = sum e_t cos - i sum o_t sin, e_t = u_t + u_{nT-t}, o_t = u_t - u_{nT-t}.
+// Each column is a product column of its own: nothing of one reaches another.  The
+// tile passes LDS as spectrum rows X[column][m], as samples U[column][t] (each wave
+// runs the real-space stage, column_realspace, on its 16 / W columns, lane ln with
+// the S contiguous samples from S ln), folded in place (e_t at t, o_t at nT - t), and
+// as X again; the accumulators of a transform wait in registers for the barrier
+// before the tile changes form.  Semantics of the transforms (ASS:664, :685): the
+// inverse ignores the imaginary parts of the DC bin and, for even nT, of the Nyquist
+// bin; the forward writes them as zero.
+// Per sample that is nT flops per transform (odd nT) or nT/2 (even): the matrix cores
+// bound the pass.  Row strides: U = 17 (mod 64) floats, X = 4 (mod 32) float2, so the
+// four rows of an operand and the 16 columns fall in distinct banks.
 // ---------------------------------------------------------------------------
-constexpr int GC_WPB = 4;
+constexpr int GC_COLS = 16;
+constexpr int gcol_waves(int S) { return S == 2 ? 4 : 8; }
+// row tiles per wave: nT <= 64 S has at most 2 S tiles (odd) or S + 1 (even)
+constexpr int gcol_tiles(int S, bool even) {
+  return ((even ? S + 1 : 2 * S) + gcol_waves(S) - 1) / gcol_waves(S);
+}
+__host__ __device__ inline int gcol_ustride(int nT) { return nT + 1 <= 17 ? 17 : (nT + 1 - 17 + 63) / 64 * 64 + 17; }
+__host__ __device__ inline int gcol_xstride(int M) { return M + 1 <= 4 ? 4 : (M + 1 - 4 + 31) / 32 * 32 + 4; }
+__host__ __device__ inline int gcol_lds_bytes(int nT) {
+  const int u = GC_COLS * gcol_ustride(nT) * 4, x = GC_COLS * gcol_xstride(nT / 2) * 8;
+  return u > x ? u : x;
+}
 
-template <int S, int MODE, int NLK>
-__global__ __launch_bounds__(256) void k_gcolumn(float2* __restrict__ spec, Tables T, Geom g, ColDesc d) {
-  constexpr int NTMAX = 64 * S;
-  __shared__ float2 s_tw[NTMAX];
-  __shared__ float2 s_buf[GC_WPB][NTMAX / 2 + 8];
-  __shared__ float s_red[GC_WPB];
-  const int tid = threadIdx.x;
-  const int wave = tid / 64, lane = tid % 64, ln = lane;
-  const int nT = g.nT, M = g.M;  // bins 0..M, M = nT / 2
-  constexpr bool spectral_in = !(MODE == COL_LOAD || MODE == COL_RAWNL);
-  constexpr bool rewrite = (MODE == COL_NL || MODE == COL_TAPER || MODE == COL_LOAD || MODE == COL_FINAL_SRC);
-  if constexpr (spectral_in || rewrite) {
-    for (int i = tid; i < nT; i += 256) s_tw[i] = T.twgt[i];
+template <bool EVEN>
+struct ColAcc {
+  static constexpr int NP = EVEN ? 2 : 1;
+  f32x4 c[NP], s[NP];
+};
+
+// One row tile; b(column r) reads the lane's (even part, odd part) operands.
+template <bool EVEN, class B>
+__device__ __forceinline__ void hm_col_tile(const DftMat& d, int rt, int lane, ColAcc<EVEN>& a, B b) {
+  const int G = d.Kp / 8, r0 = lane >> 4;
+  const float4* ap = d.A + (long)rt * G * 64 + lane;
+#pragma unroll
+  for (int p = 0; p < ColAcc<EVEN>::NP; ++p) a.c[p] = a.s[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto run = [&](int g0, int g1, f32x4& c, f32x4& s) {
+#pragma unroll 2
+    for (int g = g0; g < g1; ++g) {
+      const float4 w = ap[g * 64];
+      // matrix padding multiplies the last position by zero
+      const float2 v0 = b(min(hm_pos<EVEN>(d, 8 * g + r0), d.h));
+      const float2 v1 = b(min(hm_pos<EVEN>(d, 8 * g + 4 + r0), d.h));
+      c = mfma4(w.x, v0.x, c);
+      s = mfma4(w.y, v0.y, s);
+      c = mfma4(w.z, v1.x, c);
+      s = mfma4(w.w, v1.y, s);
+    }
+  };
+  run(0, d.Ke / 8, a.c[0], a.s[0]);
+  if constexpr (EVEN) run(d.Ke / 8, G, a.c[1], a.s[1]);
+}
+
+// f(position k <= n/2, C_k, S_k) for every output of this lane in one tile
+template <bool EVEN, class F>
+__device__ __forceinline__ void hm_col_emit(const DftMat& d, const ColAcc<EVEN>& a, int rt, int lane, F f) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int k = 16 * rt + 4 * (lane >> 4) + i;
+    if (k >= d.rows) continue;
+    if constexpr (EVEN) {
+      f(k, a.c[0][i] + a.c[1][i], a.s[0][i] + a.s[1][i]);
+      if (d.h - k != k) f(d.h - k, a.c[0][i] - a.c[1][i], a.s[1][i] - a.s[0][i]);
+    } else {
+      f(k, a.c[0][i], a.s[0][i]);
+    }
   }
-  __syncthreads();
-  float2* cb = s_buf[wave];
-  float* rb = reinterpret_cast<float*>(cb);
-  const int ncols = g.nX * g.nY;
-  const int t0 = ln * S;
+}
+
+template <int S, bool EVEN, int MODE, int NLK>
+__global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restrict__ spec, Tables T, Geom g, ColDesc d) {
+  constexpr int W = gcol_waves(S), TW = gcol_tiles(S, EVEN), NC = GC_COLS / W;
+  extern __shared__ float4 glds[];
+  __shared__ float s_red[W];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int nT = g.nT, M = g.M, ncols = g.nX * g.nY;
+  const DftMat dm = T.dmt;
+  const int LSU = gcol_ustride(nT), LSX = gcol_xstride(M);
+  float* U = reinterpret_cast<float*>(glds);
+  float2* X = reinterpret_cast<float2*>(glds);
+  const int c0 = blockIdx.x * GC_COLS;
+  const int t0 = lane * S;
   const float invN = 1.f / (float)nT;
-  const LaneCol<S, 64, false, true> lc{ln, lane, t0, nT};
+  constexpr bool spectral_in = MODE != COL_LOAD;
+  constexpr bool rewrite = (MODE == COL_NL || MODE == COL_TAPER || MODE == COL_LOAD || MODE == COL_FINAL_SRC);
   constexpr bool FIN = (MODE == COL_FINAL || MODE == COL_FINAL_SRC);
+  const LaneCol<S, 64, false, true> lc{lane, lane, t0, nT};
   const int row = (FIN || MODE == COL_TOF) ? *d.row : 0;
   const double Nn = d.nscale ? d.N * (d.nscale[0] / (d.nscale[1] + 1e-30)) : d.N;
   float wmax = 0.f;
@@ -330,120 +574,190 @@ __global__ __launch_bounds__(256) void k_gcolumn(float2* __restrict__ spec, Tabl
       if (capped && blockIdx.x == 0 && tid == 0 && d.subcap) atomicAdd(d.subcap, 1u);
     }
   }
-  const bool even = (nT & 1) == 0;
-  const int mh = (nT - 1) / 2;  // last bin with a conjugate partner
-
-  const float2* sc_cur = nullptr;  // spectrum row of the current column
-  // inverse real DFT of the current column's bins (modified by tof_bin(sel)) into
-  // this lane's samples: u[t] = (X_0 + 2 sum_{m=1}^{mh} Re(X_m e^{2 pi i m t / nT})
-  //                             + [even nT] X_{nT/2} (-1)^t) / nT
-  auto inv_spec = [&](float (&uo)[S], int sel) {
-    for (int m = ln; m <= M; m += 64) {
-      float2 x = sc_cur[m];
-      if (m == 0 || (even && m == M)) x.y = 0.f;
-      cb[m] = tof_bin(sel, m, x, even ? M : -1, d.tofref);
-    }
-    wave_sync();
-    const float x0 = cb[0].x;
-    const float xn = even ? cb[M].x : 0.f;
+  // inverse transform of the block's columns (bins modified by tof_bin(sel)) into U
+  auto inverse = [&](int sel) {
 #pragma unroll
-    for (int i = 0; i < S; ++i) {
-      const int t = t0 + i;
-      float acc = 0.f;
-      if (t < nT) {
-        int idx = 0;
-        for (int m = 1; m <= mh; ++m) {
-          idx += t;
-          if (idx >= nT) idx -= nT;
-          const float2 x = cb[m], w = s_tw[idx];  // e^{+i} = conj(w)
-          acc = fmaf(x.x, w.x, fmaf(x.y, w.y, acc));
+    for (int i = 0; i < NC; ++i) {
+      const int col = wave * NC + i, c = c0 + col;
+      if (c < ncols) {
+        const float2* sc = spec + (long)c * g.MP;
+#pragma unroll 4
+        for (int m = lane; m <= M; m += 64) {
+          float2 x = sc[m];
+          const bool real = m == 0 || m == g.nyq;
+          if (real) x.y = 0.f;
+          x = tof_bin(sel, m, x, g.nyq, d.tofref);
+          if (real) x.y = 0.f;
+          X[col * LSX + m] = real ? x : make_float2(2.f * x.x, 2.f * x.y);
         }
-        acc = fmaf(2.f, acc, x0 + ((t & 1) ? -xn : xn));
       }
-      uo[i] = t < nT ? acc * invN : 0.f;
     }
-    wave_sync();
+    __syncthreads();
+    ColAcc<EVEN> a[TW];
+    const float2* xc = X + (lane & 15) * LSX;
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+      if (wave + W * i < dm.R) hm_col_tile<EVEN>(dm, wave + W * i, lane, a[i], [&](int m) { return xc[m]; });
+    __syncthreads();
+    float* uc = U + (lane & 15) * LSU;
+#pragma unroll
+    for (int i = 0; i < TW; ++i)
+      if (wave + W * i < dm.R)
+        hm_col_emit<EVEN>(dm, a[i], wave + W * i, lane, [&](int t, float C, float Sn) {
+          uc[t] = (C - Sn) * invN;
+          if (t > 0 && 2 * t != nT) uc[nT - t] = (C + Sn) * invN;
+        });
+    __syncthreads();
+  };
+  auto samples = [&](float (&u)[S], int col) {
+#pragma unroll
+    for (int i = 0; i < S; ++i) u[i] = t0 + i < nT ? U[col * LSU + t0 + i] : 0.f;
   };
 
-  for (int cbase = blockIdx.x * GC_WPB; cbase < ncols; cbase += gridDim.x * GC_WPB) {
-    const int c = cbase + wave;
-    const bool live = c < ncols && (!d.cflag || d.cflag[c] != 0);
-    if (!live) continue;
-    float2* sc = spec + (long)c * g.MP;
-    float u[S];
-    sc_cur = sc;
-    float uq[MODE == COL_TOF ? S : 1];
-    if constexpr (!spectral_in) {
-      const float* src = d.rin + (long)c * nT;
+  if constexpr (MODE == COL_TOF) {
+    // the field (envelope: and its Hilbert transform) or its correlation with the reference
+    float u[NC][S];
+    inverse(d.tof_mode == TOF_ENVELOPE ? 0 : 2);
 #pragma unroll
-      for (int i = 0; i < S; ++i) u[i] = (t0 + i < nT) ? src[t0 + i] : 0.f;
-    } else if constexpr (MODE == COL_TOF) {
-      if (d.tof_mode == TOF_ENVELOPE) {
-        inv_spec(u, 0);
-        inv_spec(uq, 1);
-      } else {
-        inv_spec(u, 2);
-      }
-    } else {
-      inv_spec(u, 0);
+    for (int i = 0; i < NC; ++i) samples(u[i], wave * NC + i);
+    if (d.tof_mode == TOF_ENVELOPE) {
+      __syncthreads();
+      inverse(1);
     }
-
-    if constexpr (MODE == COL_TOF) {
-      const bool nz = spectrum_nonzero<64>(sc, M, ln);
-      column_tof<S, 64, false, true>(u, uq, lc, rb, d, c, live, ncols, row, nz);
-    } else {
-      column_realspace<S, 64, false, true, MODE, NLK>(u, lc, d, T, c, live, ncols, row, Nn, nsub_global, wmax);
-    }
-
-    if constexpr (rewrite) {
 #pragma unroll
-      for (int i = 0; i < S; ++i)
-        if (t0 + i < nT) rb[t0 + i] = u[i];
+    for (int i = 0; i < NC; ++i) {
+      const int col = wave * NC + i, c = c0 + col;
+      if (c >= ncols) continue;
+      float uq[S];
+      samples(uq, col);
       wave_sync();
-      // X_m = sum_t u[t] e^{-2 pi i m t / nT}, m = ln, ln + 64, ...
-      float2 res[(NTMAX / 2 + 64) / 64];
+      const bool nz = spectrum_nonzero<64>(spec + (long)c * g.MP, M, lane);
+      column_tof<S, 64, false, true>(u[i], uq, lc, U + col * LSU, d, c, true, ncols, row, nz);
+    }
+    return;
+  } else {
+    if constexpr (spectral_in) inverse(0);
+#pragma unroll 1
+    for (int i = 0; i < NC; ++i) {
+      const int col = wave * NC + i, c = c0 + col;
+      if (c >= ncols) break;
+      float* uc = U + col * LSU;
+      if constexpr (MODE == COL_LOAD) {
+        const float* src = d.rin + (long)c * nT;
+        float mx = 0.f;
+        double e2 = 0.0;
 #pragma unroll
-      for (int q = 0; q < (NTMAX / 2 + 64) / 64; ++q) {
-        const int m = ln + 64 * q;
-        float ax = 0.f, ay = 0.f;
-        if (m <= M) {
-          int idx = 0;
-          for (int t = 0; t < nT; ++t) {
-            const float v = rb[t];
-            const float2 w = s_tw[idx];
-            ax = fmaf(v, w.x, ax);
-            ay = fmaf(v, w.y, ay);
-            idx += m;
-            if (idx >= nT) idx -= nT;
-          }
-          if (m == 0 || (even && m == M)) ay = 0.f;
+        for (int q = 0; q < S; ++q) {
+          const int t = lane + 64 * q;
+          const float v = t < nT ? src[t] : 0.f;
+          mx = fmaxf(mx, fabsf(v));
+          e2 += (double)v * (double)v;
+          if (t < nT) uc[t] = v;
         }
-        res[q] = make_float2(ax, ay);
-      }
-      wave_sync();
+        for (int o = 32; o > 0; o >>= 1) e2 += __shfl_xor(e2, o, 64);
+        if (lane == 0 && d.ibefore) d.ibefore[c] = e2;
+        wmax = fmaxf(wmax, mx);
+        wave_sync();
+      } else if constexpr (MODE == COL_STORE) {
+        float* dst = d.rout + (long)c * nT;
+        for (int t = lane; t < nT; t += 64) dst[t] = uc[t];
+      } else {
+        float u[S];
+        samples(u, col);
+        column_realspace<S, 64, false, true, MODE, NLK>(u, lc, d, T, c, true, ncols, row, Nn, nsub_global, wmax);
+        if constexpr (rewrite) {
+          wave_sync();
 #pragma unroll
-      for (int q = 0; q < (NTMAX / 2 + 64) / 64; ++q) {
-        const int m = ln + 64 * q;
-        if (m <= M) sc[m] = res[q];
+          for (int q = 0; q < S; ++q)
+            if (t0 + q < nT) uc[t0 + q] = u[q];
+          wave_sync();
+        }
+      }
+      if constexpr (rewrite) {
+        // fold in place: e_t at t, o_t at nT - t (o_0 at nT, o_{nT/2} meets a zero row)
+        for (int t = lane; t <= M; t += 64) {
+          const float v = uc[t];
+          if (t == 0) {
+            uc[nT] = 0.f;
+          } else if (2 * t != nT) {
+            const float w = uc[nT - t];
+            uc[t] = v + w;
+            uc[nT - t] = v - w;
+          }
+        }
+      }
+    }
+    if constexpr (rewrite) {
+      __syncthreads();
+      ColAcc<EVEN> a[TW];
+      const float* uc = U + (lane & 15) * LSU;
+#pragma unroll
+      for (int i = 0; i < TW; ++i)
+        if (wave + W * i < dm.R)
+          hm_col_tile<EVEN>(dm, wave + W * i, lane, a[i], [&](int t) { return make_float2(uc[t], uc[nT - t]); });
+      __syncthreads();
+      float2* xc = X + (lane & 15) * LSX;
+#pragma unroll
+      for (int i = 0; i < TW; ++i)
+        if (wave + W * i < dm.R)
+          hm_col_emit<EVEN>(dm, a[i], wave + W * i, lane, [&](int m, float C, float Sn) {
+            xc[m] = make_float2(C, (m == 0 || m == g.nyq) ? 0.f : -Sn);
+          });
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < NC; ++i) {
+        const int col = wave * NC + i, c = c0 + col;
+        if (c < ncols) {
+          float2* sc = spec + (long)c * g.MP;
+          for (int m = lane; m <= M; m += 64) sc[m] = X[col * LSX + m];
+        }
+      }
+    }
+    if constexpr (FIN || MODE == COL_LOAD || MODE == COL_MAXABS) {
+      if (MODE != COL_MAXABS && !d.stats) return;
+      for (int o = 32; o > 0; o >>= 1) wmax = fmaxf(wmax, __shfl_xor(wmax, o, 64));
+      if (lane == 0) s_red[wave] = wmax;
+      __syncthreads();
+      if (tid == 0) {
+        float m = s_red[0];
+        for (int k = 1; k < W; ++k) m = fmaxf(m, s_red[k]);
+        if constexpr (MODE == COL_MAXABS) {
+          d.partial[blockIdx.x] = __float_as_uint(m);
+        } else {
+          unsigned* slot = FIN ? d.stats + row + 1 : d.stats;
+          if (!FIN || row < d.max_rows) atomicMax(slot, __float_as_uint(m));
+        }
       }
     }
   }
+}
 
-  if constexpr (FIN || MODE == COL_LOAD || MODE == COL_MAXABS) {
-    if (MODE != COL_MAXABS && !d.stats) return;
-    for (int o = 32; o > 0; o >>= 1) wmax = fmaxf(wmax, __shfl_xor(wmax, o, 64));
-    if (lane == 0) s_red[wave] = wmax;
-    __syncthreads();
-    if (tid == 0) {
-      float m = s_red[0];
-      for (int k = 1; k < GC_WPB; ++k) m = fmaxf(m, s_red[k]);
-      if constexpr (MODE == COL_MAXABS) {
-        d.partial[blockIdx.x] = __float_as_uint(m);
-      } else {
-        unsigned* slot = FIN ? d.stats + row + 1 : d.stats;
-        if (!FIN || row < d.max_rows) atomicMax(slot, __float_as_uint(m));
-      }
+// Nonlinear update of real columns of any length (COL_RAWNL, no transform): one wave
+// per column, lane ln holds the S contiguous samples from S ln.
+constexpr int GR_WPB = 4;
+template <int S, int NLK>
+__global__ __launch_bounds__(64 * GR_WPB) void k_gcolumn_raw(Tables T, Geom g, ColDesc d) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int nT = g.nT, ncols = g.nX * g.nY, t0 = lane * S;
+  const LaneCol<S, 64, false, true> lc{lane, lane, t0, nT};
+  const double Nn = d.nscale ? d.N * (d.nscale[0] / (d.nscale[1] + 1e-30)) : d.N;
+  float wmax = 0.f;
+  int nsub_global = 1;
+  if constexpr (NLK != NL_NONE) {
+    if (d.subcycle == SUBCYCLE_GLOBAL) {
+      const float gm = __uint_as_float(*d.gmax);
+      bool capped;
+      nsub_global = substeps_for(Nn * (double)gm * d.dz / d.dT, (double)d.cfl_target, gm, &capped);
+      if (capped && blockIdx.x == 0 && threadIdx.x == 0 && d.subcap) atomicAdd(d.subcap, 1u);
     }
+  }
+  for (int c = blockIdx.x * GR_WPB + wave; c < ncols; c += gridDim.x * GR_WPB) {
+    if (d.cflag && d.cflag[c] == 0) continue;
+    const float* src = d.rin + (long)c * nT;
+    float u[S];
+#pragma unroll
+    for (int i = 0; i < S; ++i) u[i] = (t0 + i < nT) ? src[t0 + i] : 0.f;
+    column_realspace<S, 64, false, true, COL_RAWNL, NLK>(u, lc, d, T, c, true, ncols, 0, Nn, nsub_global, wmax);
   }
 }
 

@@ -1,0 +1,164 @@
+// Launchers of the general-size kernels (generic.h).
+#include "generic.h"
+
+#include <algorithm>
+
+#include "generic_launch.h"
+
+namespace ash {
+
+DftMat dft_matrix_shape(int n) {
+  DftMat d{};
+  d.n = n;
+  d.h = n / 2;
+  d.even = n % 2 == 0;
+  auto up = [](int v, int m) { return (v + m - 1) / m * m; };
+  d.rows = d.even ? d.h / 2 + 1 : d.h + 1;
+  d.R = up(d.rows, 16) / 16;
+  d.Ke = up(d.even ? d.h / 2 + 1 : d.h + 1, 8);
+  d.Kp = d.Ke + (d.even ? up((d.h + 1) / 2, 8) : 0);
+  return d;
+}
+size_t dft_matrix_bytes(const DftMat& d) { return (size_t)d.R * (d.Kp / 8) * 64 * sizeof(float4); }
+void dft_matrix_fill(const DftMat& d, const float2* tw, float4* A, hipStream_t s) {
+  const long tot = (long)d.R * (d.Kp / 8) * 64;
+  const dim3 grid((unsigned)std::min<long>((tot + 255) / 256, 1024));
+  if (d.even) hipLaunchKernelGGL(k_dft_matrix<true>, grid, dim3(256), 0, s, d, tw, A);
+  else hipLaunchKernelGGL(k_dft_matrix<false>, grid, dim3(256), 0, s, d, tw, A);
+}
+
+namespace {
+
+// Waves of a line block: four while they take at most three row tiles each, else
+// eight (at most four tiles each at n = 1024).
+int line_waves(const DftMat& d) { return d.R <= 12 ? 4 : 8; }
+int line_tiles(const DftMat& d) { return (d.R + line_waves(d) - 1) / line_waves(d); }
+size_t line_lds(const DftMat& d) { return (size_t)d.Kp * 16 * sizeof(float4); }
+
+template <int T_>
+void launch_inv_sa(float2* spec, const Tables& T, const Geom& g, const EpiDesc& e, dim3 grid, dim3 block, size_t lds,
+                   hipStream_t s) {
+  if (T.dmx.even) hipLaunchKernelGGL((k_gx_inv_sa<true, T_>), grid, block, lds, s, spec, T, g, e);
+  else hipLaunchKernelGGL((k_gx_inv_sa<false, T_>), grid, block, lds, s, spec, T, g, e);
+}
+
+template <int T_, bool PRECISE>
+void launch_ypass(float2* spec, const Tables& T, const Geom& g, const OpDesc& op, dim3 grid, dim3 block, size_t lds,
+                  hipStream_t s) {
+  if (T.dmy.even) hipLaunchKernelGGL((k_gy_pass<true, T_, PRECISE>), grid, block, lds, s, spec, T, g, op);
+  else hipLaunchKernelGGL((k_gy_pass<false, T_, PRECISE>), grid, block, lds, s, spec, T, g, op);
+}
+template <int T_>
+void launch_ypass_p(float2* spec, const Tables& T, const Geom& g, const OpDesc& op, dim3 grid, dim3 block, size_t lds,
+                    hipStream_t s) {
+  if (op.precise) launch_ypass<T_, true>(spec, T, g, op, grid, block, lds, s);
+  else launch_ypass<T_, false>(spec, T, g, op, grid, block, lds, s);
+}
+
+}  // namespace
+
+void gen_xfwd(float2* spec, const Tables& T, const Geom& g, hipStream_t s) {
+  const dim3 grid(g.nY * g.nfb), block(64 * line_waves(T.dmx));
+  if (T.dmx.even) hipLaunchKernelGGL(k_gx_fwd<true>, grid, block, line_lds(T.dmx), s, spec, T, g);
+  else hipLaunchKernelGGL(k_gx_fwd<false>, grid, block, line_lds(T.dmx), s, spec, T, g);
+}
+
+void gen_xinv(int epi, float2* spec, const Tables& T, const Geom& g, const EpiDesc& e, hipStream_t s) {
+  const dim3 grid(g.nY * g.nfb), block(64 * line_waves(T.dmx));
+  const size_t lds = line_lds(T.dmx);
+  if (epi == 2) {
+    switch (line_tiles(T.dmx)) {
+      case 1: launch_inv_sa<1>(spec, T, g, e, grid, block, lds, s); break;
+      case 2: launch_inv_sa<2>(spec, T, g, e, grid, block, lds, s); break;
+      case 3: launch_inv_sa<3>(spec, T, g, e, grid, block, lds, s); break;
+      default: launch_inv_sa<4>(spec, T, g, e, grid, block, lds, s); break;
+    }
+  } else if (epi == 1) {
+    if (T.dmx.even) hipLaunchKernelGGL((k_gx_inv<true, 1>), grid, block, lds, s, spec, T, g, e);
+    else hipLaunchKernelGGL((k_gx_inv<false, 1>), grid, block, lds, s, spec, T, g, e);
+  } else {
+    if (T.dmx.even) hipLaunchKernelGGL((k_gx_inv<true, 0>), grid, block, lds, s, spec, T, g, e);
+    else hipLaunchKernelGGL((k_gx_inv<false, 0>), grid, block, lds, s, spec, T, g, e);
+  }
+}
+
+void gen_ypass(float2* spec, const Tables& T, const Geom& g, const OpDesc& op, hipStream_t s) {
+  const dim3 grid(g.nX * g.nfb), block(64 * line_waves(T.dmy));
+  const size_t lds = line_lds(T.dmy);
+  switch (line_tiles(T.dmy)) {
+    case 1: launch_ypass_p<1>(spec, T, g, op, grid, block, lds, s); break;
+    case 2: launch_ypass_p<2>(spec, T, g, op, grid, block, lds, s); break;
+    case 3: launch_ypass_p<3>(spec, T, g, op, grid, block, lds, s); break;
+    default: launch_ypass_p<4>(spec, T, g, op, grid, block, lds, s); break;
+  }
+}
+
+void gen_ypower(const float2* spec, const Tables& T, const Geom& g, double* acc, hipStream_t s) {
+  const dim3 grid(g.nX * g.nfb), block(64 * line_waves(T.dmy));
+  if (T.dmy.even) hipLaunchKernelGGL(k_gy_power<true>, grid, block, line_lds(T.dmy), s, spec, T, g, acc);
+  else hipLaunchKernelGGL(k_gy_power<false>, grid, block, line_lds(T.dmy), s, spec, T, g, acc);
+}
+
+void gen_ysa(float2* spec, const Tables& T, const Geom& g, const ScreenDesc& sd, hipStream_t s) {
+  const size_t lds = (size_t)ysa_rows(g.nY, sd.band, sd.phase != nullptr) * LF * sizeof(float2);
+  hipLaunchKernelGGL(k_gy_sa, dim3(g.nX * g.nfb), dim3(256), lds, s, spec, T, g, sd);
+}
+
+int gen_column_blocks(int ncols) { return (ncols + GC_COLS - 1) / GC_COLS; }
+
+namespace {
+
+template <int S, int MODE, int NLK>
+void launch_gcol_SMN(float2* spec, const Tables& T, const Geom& g, const ColDesc& cd, hipStream_t s) {
+  const dim3 grid(gen_column_blocks(g.nX * g.nY)), block(64 * gcol_waves(S));
+  const size_t lds = gcol_lds_bytes(g.nT);
+  if (T.dmt.even) hipLaunchKernelGGL((k_gcolumn<S, true, MODE, NLK>), grid, block, lds, s, spec, T, g, cd);
+  else hipLaunchKernelGGL((k_gcolumn<S, false, MODE, NLK>), grid, block, lds, s, spec, T, g, cd);
+}
+template <int S, int NLK>
+void launch_graw(const Tables& T, const Geom& g, const ColDesc& cd, hipStream_t s) {
+  const int blocks = std::min((g.nX * g.nY + GR_WPB - 1) / GR_WPB, 2048);
+  hipLaunchKernelGGL((k_gcolumn_raw<S, NLK>), dim3(blocks), dim3(64 * GR_WPB), 0, s, T, g, cd);
+}
+template <int S>
+void launch_gcol_S(float2* spec, const Tables& T, const Geom& g, const ColDesc& cd, hipStream_t s) {
+  switch (cd.mode) {
+    case COL_LOAD: launch_gcol_SMN<S, COL_LOAD, NL_NONE>(spec, T, g, cd, s); break;
+    case COL_NL:  // (the march's updates; KT_MINMOD is an operator of its own)
+      if (cd.nl == NL_KT) launch_gcol_SMN<S, COL_NL, NL_KT>(spec, T, g, cd, s);
+      else if (cd.nl == NL_TVD) launch_gcol_SMN<S, COL_NL, NL_TVD>(spec, T, g, cd, s);
+      else launch_gcol_SMN<S, COL_NL, NL_RUSANOV>(spec, T, g, cd, s);
+      break;
+    case COL_TAPER: launch_gcol_SMN<S, COL_TAPER, NL_NONE>(spec, T, g, cd, s); break;
+    case COL_FINAL:
+      if (cd.n_src > 0 || cd.smask) launch_gcol_SMN<S, COL_FINAL_SRC, NL_NONE>(spec, T, g, cd, s);
+      else launch_gcol_SMN<S, COL_FINAL, NL_NONE>(spec, T, g, cd, s);
+      break;
+    case COL_STORE: launch_gcol_SMN<S, COL_STORE, NL_NONE>(spec, T, g, cd, s); break;
+    case COL_RAWNL:
+      switch (cd.nl) {
+        case NL_KT: launch_graw<S, NL_KT>(T, g, cd, s); break;
+        case NL_KT_MINMOD: launch_graw<S, NL_KT_MINMOD>(T, g, cd, s); break;
+        case NL_RUSANOV: launch_graw<S, NL_RUSANOV>(T, g, cd, s); break;
+        case NL_TVD: launch_graw<S, NL_TVD>(T, g, cd, s); break;
+        default: launch_graw<S, NL_NONE>(T, g, cd, s); break;
+      }
+      break;
+    case COL_MAXABS: launch_gcol_SMN<S, COL_MAXABS, NL_NONE>(spec, T, g, cd, s); break;
+    case COL_TOF: launch_gcol_SMN<S, COL_TOF, NL_NONE>(spec, T, g, cd, s); break;
+    default: break;
+  }
+}
+
+}  // namespace
+
+void gen_column(float2* spec, const Tables& T, const Geom& g, const ColDesc& cd, hipStream_t s) {
+  // S real samples per lane, 64 S >= nT
+  if (g.nT <= 128) launch_gcol_S<2>(spec, T, g, cd, s);
+  else if (g.nT <= 256) launch_gcol_S<4>(spec, T, g, cd, s);
+  else if (g.nT <= 512) launch_gcol_S<8>(spec, T, g, cd, s);
+  else if (g.nT <= 1024) launch_gcol_S<16>(spec, T, g, cd, s);
+  else launch_gcol_S<32>(spec, T, g, cd, s);
+}
+
+}  // namespace ash

@@ -109,6 +109,14 @@ __device__ __forceinline__ void gst(float2* base, uint32_t off, float2 v) {
 // ---------------------------------------------------------------------------
 // Per-plan constant tables (device memory, built on the host in FP64).
 // ---------------------------------------------------------------------------
+// DFT matrix of an axis outside the FFT set (generic.h): n = length, h = n / 2, `rows`
+// matrix rows in R tiles of 16, Kp matrix columns (multiple of 8) of which the first
+// Ke take the even input positions when n is even (all of them otherwise).
+struct DftMat {
+  const float4* A;
+  int n, h, rows, R, Ke, Kp, even;
+};
+
 struct Tables {
   const double* kx;      // [nX] natural-order kx (ASS:403-408 centred grid)
   const double* ky;      // [nY]
@@ -131,9 +139,8 @@ struct Tables {
   const float2* twx;     // [nX] exp(-2 pi i k / nX)
   const float2* twy;     // [nY]
   const float2* twc;     // column-transform pass twiddles: forward passes, then inverse passes
-  const float2* twgx;    // [nX] exp(-2 pi i k / nX), general-size x kernels
-  const float2* twgy;    // [nY]
-  const float2* twgt;    // [nT] exp(-2 pi i k / nT): column packing, general-length column kernel
+  const float2* twgt;    // [nT] exp(-2 pi i k / nT): column packing
+  DftMat dmx, dmy, dmt;  // axes that run the general-size kernels
 };
 
 struct Geom {
@@ -749,7 +756,7 @@ __device__ __forceinline__ float tone_burst(double tm, double w0, double ncyc, d
 }
 
 // Dense field of a sparse source: out[c][t] = mask[c] ? tone_burst(taxis[t] - delay[c]) : 0.
-__global__ __launch_bounds__(256) void k_source_field(const unsigned char* __restrict__ mask,
+static __global__ __launch_bounds__(256) void k_source_field(const unsigned char* __restrict__ mask,
                                                       const double* __restrict__ delay,
                                                       const double* __restrict__ taxis, long ncols, int nT,
                                                       double w0, double ncyc, double cexp, double p0,
@@ -870,16 +877,16 @@ __device__ __forceinline__ void kt_dflux_lane(const float* h, bool first, bool l
 
 namespace ash {
 
-__global__ void k_set_row(int* row, int v) { *row = v; }
-__global__ void k_set_u32(unsigned* a, unsigned v) { *a = v; }
-__global__ void k_copy_u32x2(const unsigned* a, const unsigned* b, unsigned* out) { out[0] = *a; out[1] = *b; }
+static __global__ void k_set_row(int* row, int v) { *row = v; }
+static __global__ void k_set_u32(unsigned* a, unsigned v) { *a = v; }
+static __global__ void k_copy_u32x2(const unsigned* a, const unsigned* b, unsigned* out) { out[0] = *a; out[1] = *b; }
 
 // Partial maxima of |u| over a real field of ncols columns of nT samples: block b
 // covers columns [64 b, 64 b + 64) and writes partial[b] (float bits).  The
 // maximum is taken on the bit patterns of |u|, which order like the values and
 // put a NaN above +inf, so a NaN sample shows in the result.
 constexpr int ABSMAX_COLS = 64;
-__global__ __launch_bounds__(256) void k_absmax_cols(const float* __restrict__ u, long ncols, int nT,
+static __global__ __launch_bounds__(256) void k_absmax_cols(const float* __restrict__ u, long ncols, int nT,
                                                      unsigned* __restrict__ partial) {
   __shared__ unsigned s_red[4];
   const long c0 = (long)blockIdx.x * ABSMAX_COLS;
@@ -895,7 +902,7 @@ __global__ __launch_bounds__(256) void k_absmax_cols(const float* __restrict__ u
 
 // out[0] = max of n partial maxima (float bits; all finite or +inf values are
 // non-negative floats, whose bit patterns order like the values).  One block.
-__global__ __launch_bounds__(1024) void k_reduce_max(const unsigned* __restrict__ partial, int n,
+static __global__ __launch_bounds__(1024) void k_reduce_max(const unsigned* __restrict__ partial, int n,
                                                      unsigned* __restrict__ out) {
   __shared__ unsigned s_red[16];
   unsigned m = 0u;
@@ -909,7 +916,7 @@ __global__ __launch_bounds__(1024) void k_reduce_max(const unsigned* __restrict_
     out[0] = r;
   }
 }
-__global__ void k_zero2(double* a) { a[0] = 0.0; a[1] = 0.0; }
+static __global__ void k_zero2(double* a) { a[0] = 0.0; a[1] = 0.0; }
 
 // y transform of one (kx row, f block) tile and the power-weighted obliquity
 // sums of its plane-wave content (ASS:630-643): acc[0] += sum P k/k_z and
@@ -966,6 +973,6 @@ __global__ __launch_bounds__(LNT) void k_ypower(const float2* __restrict__ spec,
     atomicAdd(acc + 1, b);
   }
 }
-__global__ void k_advance_row(int* row) { *row += 1; }
+static __global__ void k_advance_row(int* row) { *row += 1; }
 
 }  // namespace ash
