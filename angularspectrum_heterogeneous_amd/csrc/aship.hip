@@ -374,8 +374,8 @@ int build_tables(ash_plan* p) {
   if ((rc = upload(p, twiddles(nY), &p->T.twy))) return rc;
   if ((rc = upload(p, twiddles(nT), &p->T.twgt))) return rc;
   // DFT matrices of the axes outside the FFT set, filled on the device
-  auto matrix = [p](int n, const float2* tw, DftMat* m) -> int {
-    *m = dft_matrix_shape(n);
+  auto matrix = [p](int n, bool columns, const float2* tw, DftMat* m) -> int {
+    *m = dft_matrix_shape(n, columns);
     const size_t bytes = dft_matrix_bytes(*m);
     void* a = nullptr;
     p->allocs.reserve(p->allocs.size() + 1);
@@ -386,9 +386,9 @@ int build_tables(ash_plan* p) {
     dft_matrix_fill(*m, tw, (float4*)a, nullptr);
     return ASH_OK;
   };
-  if (p->gen_x && (rc = matrix(nX, p->T.twx, &p->T.dmx))) return rc;
-  if (p->gen_y && (rc = matrix(nY, p->T.twy, &p->T.dmy))) return rc;
-  if (p->gen_t && (rc = matrix(nT, p->T.twgt, &p->T.dmt))) return rc;
+  if (p->gen_x && (rc = matrix(nX, false, p->T.twx, &p->T.dmx))) return rc;
+  if (p->gen_y && (rc = matrix(nY, false, p->T.twy, &p->T.dmy))) return rc;
+  if (p->gen_t && (rc = matrix(nT, true, p->T.twgt, &p->T.dmt))) return rc;
   if (!p->gen_t) {
     // pass-major twiddles of the column transform, [r * Ns + k] = W_{Ns R}^{k r}
     auto radices = [&](bool inv) {

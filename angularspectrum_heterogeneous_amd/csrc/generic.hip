@@ -7,7 +7,7 @@
 
 namespace ash {
 
-DftMat dft_matrix_shape(int n) {
+DftMat dft_matrix_shape(int n, bool columns) {
   DftMat d{};
   d.n = n;
   d.h = n / 2;
@@ -17,6 +17,8 @@ DftMat dft_matrix_shape(int n) {
   d.R = up(d.rows, 16) / 16;
   d.Ke = up(d.even ? d.h / 2 + 1 : d.h + 1, 8);
   d.Kp = d.Ke + (d.even ? up((d.h + 1) / 2, 8) : 0);
+  d.rs = columns ? d.Kp / 8 * 64 : 64;
+  d.gs = columns ? 64 : d.R * 64;
   return d;
 }
 size_t dft_matrix_bytes(const DftMat& d) { return (size_t)d.R * (d.Kp / 8) * 64 * sizeof(float4); }
@@ -35,68 +37,47 @@ int line_waves(const DftMat& d) { return d.R <= 12 ? 4 : 8; }
 int line_tiles(const DftMat& d) { return (d.R + line_waves(d) - 1) / line_waves(d); }
 size_t line_lds(const DftMat& d) { return (size_t)d.Kp * 16 * sizeof(float4); }
 
-template <int T_>
-void launch_inv_sa(float2* spec, const Tables& T, const Geom& g, const EpiDesc& e, dim3 grid, dim3 block, size_t lds,
-                   hipStream_t s) {
-  if (T.dmx.even) hipLaunchKernelGGL((k_gx_inv_sa<true, T_>), grid, block, lds, s, spec, T, g, e);
-  else hipLaunchKernelGGL((k_gx_inv_sa<false, T_>), grid, block, lds, s, spec, T, g, e);
-}
-
-template <int T_, bool PRECISE>
-void launch_ypass(float2* spec, const Tables& T, const Geom& g, const OpDesc& op, dim3 grid, dim3 block, size_t lds,
-                  hipStream_t s) {
-  if (T.dmy.even) hipLaunchKernelGGL((k_gy_pass<true, T_, PRECISE>), grid, block, lds, s, spec, T, g, op);
-  else hipLaunchKernelGGL((k_gy_pass<false, T_, PRECISE>), grid, block, lds, s, spec, T, g, op);
-}
-template <int T_>
-void launch_ypass_p(float2* spec, const Tables& T, const Geom& g, const OpDesc& op, dim3 grid, dim3 block, size_t lds,
-                    hipStream_t s) {
-  if (op.precise) launch_ypass<T_, true>(spec, T, g, op, grid, block, lds, s);
-  else launch_ypass<T_, false>(spec, T, g, op, grid, block, lds, s);
-}
+// CALL with T_ = the most row tiles of a wave and EVEN = the length's parity
+#define DISPATCH_TILES(d, ...)                                       \
+  do {                                                               \
+    switch (line_tiles(d) * 2 + (d).even) {                          \
+      case 2: { constexpr int T_ = 1; constexpr bool EVEN = false; __VA_ARGS__; } break; \
+      case 3: { constexpr int T_ = 1; constexpr bool EVEN = true; __VA_ARGS__; } break;  \
+      case 4: { constexpr int T_ = 2; constexpr bool EVEN = false; __VA_ARGS__; } break; \
+      case 5: { constexpr int T_ = 2; constexpr bool EVEN = true; __VA_ARGS__; } break;  \
+      case 6: { constexpr int T_ = 3; constexpr bool EVEN = false; __VA_ARGS__; } break; \
+      case 7: { constexpr int T_ = 3; constexpr bool EVEN = true; __VA_ARGS__; } break;  \
+      default: { constexpr int T_ = 4; constexpr bool EVEN = false; __VA_ARGS__; } break; \
+    }                                                                \
+  } while (0)
 
 }  // namespace
 
 void gen_xfwd(float2* spec, const Tables& T, const Geom& g, hipStream_t s) {
   const dim3 grid(g.nY * g.nfb), block(64 * line_waves(T.dmx));
-  if (T.dmx.even) hipLaunchKernelGGL(k_gx_fwd<true>, grid, block, line_lds(T.dmx), s, spec, T, g);
-  else hipLaunchKernelGGL(k_gx_fwd<false>, grid, block, line_lds(T.dmx), s, spec, T, g);
+  const size_t lds = line_lds(T.dmx);
+  DISPATCH_TILES(T.dmx, hipLaunchKernelGGL((k_gx_fwd<EVEN, T_>), grid, block, lds, s, spec, T, g));
 }
 
 void gen_xinv(int epi, float2* spec, const Tables& T, const Geom& g, const EpiDesc& e, hipStream_t s) {
   const dim3 grid(g.nY * g.nfb), block(64 * line_waves(T.dmx));
   const size_t lds = line_lds(T.dmx);
-  if (epi == 2) {
-    switch (line_tiles(T.dmx)) {
-      case 1: launch_inv_sa<1>(spec, T, g, e, grid, block, lds, s); break;
-      case 2: launch_inv_sa<2>(spec, T, g, e, grid, block, lds, s); break;
-      case 3: launch_inv_sa<3>(spec, T, g, e, grid, block, lds, s); break;
-      default: launch_inv_sa<4>(spec, T, g, e, grid, block, lds, s); break;
-    }
-  } else if (epi == 1) {
-    if (T.dmx.even) hipLaunchKernelGGL((k_gx_inv<true, 1>), grid, block, lds, s, spec, T, g, e);
-    else hipLaunchKernelGGL((k_gx_inv<false, 1>), grid, block, lds, s, spec, T, g, e);
-  } else {
-    if (T.dmx.even) hipLaunchKernelGGL((k_gx_inv<true, 0>), grid, block, lds, s, spec, T, g, e);
-    else hipLaunchKernelGGL((k_gx_inv<false, 0>), grid, block, lds, s, spec, T, g, e);
-  }
+  if (epi == 2) DISPATCH_TILES(T.dmx, hipLaunchKernelGGL((k_gx_inv_sa<EVEN, T_>), grid, block, lds, s, spec, T, g, e));
+  else if (epi == 1) DISPATCH_TILES(T.dmx, hipLaunchKernelGGL((k_gx_inv<EVEN, T_, 1>), grid, block, lds, s, spec, T, g, e));
+  else DISPATCH_TILES(T.dmx, hipLaunchKernelGGL((k_gx_inv<EVEN, T_, 0>), grid, block, lds, s, spec, T, g, e));
 }
 
 void gen_ypass(float2* spec, const Tables& T, const Geom& g, const OpDesc& op, hipStream_t s) {
   const dim3 grid(g.nX * g.nfb), block(64 * line_waves(T.dmy));
   const size_t lds = line_lds(T.dmy);
-  switch (line_tiles(T.dmy)) {
-    case 1: launch_ypass_p<1>(spec, T, g, op, grid, block, lds, s); break;
-    case 2: launch_ypass_p<2>(spec, T, g, op, grid, block, lds, s); break;
-    case 3: launch_ypass_p<3>(spec, T, g, op, grid, block, lds, s); break;
-    default: launch_ypass_p<4>(spec, T, g, op, grid, block, lds, s); break;
-  }
+  if (op.precise) DISPATCH_TILES(T.dmy, hipLaunchKernelGGL((k_gy_pass<EVEN, T_, true>), grid, block, lds, s, spec, T, g, op));
+  else DISPATCH_TILES(T.dmy, hipLaunchKernelGGL((k_gy_pass<EVEN, T_, false>), grid, block, lds, s, spec, T, g, op));
 }
 
 void gen_ypower(const float2* spec, const Tables& T, const Geom& g, double* acc, hipStream_t s) {
   const dim3 grid(g.nX * g.nfb), block(64 * line_waves(T.dmy));
-  if (T.dmy.even) hipLaunchKernelGGL(k_gy_power<true>, grid, block, line_lds(T.dmy), s, spec, T, g, acc);
-  else hipLaunchKernelGGL(k_gy_power<false>, grid, block, line_lds(T.dmy), s, spec, T, g, acc);
+  const size_t lds = line_lds(T.dmy);
+  DISPATCH_TILES(T.dmy, hipLaunchKernelGGL((k_gy_power<EVEN, T_>), grid, block, lds, s, spec, T, g, acc));
 }
 
 void gen_ysa(float2* spec, const Tables& T, const Geom& g, const ScreenDesc& sd, hipStream_t s) {
@@ -111,7 +92,7 @@ namespace {
 template <int S, int MODE, int NLK>
 void launch_gcol_SMN(float2* spec, const Tables& T, const Geom& g, const ColDesc& cd, hipStream_t s) {
   const dim3 grid(gen_column_blocks(g.nX * g.nY)), block(64 * gcol_waves(S));
-  const size_t lds = gcol_lds_bytes(g.nT);
+  const size_t lds = (size_t)GC_COLS * gcol_pitch(g.nT, S) * sizeof(float);
   if (T.dmt.even) hipLaunchKernelGGL((k_gcolumn<S, true, MODE, NLK>), grid, block, lds, s, spec, T, g, cd);
   else hipLaunchKernelGGL((k_gcolumn<S, false, MODE, NLK>), grid, block, lds, s, spec, T, g, cd);
 }

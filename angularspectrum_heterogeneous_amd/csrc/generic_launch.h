@@ -4,8 +4,9 @@
 
 namespace ash {
 
-// Shape of the DFT matrix of an axis of length n (A is null), and the device memory it takes.
-DftMat dft_matrix_shape(int n);
+// Shape of the DFT matrix of a line axis or the column axis of length n (A is null), and
+// the device memory it takes.
+DftMat dft_matrix_shape(int n, bool columns);
 size_t dft_matrix_bytes(const DftMat& d);
 // Fills A (dft_matrix_bytes on the device) from the axis' full-length twiddle table.
 void dft_matrix_fill(const DftMat& d, const float2* tw, float4* A, hipStream_t s);

@@ -111,10 +111,12 @@ __device__ __forceinline__ void gst(float2* base, uint32_t off, float2 v) {
 // ---------------------------------------------------------------------------
 // DFT matrix of an axis outside the FFT set (generic.h): n = length, h = n / 2, `rows`
 // matrix rows in R tiles of 16, Kp matrix columns (multiple of 8) of which the first
-// Ke take the even input positions when n is even (all of them otherwise).
+// Ke take the even input positions when n is even (all of them otherwise).  Entry
+// (row tile rt, column group g) starts at A + rt * rs + g * gs.
 struct DftMat {
   const float4* A;
   int n, h, rows, R, Ke, Kp, even;
+  int rs, gs;
 };
 
 struct Tables {
