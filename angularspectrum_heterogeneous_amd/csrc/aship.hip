@@ -201,6 +201,8 @@ struct ash_net {
   uint16_t* Dg[2] = {};     // back-propagated gradients, same shape
   float* y = nullptr;       // [max_cols][nT]
   float* amp = nullptr;     // [max_cols]
+  float4* part = nullptr;   // per-block partial weight gradients [NLAY][part_blocks][WG_QUADS]
+  int part_blocks = 0;      // blocks of a full batch (max_cols)
   std::vector<void*> allocs;
 };
 
@@ -1654,6 +1656,8 @@ int ash_net_create(int32_t nT, int32_t max_cols, ash_net** out) try {
   for (int j = 0; j < 2 && !rc; ++j) rc = alloc((void**)&n->Dg[j], act * 2);
   if (!rc) rc = alloc((void**)&n->y, (size_t)max_cols * nT * 4);
   if (!rc) rc = alloc((void**)&n->amp, (size_t)max_cols * 4);
+  n->part_blocks = net::wgrad_blocks((long)max_cols * nT / 32);
+  if (!rc) rc = alloc((void**)&n->part, (size_t)net::NLAY * n->part_blocks * net::WG_QUADS * sizeof(float4));
   if (!rc) {
     // trainable entries: W1 input channels 0-1, W4 and b4 output channel 0, all of layers 2-3
     std::vector<float> mk(np, 1.f);
@@ -1732,20 +1736,21 @@ int ash_net_loss_grad(ash_net* n, const float* u, const float* un, int32_t ncols
   const int nT = n->nT;
   int rc = net_forward(n, u, ncols, n->y, n->amp, s);
   if (rc) return rc;
-  hipLaunchKernelGGL(net::k_net_loss, dim3((nT + 255) / 256, ncols), dim3(256), 0, s, n->y, u, un, n->amp, nT,
+  hipLaunchKernelGGL(net::k_net_loss, dim3(ncols), dim3(256), 0, s, n->y, u, un, n->amp, nT,
                      (float)c, (float)(1.0 / ((double)ncols * nT)), n->Dg[0], loss);
-  HIP_TRY(hipMemsetAsync(grads, 0, net::PARAM_COUNT * 4, s));
   const dim3 grid(nT / net::TT, ncols);
+  const int nb = net::wgrad_blocks((long)ncols * nT / 32);  // <= part_blocks
+  const long stride = (long)n->part_blocks * net::WG_QUADS;
   int cur = 0;
   for (int j = 3; j >= 0; --j) {
-    float* gW = grads + j * net::LAYER_SIZE;
-    hipLaunchKernelGGL(net::k_net_wgrad, grid, dim3(256), 0, s, n->Dg[cur], n->X[j], nT, gW, gW + net::W_SIZE);
+    hipLaunchKernelGGL(net::k_net_wgrad, dim3(nb), dim3(256), 0, s, n->Dg[cur], n->X[j], nT, ncols, n->part + j * stride);
     if (j > 0) {
       hipLaunchKernelGGL(net::k_net_conv<2>, grid, dim3(256), 0, s, n->Dg[cur], nT, n->Wt + j * net::W_SIZE,
                          (const float*)nullptr, n->X[j], n->Dg[1 - cur], (float*)nullptr);
       cur = 1 - cur;
     }
   }
+  hipLaunchKernelGGL(net::k_net_wgrad_sum, dim3(net::WG_QUADS / 32, net::NLAY), dim3(256), 0, s, n->part, nb, stride, grads);
   return check_launch();
 } catch (...) {
   return caught_exception();

@@ -297,7 +297,7 @@ __global__ __launch_bounds__(INF_THREADS) void k_net_infer(float* __restrict__ R
 // Training path: per-layer kernels over a batch of B columns, activations in
 // global memory as [B][nT][32] bf16.
 // ---------------------------------------------------------------------------
-constexpr int TT = 128;  // outputs per block of the per-layer kernels
+constexpr int TT = 256;  // outputs per block of the per-layer kernels
 
 // Features and per-column amplitude: one block (256 threads) per column.
 __global__ __launch_bounds__(256) void k_net_feat(const float* __restrict__ u, int nT, u16* __restrict__ X0,
@@ -313,17 +313,23 @@ __global__ __launch_bounds__(256) void k_net_feat(const float* __restrict__ u, i
   const float A = fmaxf(fmaxf(sred[0], sred[1]), fmaxf(sred[2], sred[3]));
   if (tid == 0) amp[b] = A;
   const float As = A > 0.f ? A : 1.f;
-  for (int t = tid; t < nT; t += 256) {
-    const float x = g[t] / As;
-    uint4* row = reinterpret_cast<uint4*>(X0 + ((long)b * nT + t) * C);
-    row[0] = make_uint4((uint32_t)f2bf(x) | ((uint32_t)f2bf(x * x) << 16), 0u, 0u, 0u);
-    row[1] = row[2] = row[3] = make_uint4(0u, 0u, 0u, 0u);
+  // four threads per 64-byte row, so a wave stores 1 KB in a row (one thread per row
+  // left each store instruction 64 bytes apart per lane: 16.3 -> 9.4 us at 256x1024)
+  uint4* rows = reinterpret_cast<uint4*>(X0 + (long)b * nT * C);
+  for (int i = tid; i < nT * 4; i += 256) {
+    uint4 v = make_uint4(0u, 0u, 0u, 0u);
+    if ((i & 3) == 0) {
+      const float x = g[i >> 2] / As;
+      v.x = (uint32_t)f2bf(x) | ((uint32_t)f2bf(x * x) << 16);
+    }
+    rows[i] = v;
   }
 }
 
 // MODE 0: out = bf16(relu(conv + bias)); MODE 1: y = conv[ch 0] + bias[0] (float);
 // MODE 2: out = bf16(conv * (mask > 0)) (input gradient through a relu).
-// grid (nT / TT, B), 256 threads.
+// grid (nT / TT, B), 256 threads; TT = 256 outputs per block, so the 18 KB of weights
+// that every wave holds serve four 16-position tiles (17.5 -> 14.4 us against two).
 template <int MODE>
 __global__ __launch_bounds__(256) void k_net_conv(const u16* __restrict__ in, int nT, const u16* __restrict__ W,
                                                   const float* __restrict__ bias, const u16* __restrict__ mask,
@@ -374,78 +380,199 @@ __global__ __launch_bounds__(256) void k_net_conv(const u16* __restrict__ in, in
 }
 
 // Loss (mean square over all samples) and its gradient, in channel 0 of dY:
-// y* = (u_next - u) / (c A^2).  grid (nT / 256, B), 256 threads.
+// y* = (u_next - u) / (c A^2).  One block (256 threads) per column: one double atomic
+// per column on the loss (one per 256 samples queued on its address: 18.4 -> 9.4 us at
+// 256x1024).
 __global__ __launch_bounds__(256) void k_net_loss(const float* __restrict__ y, const float* __restrict__ u,
                                                   const float* __restrict__ un, const float* __restrict__ amp,
                                                   int nT, float c, float inv_count, u16* __restrict__ dY,
                                                   double* __restrict__ loss) {
   __shared__ double sred[4];
-  const int b = blockIdx.y, t = blockIdx.x * 256 + threadIdx.x;
+  __shared__ float sg[256];
+  const int b = blockIdx.x, tid = threadIdx.x;
+  const float A = amp[b];
+  const float s = A > 0.f ? c * A * A : 1.f;
   double l2 = 0.0;
-  if (t < nT) {
-    const long i = (long)b * nT + t;
-    const float A = amp[b];
-    const float s = A > 0.f ? c * A * A : 1.f;
+  for (int t0 = 0; t0 < nT; t0 += 256) {  // nT is a multiple of 256
+    const long i = (long)b * nT + t0 + tid;
     const float ys = A > 0.f ? (un[i] - u[i]) / s : 0.f;
     const float r = y[i] - ys;
-    l2 = (double)r * (double)r;
-    uint4* row = reinterpret_cast<uint4*>(dY + i * C);
-    row[0] = make_uint4((uint32_t)f2bf(2.f * r * inv_count), 0u, 0u, 0u);
-    row[1] = row[2] = row[3] = make_uint4(0u, 0u, 0u, 0u);
+    l2 += (double)r * (double)r;
+    __syncthreads();  // the previous rows are written
+    sg[tid] = 2.f * r * inv_count;
+    __syncthreads();
+    // the rows of dY by four threads each (as k_net_feat)
+    uint4* rows = reinterpret_cast<uint4*>(dY + ((long)b * nT + t0) * C);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int e = tid + 256 * k;
+      rows[e] = make_uint4((e & 3) == 0 ? (uint32_t)f2bf(sg[e >> 2]) : 0u, 0u, 0u, 0u);
+    }
   }
   for (int o = 32; o > 0; o >>= 1) l2 += __shfl_xor(l2, o, 64);
-  if ((threadIdx.x & 63) == 0) sred[threadIdx.x >> 6] = l2;
+  if ((tid & 63) == 0) sred[tid >> 6] = l2;
   __syncthreads();
-  if (threadIdx.x == 0) atomicAdd(loss, (sred[0] + sred[1] + sred[2] + sred[3]) * (double)inv_count);
+  if (tid == 0) atomicAdd(loss, (sred[0] + sred[1] + sred[2] + sred[3]) * (double)inv_count);
 }
 
 // Weight and bias gradients of one layer on the matrix cores: for every tap k,
-// gW[co][ci][k] += sum_t D[t][co] X[t+k-4][ci] is a 32 x 32 product with the
-// sum over t as the reduction dimension.  The block's tiles are staged in LDS
-// transposed ([channel][t], bf16): A operands (8 consecutive t of one co) are
-// single 16-byte reads; B operands start at an odd offset for odd k and are
-// assembled from 2-byte reads.  grid (nT / TT, B), 256 threads.
-constexpr int WS_D = TT + 8;   // row stride of dT (272 B, a multiple of 16 B)
-constexpr int WS_X = TT + 16;  // row stride of xT (288 B)
+// gW[co][ci][k] = sum_t D[t][co] X[t+k-4][ci] is a 32 x 32 product with the sum over
+// t as the reduction dimension, 32 samples per product.
+//
+// A lane (p = lane % 16, g = lane / 16) reads the channel pair 2p, 2p+1 of rows
+// 8g .. 8g+7 of D and of rows 8g-4 .. 8g+11 of X straight from the [t][32] activations
+// and splits the pairs with byte permutes: the even channels form one 16-row operand,
+// the odd ones another, so no transpose through LDS is needed, and the nine taps are
+// nine windows of the same registers.  A wave keeps all 9 x 2 x 2 tiles (and the bias
+// sums: a product with ones) in accumulators over its share of the samples; the four
+// waves of a block add up in LDS, and the block writes one partial that
+// k_net_wgrad_sum adds over the blocks, in a fixed order.
+//
+// At 256 columns of 1024: 34 MB read per layer.  The earlier form (a block per 128
+// samples, transposed 2-byte LDS tiles, one float atomic per entry and block: 19
+// million) took 897 us a layer, this one 19.5.
+constexpr int WG_TILES = KW * 4 + 2;           // 16 x 16 tiles of a partial: [tap][co parity][ci parity], bias [co parity]
+constexpr int WG_QUADS = WG_TILES * 64;        // float4 entries of a partial
+constexpr int WG_MAX_BLOCKS = 256;
+// blocks for n 32-sample groups: at least four groups per wave
+__host__ __device__ inline int wgrad_blocks(long groups) {
+  const long b = groups / 16;
+  return b < 1 ? 1 : b > WG_MAX_BLOCKS ? WG_MAX_BLOCKS : (int)b;
+}
+
 __global__ __launch_bounds__(256) void k_net_wgrad(const u16* __restrict__ Dg, const u16* __restrict__ X, int nT,
-                                                   float* __restrict__ gW, float* __restrict__ gb) {
-  __shared__ __align__(16) u16 dT[C * WS_D];  // dT[co][p] = D[t0 + p][co]
-  __shared__ __align__(16) u16 xT[C * WS_X];  // xT[ci][p] = X[t0 - 4 + p][ci]
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int b = blockIdx.y, t0 = blockIdx.x * TT;
-  const long cb = (long)b * nT;
-  for (int i = tid; i < TT * C; i += 256) {
-    const int pp = i / C, ch = i % C, t = t0 + pp;
-    dT[ch * WS_D + pp] = t < nT ? Dg[(cb + t) * C + ch] : (u16)0;
-  }
-  for (int i = tid; i < (TT + 2 * HW) * C; i += 256) {
-    const int pp = i / C, ch = i % C, t = t0 - HW + pp;
-    xT[ch * WS_X + pp] = (t >= 0 && t < nT) ? X[(cb + t) * C + ch] : (u16)0;
-  }
-  __syncthreads();
-  const int g = lane >> 4, r = lane & 15;
-  // 9 taps x 2 co tiles x 2 ci tiles of 16 x 16
-  for (int u = wave; u < KW * 4; u += 4) {
-    const int k = u >> 2, mt = (u >> 1) & 1, nt = u & 1;
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                                                   int ncols, float4* __restrict__ part) {
+  __shared__ float4 red[WG_QUADS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int p = lane & 15, g = lane >> 4;
+  const int per = nT / 32;
+  const long groups = (long)ncols * per;
+  const long gw = (long)blockIdx.x * 4 + wave, nw = (long)gridDim.x * 4;
+  const long first = gw * groups / nw, end = (gw + 1) * groups / nw;
+  const uint32_t* D32 = reinterpret_cast<const uint32_t*>(Dg) + p;
+  const uint32_t* X32 = reinterpret_cast<const uint32_t*>(X) + p;
+  f32x4 acc[KW][2][2], accb[2];
 #pragma unroll
-    for (int kb = 0; kb < TT / 32; ++kb) {
-      const int tb = 32 * kb + 8 * g;
-      const bf16x8 av = *reinterpret_cast<const bf16x8*>(dT + (16 * mt + r) * WS_D + tb);
-      const u16* xr = xT + (16 * nt + r) * WS_X + tb + k;
-      bf16x8 bv;
+  for (int k = 0; k < KW; ++k)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) bv[j] = __builtin_bit_cast(__bf16, xr[j]);
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv, acc, 0, 0, 0);
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[k][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  accb[0] = accb[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint32_t one2 = 0x3f803f80u;
+  const bf16x8 ones = __builtin_bit_cast(bf16x8, make_uint4(one2, one2, one2, one2));
+  // groups two ahead are in flight under a group's 38 products (one wave per SIMD: the
+  // accumulators leave room for no second)
+  uint32_t d[2][8], x[2][16];
+  int col = (int)(first / per), tb0 = (int)(first % per) * 32;  // of the next group loaded
+  auto load = [&](int q) {
+    const int tb = tb0 + 8 * g;
+    const uint32_t* dr = D32 + ((long)col * nT + tb) * (C / 2);
+    const uint32_t* xr = X32 + (long)col * nT * (C / 2);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) d[q][j] = dr[j * (C / 2)];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) x[q][j] = xr[min(max(tb - HW + j, 0), nT - 1) * (C / 2)];
+    tb0 += 32;
+    if (tb0 == nT) { tb0 = 0; ++col; }
+  };
+  int tu = tb0;  // of the group used
+  auto use = [&](int q, bool more) {
+    uint32_t dp[2][4], xp[2][15];
+    const int tb = tu + 8 * g - HW;
+    tu = tu + 32 == nT ? 0 : tu + 32;
+#pragma unroll
+    for (int j = 0; j < 16; ++j)  // zero outside the column
+      if (tb + j < 0 || tb + j >= nT) x[q][j] = 0u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      dp[0][j] = __builtin_amdgcn_perm(d[q][2 * j + 1], d[q][2 * j], 0x05040100u);
+      dp[1][j] = __builtin_amdgcn_perm(d[q][2 * j + 1], d[q][2 * j], 0x07060302u);
     }
-    // D[co = 16 mt + 4 g + i][ci = 16 nt + r]
 #pragma unroll
-    for (int i = 0; i < 4; ++i) atomicAdd(&gW[((16 * mt + 4 * g + i) * C + 16 * nt + r) * KW + k], acc[i]);
+    for (int j = 0; j < 15; ++j) {
+      xp[0][j] = __builtin_amdgcn_perm(x[q][j + 1], x[q][j], 0x05040100u);
+      xp[1][j] = __builtin_amdgcn_perm(x[q][j + 1], x[q][j], 0x07060302u);
+    }
+    if (more) load(q);
+    __builtin_amdgcn_sched_barrier(0);
+    bf16x8 av[2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+      av[a] = __builtin_bit_cast(bf16x8, make_uint4(dp[a][0], dp[a][1], dp[a][2], dp[a][3]));
+      accb[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[a], ones, accb[a], 0, 0, 0);
+    }
+#pragma unroll
+    for (int k = 0; k < KW; ++k)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const bf16x8 bv = __builtin_bit_cast(bf16x8, make_uint4(xp[b][k], xp[b][k + 2], xp[b][k + 4], xp[b][k + 6]));
+#pragma unroll
+        for (int a = 0; a < 2; ++a) acc[k][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[a], bv, acc[k][a][b], 0, 0, 0);
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  if (first < end) load(0);
+  if (first + 1 < end) load(1);
+  for (long ch = first; ch < end; ch += 2) {
+    use(0, ch + 2 < end);
+    if (ch + 1 < end) use(1, ch + 3 < end);
   }
-  if (tid < C) {
-    float s = 0.f;
-    for (int pp = 0; pp < TT; ++pp) s += bf2f(dT[tid * WS_D + pp]);
-    atomicAdd(&gb[tid], s);
+  auto tile = [&](int i) -> f32x4& { return i < KW * 4 ? acc[i >> 2][(i >> 1) & 1][i & 1] : accb[i - KW * 4]; };
+  float4* out = part + (long)blockIdx.x * WG_QUADS;
+  for (int w = 0; w < 4; ++w) {
+    if (wave == w) {
+#pragma unroll
+      for (int i = 0; i < WG_TILES; ++i) {
+        const f32x4 t = tile(i);
+        float4 v = make_float4(t[0], t[1], t[2], t[3]);
+        if (w > 0) {
+          const float4 o = red[i * 64 + lane];
+          v = make_float4(v.x + o.x, v.y + o.y, v.z + o.z, v.w + o.w);
+        }
+        if (w < 3) red[i * 64 + lane] = v;
+        else out[i * 64 + lane] = v;
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Adds the partials of the layers' weight gradients (blocks[j] of layer j, laid out
+// part[j][block][tile][lane]) into the parameter gradients.  Tile element i of lane l
+// is D[co][ci] at co = 2 (4 (l / 16) + i) + a, ci = 2 (l % 16) + b.  One block takes
+// 32 float4 entries, eight threads each over the partials.
+__global__ __launch_bounds__(256) void k_net_wgrad_sum(const float4* __restrict__ part, int nblocks, long layer_stride,
+                                                       float* __restrict__ grads) {
+  __shared__ float4 red[8][32];
+  const int q = threadIdx.x & 31, r = threadIdx.x >> 5;
+  const int e = blockIdx.x * 32 + q, j = blockIdx.y;
+  const float4* src = part + j * layer_stride + e;
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+  for (int b = r; b < nblocks; b += 8) {
+    const float4 v = src[(long)b * WG_QUADS];
+    s = make_float4(s.x + v.x, s.y + v.y, s.z + v.z, s.w + v.w);
+  }
+  red[r][q] = s;
+  __syncthreads();
+  if (r != 0) return;
+#pragma unroll
+  for (int k = 1; k < 8; ++k) {
+    const float4 v = red[k][q];
+    s = make_float4(s.x + v.x, s.y + v.y, s.z + v.z, s.w + v.w);
+  }
+  const int t = e >> 6, lane = e & 63, n = lane & 15, g = lane >> 4;
+  float* gl = grads + (long)j * LAYER_SIZE;
+  const float v[4] = {s.x, s.y, s.z, s.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if (t < KW * 4) {
+      const int k = t >> 2, a = (t >> 1) & 1, b = t & 1;
+      gl[((2 * (4 * g + i) + a) * C + 2 * n + b) * KW + k] = v[i];
+    } else if (n == 0) {
+      gl[W_SIZE + 2 * (4 * g + i) + (t - KW * 4)] = v[i];
+    }
   }
 }
 

@@ -162,3 +162,40 @@ def test_learned_march_config1():
     print(f"  learned vs KT {errs}; linear (no nonlinear update) vs KT field {lin_err:.2e}")
     assert errs["field"] <= 1e-3
     assert errs["field"] < lin_err / 10
+
+
+@pytest.mark.parametrize("ncols,nT", [(1, 256), (3, 512), (65, 256), (127, 1024)])
+def test_weight_gradient_sums_match_float64(ncols, nT):
+    """The weight-gradient kernel over its shares of the samples: one 32-sample group
+    per wave or none, uneven shares, columns split between waves and blocks.
+
+    Every layer passes channel 0 through its centre tap, so the output layer's input is
+    relu(bf16(u / A)) and its gradients are plain sums of products of bf16 values, formed
+    here in float64.  The kernel adds n = 32 samples per product, at most 16 products and
+    256 partials in float32: relative to the sum of magnitudes below
+    6e-8 (32 + 16 + 256 / 8 + 8) = 5e-6."""
+    import torch
+    from angularspectrum_heterogeneous_amd import learned as L
+    p = np.zeros(L.PARAM_COUNT, np.float32)
+    for j in range(L.NLAY):
+        p[j * L.LAYER_SIZE:j * L.LAYER_SIZE + L.W_SIZE].reshape(L.C, L.C, L.KW)[0, 0, L.KW // 2] = 1.0
+    net = L.LearnedStep(nT, max_cols=ncols, params=p)
+    rng = np.random.default_rng(ncols)
+    t = np.arange(nT)[None, :]
+    u = (np.sin(2 * np.pi * t / 25 + rng.uniform(0, 6, (ncols, 1))) * 1e6).astype(np.float32)
+    un = (u + 50 * rng.standard_normal(u.shape)).astype(np.float32)
+    ud, und = torch.from_numpy(u).cuda(), torch.from_numpy(un).cuda()
+    c = 3.7e-9
+    _, grads = net.loss_grad(ud, und, c)
+    f32 = dict(dtype=torch.float32, device="cuda")
+    A = ud.abs().amax(1, keepdim=True)
+    x3 = torch.relu((ud / A).to(torch.bfloat16).float())
+    r = x3 - (und - ud) / (torch.tensor(c, **f32) * A * A)
+    dy = (2 * r * torch.tensor(1.0 / (ncols * nT), **f32)).to(torch.bfloat16).double()
+    pad = torch.nn.functional.pad(x3.double(), (L.KW // 2, L.KW // 2))
+    got = grads[3 * L.LAYER_SIZE:].double()
+    for k in range(L.KW):
+        prod = dy * pad[:, k:k + nT]
+        assert abs(got[k] - prod.sum()) <= 5e-6 * prod.abs().sum(), k
+    assert abs(got[L.W_SIZE] - dy.sum()) <= 5e-6 * dy.abs().sum()
+    assert not got[L.C * L.KW:L.W_SIZE].any()  # output channels held at zero
