@@ -161,6 +161,7 @@ struct ash_plan {
   bool loaded = false;
   int host_row = -1;
   bool gen_x = false, gen_y = false, gen_t = false;  // axis runs the general-size kernels
+  DftMat dmx{}, dmy{}, dmt{};                        // and its DFT matrix
   int sa_band = 0;      // last row index (from each edge) with a nonzero super-absorbing y weight
   int precise_ops = 0;  // evaluate the k-space operators in FP64 (set from ASH_PRECISE_OPS)
   // graph of a plain step
@@ -388,9 +389,9 @@ int build_tables(ash_plan* p) {
     dft_matrix_fill(*m, tw, (float4*)a, nullptr);
     return ASH_OK;
   };
-  if (p->gen_x && (rc = matrix(nX, false, p->T.twx, &p->T.dmx))) return rc;
-  if (p->gen_y && (rc = matrix(nY, false, p->T.twy, &p->T.dmy))) return rc;
-  if (p->gen_t && (rc = matrix(nT, true, p->T.twgt, &p->T.dmt))) return rc;
+  if (p->gen_x && (rc = matrix(nX, false, p->T.twx, &p->dmx))) return rc;
+  if (p->gen_y && (rc = matrix(nY, false, p->T.twy, &p->dmy))) return rc;
+  if (p->gen_t && (rc = matrix(nT, true, p->T.twgt, &p->dmt))) return rc;
   if (!p->gen_t) {
     // pass-major twiddles of the column transform, [r * Ns + k] = W_{Ns R}^{k r}
     auto radices = [&](bool inv) {
@@ -523,8 +524,7 @@ void launch_col_MN(ash_plan* p, const ColDesc& cd, hipStream_t s) {
   // persistent: each wave walks several columns.  The final pass runs one
   // resident round of blocks (measured fastest for it: 74 against 83 us at
   // 256x256x1024 with 4096 blocks); the other passes take the tuned grid.
-  const bool fin = MODE == COL_FINAL || MODE == COL_FINAL_SRC;
-  blocks = std::min(blocks, fin ? p->fin_grid : p->col_grid);
+  blocks = std::min(blocks, MODE == COL_FINAL ? p->fin_grid : p->col_grid);
   hipLaunchKernelGGL((k_column<M, MODE, NLK>), dim3(blocks), dim3(256), 0, s, p->spec, p->T, p->g, cd);
 }
 template <int M, int MODE>
@@ -543,10 +543,8 @@ void launch_col_M(ash_plan* p, const ColDesc& cd, hipStream_t s) {
     case COL_LOAD: launch_col_MN<M, COL_LOAD, NL_NONE>(p, cd, s); break;
     case COL_NL: launch_col_MM<M, COL_NL>(p, cd, s); break;
     case COL_TAPER: launch_col_MN<M, COL_TAPER, NL_NONE>(p, cd, s); break;
-    case COL_FINAL:
-      if (cd.n_src > 0 || cd.smask) launch_col_MN<M, COL_FINAL_SRC, NL_NONE>(p, cd, s);
-      else launch_col_MN<M, COL_FINAL, NL_NONE>(p, cd, s);
-      break;
+    case COL_FINAL: launch_col_MN<M, COL_FINAL, NL_NONE>(p, cd, s); break;
+    case COL_INJECT: launch_col_MN<M, COL_INJECT, NL_NONE>(p, cd, s); break;
     case COL_STORE: launch_col_MN<M, COL_STORE, NL_NONE>(p, cd, s); break;
     case COL_RAWNL: launch_col_MM<M, COL_RAWNL>(p, cd, s); break;
     case COL_TOREAL: launch_col_MN<M, COL_TOREAL, NL_NONE>(p, cd, s); break;
@@ -569,7 +567,7 @@ void launch_col_M(ash_plan* p, const ColDesc& cd, hipStream_t s) {
 void xfwd(ash_plan* p, hipStream_t s) {
   ProfScope ps(p, ASH_K_XFWD, s);
   if (p->gen_x) {
-    gen_xfwd(p->spec, p->T, p->g, s);
+    gen_xfwd(p->spec, p->g, p->dmx, s);
     return;
   }
   DISPATCH_L(p->g.nX, launch_xfwd_L<L>(p, s));
@@ -577,7 +575,7 @@ void xfwd(ash_plan* p, hipStream_t s) {
 void ypass(ash_plan* p, const OpDesc& op, hipStream_t s) {
   ProfScope ps(p, ASH_K_YPASS, s);
   if (p->gen_y) {
-    gen_ypass(p->spec, p->T, p->g, op, s);
+    gen_ypass(p->spec, p->T, p->g, p->dmy, op, s);
     return;
   }
   DISPATCH_L(p->g.nY, launch_ypass_L<L>(p, op, s));
@@ -585,7 +583,7 @@ void ypass(ash_plan* p, const OpDesc& op, hipStream_t s) {
 void xinv(ash_plan* p, int epi, const EpiDesc& e, hipStream_t s) {
   ProfScope ps(p, ASH_K_XINV, s);
   if (p->gen_x) {
-    gen_xinv(epi, p->spec, p->T, p->g, e, s);
+    gen_xinv(epi, p->spec, p->T, p->g, p->dmx, e, s);
     return;
   }
   if (epi == 0) { DISPATCH_L(p->g.nX, (launch_xinv_L<L, 0>(p, e, s))); }
@@ -601,7 +599,7 @@ void launch_ypower_L(ash_plan* p, hipStream_t s) {
 void ypower(ash_plan* p, hipStream_t s) {
   ProfScope ps(p, ASH_K_YPASS, s);
   if (p->gen_y) {
-    gen_ypower(p->spec, p->T, p->g, p->obl_acc, s);
+    gen_ypower(p->spec, p->T, p->g, p->dmy, p->obl_acc, s);
     return;
   }
   DISPATCH_L(p->g.nY, launch_ypower_L<L>(p, s));
@@ -640,7 +638,7 @@ void column(ash_plan* p, const ColDesc& cd, hipStream_t s) {
                  : cd.mode == COL_FINAL ? ASH_K_COL_FINAL : ASH_K_COL_OTHER;
   ProfScope ps(p, kind, s);
   if (p->gen_t) {
-    gen_column(p->spec, p->T, p->g, cd, s);
+    gen_column(p->spec, p->T, p->g, p->dmt, cd, s);
     return;
   }
   switch (p->g.M) {
@@ -843,6 +841,21 @@ void enqueue_step(ash_plan* p, const ash_step_io* io, hipStream_t s) {
       ysa(p, s2, s);
     }
   }
+  // Source slices: their spectra are added to the columns that carry one, then every
+  // column takes the read-only final pass.  (One pass that did both held the tone
+  // burst's FP64 arithmetic for all columns and rewrote all of them: 742 us at
+  // 384x384x1024 with a bowl slice.)
+  if (io->n_src_dense > 0 || io->src_mask_dev) {
+    ColDesc ci = col_base(p);
+    ci.mode = COL_INJECT;
+    ci.n_src = io->n_src_dense;
+    for (int k = 0; k < io->n_src_dense && k < 4; ++k) ci.src[k] = io->src_dense_dev[k];
+    ci.smask = io->src_mask_dev;
+    ci.sdelay = io->src_delay_dev;
+    ci.taxis = io->taxis_dev;
+    ci.s_f0 = io->src_f0; ci.s_p0 = io->src_p0; ci.s_ncyc = io->src_ncycles; ci.s_dur = io->src_dur;
+    column(p, ci, s);
+  }
   ColDesc cd = col_base(p);
   cd.mode = COL_FINAL;
   cd.row = p->d_row;
@@ -851,12 +864,6 @@ void enqueue_step(ash_plan* p, const ash_step_io* io, hipStream_t s) {
   cd.stats = io->stats_dev;
   cd.ibefore = p->ibefore;
   cd.rout = io->field_out_dev;
-  cd.n_src = io->n_src_dense;
-  for (int k = 0; k < io->n_src_dense && k < 4; ++k) cd.src[k] = io->src_dense_dev[k];
-  cd.smask = io->src_mask_dev;
-  cd.sdelay = io->src_delay_dev;
-  cd.taxis = io->taxis_dev;
-  cd.s_f0 = io->src_f0; cd.s_p0 = io->src_p0; cd.s_ncyc = io->src_ncycles; cd.s_dur = io->src_dur;
   column(p, cd, s);
   if (p->tof_mode != 0 && io->tof_dev) {
     // time of flight of the field after the step (ASS:1538-1545), read only

@@ -241,7 +241,7 @@ template <int S, int LPC, bool STRIDED, bool BOUNDED, int MODE, int NLK>
 __device__ __forceinline__ void column_realspace(float (&u)[S], const LaneCol<S, LPC, STRIDED, BOUNDED>& L,
                                                  const ColDesc& d, const Tables& T, int c, bool live, int ncols,
                                                  int row, double Nn, int nsub_global, float& wmax) {
-  constexpr bool FIN = (MODE == COL_FINAL || MODE == COL_FINAL_SRC);
+  constexpr bool FIN = MODE == COL_FINAL;
   const float* tt = d.taper == 1 ? T.tapt_h : T.tapt_f;
   if constexpr (MODE == COL_NL || MODE == COL_TAPER || MODE == COL_RAWNL) {
     if (d.taper) {
@@ -362,30 +362,6 @@ __device__ __forceinline__ void column_realspace(float (&u)[S], const LaneCol<S,
     }
     if (MODE == COL_RAWNL && live) L.store(d.rout + (long)c * L.nT, u);
   } else if constexpr (FIN) {
-    if constexpr (MODE == COL_FINAL_SRC) {
-      // loads without a test each (clamped into the column, padding masked after),
-      // so they issue back to back
-      if (live) {
-        for (int k = 0; k < d.n_src; ++k) {
-          const float* sp = d.src[k] + (long)c * L.nT;
-          float sv[S];
-#pragma unroll
-          for (int i = 0; i < S; ++i) sv[i] = sp[min(L.t(i), L.nT - 1)];
-#pragma unroll
-          for (int i = 0; i < S; ++i) u[i] += L.in(i) ? sv[i] : 0.f;
-        }
-      }
-      if (d.smask && live && d.smask[c]) {
-        const double dl = d.sdelay[c];
-        const double w0 = 2.0 * 3.14159265358979323846 * d.s_f0;
-        const double cexp = 2.0 * d.s_dur;
-        float tv[S];
-#pragma unroll
-        for (int i = 0; i < S; ++i) tv[i] = d.taxis[min(L.t(i), L.nT - 1)];
-#pragma unroll
-        for (int i = 0; i < S; ++i) u[i] += L.in(i) ? tone_burst(tv[i] - dl, w0, d.s_ncyc, cexp, d.s_p0) : 0.f;
-      }
-    }
     // (padding samples of a bounded lane are zero: they add nothing to e2 but are
     // kept out of the extrema)
     float mn = BOUNDED ? INFINITY : u[0], mx = BOUNDED ? -INFINITY : u[0];
@@ -444,6 +420,21 @@ __device__ __forceinline__ void column_realspace(float (&u)[S], const LaneCol<S,
 #pragma unroll
     for (int i = 0; i < S; ++i) wmax = fmaxf(wmax, live ? fabsf(u[i]) : 0.f);
   }
+}
+
+// Source slices of a step: whether column c has one, and its sample t (dense slices,
+// then the sparse tone burst, each a float32 as the reference stores them).
+__device__ __forceinline__ bool column_has_source(const ColDesc& d, int c) {
+  return d.n_src > 0 || (d.smask && d.smask[c] != 0);
+}
+__device__ __forceinline__ float source_sample(const ColDesc& d, int c, int nT, int t) {
+  float u = 0.f;
+  for (int k = 0; k < d.n_src; ++k) u += d.src[k][(long)c * nT + t];
+  if (d.smask && d.smask[c]) {
+    const double w0 = 2.0 * 3.14159265358979323846 * d.s_f0;
+    u += tone_burst(d.taxis[t] - d.sdelay[c], w0, d.s_ncyc, 2.0 * d.s_dur, d.s_p0);
+  }
+  return u;
 }
 
 // True on every lane of the column when any of its rfft bins 0..M is nonzero.
@@ -544,8 +535,8 @@ __global__ __launch_bounds__(256) void k_column(float2* __restrict__ spec, Table
   const int tid = threadIdx.x;
   const int wave = tid / 64, lane = tid % 64;
   const int cw = lane / LPC, ln = lane % LPC;
-  constexpr bool spectral_in = !(MODE == COL_LOAD || MODE == COL_RAWNL);
-  constexpr bool rewrite = (MODE == COL_NL || MODE == COL_TAPER || MODE == COL_LOAD || MODE == COL_FINAL_SRC);
+  constexpr bool spectral_in = !(MODE == COL_LOAD || MODE == COL_RAWNL || MODE == COL_INJECT);
+  constexpr bool rewrite = (MODE == COL_NL || MODE == COL_TAPER || MODE == COL_LOAD || MODE == COL_INJECT);
   if constexpr (spectral_in || rewrite) {
     // (COL_RAWNL runs no transform and may be launched without tables)
     for (int i = tid; i < TWT; i += 256) s_tw[i] = T.twc[i];
@@ -575,7 +566,7 @@ __global__ __launch_bounds__(256) void k_column(float2* __restrict__ spec, Table
   // contiguous samples
   constexpr bool STRIDED = !(MODE == COL_NL || MODE == COL_RAWNL);
   const LaneCol<S, LPC, STRIDED, false> lc{ln, lane, t0, NT_};
-  constexpr bool FIN = (MODE == COL_FINAL || MODE == COL_FINAL_SRC);
+  constexpr bool FIN = MODE == COL_FINAL;
   const int row = (FIN || MODE == COL_TOF) ? *d.row : 0;
   // Burgers coefficient, scaled by the beam obliquity when requested (ASS:934)
   const double Nn = d.nscale ? d.N * (d.nscale[0] / (d.nscale[1] + 1e-30)) : d.N;
@@ -653,7 +644,11 @@ __global__ __launch_bounds__(256) void k_column(float2* __restrict__ spec, Table
   };
   for (int cbase = blockIdx.x * per_iter; cbase < ncols; cbase += gridDim.x * per_iter) {
     const int c = cbase + wave * CPW + cw;
-    const bool live = c < ncols && (!d.cflag || d.cflag[c] != 0);
+    bool live = c < ncols && (!d.cflag || d.cflag[c] != 0);
+    if constexpr (MODE == COL_INJECT) {
+      live = c < ncols && column_has_source(d, c);
+      if (__ballot(live) == 0) continue;
+    }
     if (CPW == 1 && !live) continue;  // one column per wave: skip it whole
     float2* sc = spec + (long)c * g.MP;
     sc_cur = live ? sc : nullptr;
@@ -661,7 +656,23 @@ __global__ __launch_bounds__(256) void k_column(float2* __restrict__ spec, Table
     float uq[MODE == COL_TOF ? S : 1];
 
     // ---------------- stage 1: real samples t0 .. t0+S-1 of the column ----------------
-    if constexpr (!spectral_in && STRIDED) {
+    if constexpr (MODE == COL_INJECT) {
+      // one copy of the tone burst's code in a loop; the samples pass through LDS
+#pragma unroll 1
+      for (int k = ln; k < M; k += LPC) {
+        float2 x = make_float2(0.f, 0.f);
+        if (live) x = make_float2(source_sample(d, c, NT_, 2 * k), source_sample(d, c, NT_, 2 * k + 1));
+        cb[pidx(k)] = x;
+      }
+      wave_sync();
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const float2 x = cb[pidx(ln + LPC * e)];
+        u[2 * e] = x.x;
+        u[2 * e + 1] = x.y;
+      }
+      wave_sync();
+    } else if constexpr (!spectral_in && STRIDED) {
       const float2* src = reinterpret_cast<const float2*>(d.rin + (long)c * NT_);
 #pragma unroll
       for (int e = 0; e < E; ++e) {
@@ -688,7 +699,9 @@ __global__ __launch_bounds__(256) void k_column(float2* __restrict__ spec, Table
     }
 
     // ---------------- stage 2: real-space work ----------------
-    if constexpr (MODE == COL_TOF) {
+    if constexpr (MODE == COL_INJECT) {
+      // the transform is linear: the source's spectrum is added below
+    } else if constexpr (MODE == COL_TOF) {
       const bool nz = spectrum_nonzero<LPC>(sc, live ? M : -1, ln);
       column_tof<S, LPC, STRIDED, false>(u, uq, lc, reinterpret_cast<float*>(cb), d, c, live, ncols, row, nz);
     } else {
@@ -709,6 +722,13 @@ __global__ __launch_bounds__(256) void k_column(float2* __restrict__ spec, Table
         for (int e = 0; e < E; ++e) v[e] = cb[pidx(ln + LPC * e)];
         wave_sync();
       }
+      // (COL_INJECT: the bins that the source's are added to)
+      float2 old[MODE == COL_INJECT ? E : 1], oldM = make_float2(0.f, 0.f);
+      if constexpr (MODE == COL_INJECT) {
+#pragma unroll
+        for (int e = 0; e < E; ++e) old[e] = live ? sc[ln + LPC * e] : make_float2(0.f, 0.f);
+        if (live) oldM = sc[M];
+      }
       cfft<M, false>(v, cb, twf, ln);
 #pragma unroll
       for (int e = 0; e < E; ++e) cb[pidx(ln + LPC * e)] = v[e];
@@ -723,9 +743,11 @@ __global__ __launch_bounds__(256) void k_column(float2* __restrict__ spec, Table
         // halves folded into the table and the fmas
         const float2 df = csub(zk, zm);
         const float2 t = cmul(twn(e), df);
-        if (live) sc[k] = make_float2(fmaf(0.5f, zk.x, fmaf(0.5f, zm.x, t.y)), fmaf(0.5f, zk.y, fmaf(0.5f, zm.y, -t.x)));
+        float2 x = make_float2(fmaf(0.5f, zk.x, fmaf(0.5f, zm.x, t.y)), fmaf(0.5f, zk.y, fmaf(0.5f, zm.y, -t.x)));
+        if constexpr (MODE == COL_INJECT) x = cadd(old[e], x);
+        if (live) sc[k] = x;
       }
-      if (ln == 0 && live) sc[M] = make_float2(z0.x - z0.y, 0.f);
+      if (ln == 0 && live) sc[M] = make_float2(oldM.x + (z0.x - z0.y), oldM.y);
       wave_sync();
     }
   }

@@ -242,9 +242,8 @@ __device__ __forceinline__ void hm_fold(float4* eo, const DftMat& d, int tid, in
 // x-sweep, forward DFT along x.  Tile = (y, 16 f bins).  Padding lines past the last
 // bin are zero and stay zero, so no load or store is guarded.
 template <bool EVEN, int T_>
-__global__ __launch_bounds__(512) void k_gx_fwd(float2* __restrict__ spec, Tables T, Geom g) {
+__global__ __launch_bounds__(512) void k_gx_fwd(float2* __restrict__ spec, Geom g, DftMat d) {
   extern __shared__ float4 eo[];
-  const DftMat d = T.dmx;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
   const int y = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
   const uint32_t sxb = (uint32_t)g.nY * g.MP * 8u;
@@ -262,9 +261,8 @@ __global__ __launch_bounds__(512) void k_gx_fwd(float2* __restrict__ spec, Table
 
 // x-sweep, inverse DFT along x + the epilogues 0 and 1 of k_xfft_inv.
 template <bool EVEN, int T_, int EPI>
-__global__ __launch_bounds__(512) void k_gx_inv(float2* __restrict__ spec, Tables T, Geom g, EpiDesc ep) {
+__global__ __launch_bounds__(512) void k_gx_inv(float2* __restrict__ spec, Tables T, Geom g, DftMat d, EpiDesc ep) {
   extern __shared__ float4 eo[];
-  const DftMat d = T.dmx;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
   const int y = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
   const uint32_t sxb = (uint32_t)g.nY * g.MP * 8u;
@@ -295,9 +293,8 @@ __global__ __launch_bounds__(512) void k_gx_inv(float2* __restrict__ spec, Table
 // which pass through the tile's LDS (n * 16 float2 fit the folded tile) once every
 // wave holds its T row tiles in registers.
 template <bool EVEN, int T_>
-__global__ __launch_bounds__(512) void k_gx_inv_sa(float2* __restrict__ spec, Tables T, Geom g, EpiDesc ep) {
+__global__ __launch_bounds__(512) void k_gx_inv_sa(float2* __restrict__ spec, Tables T, Geom g, DftMat d, EpiDesc ep) {
   extern __shared__ float4 eo[];
-  const DftMat d = T.dmx;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
   const int y = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
   const uint32_t sxb = (uint32_t)g.nY * g.MP * 8u;
@@ -368,9 +365,8 @@ __device__ __forceinline__ LineConst line_const(const Tables& T, const OpDesc& o
 // evaluated at every position's own wavenumber (the grids are mirror images only up
 // to rounding, and one ulp decides a mode at the evanescent cutoff).
 template <bool EVEN, int T_, bool PRECISE>
-__global__ __launch_bounds__(512) void k_gy_pass(float2* __restrict__ spec, Tables T, Geom g, OpDesc op) {
+__global__ __launch_bounds__(512) void k_gy_pass(float2* __restrict__ spec, Tables T, Geom g, DftMat d, OpDesc op) {
   extern __shared__ float4 eo[];
-  const DftMat d = T.dmy;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
   const int x = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
   const uint32_t syb = (uint32_t)g.MP * 8u;
@@ -431,11 +427,10 @@ __global__ __launch_bounds__(512) void k_gy_pass(float2* __restrict__ spec, Tabl
 // Power-weighted obliquity sums of a (kx row, f block) tile (as k_ypower): forward
 // DFT along y, then acc[0] += sum P k/k_z, acc[1] += sum P over propagating modes.
 template <bool EVEN, int T_>
-__global__ __launch_bounds__(512) void k_gy_power(const float2* __restrict__ spec, Tables T, Geom g,
+__global__ __launch_bounds__(512) void k_gy_power(const float2* __restrict__ spec, Tables T, Geom g, DftMat d,
                                                   double* __restrict__ acc) {
   extern __shared__ float4 eo[];
   __shared__ double sred[2][8];
-  const DftMat d = T.dmy;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
   const int x = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
   const uint32_t syb = (uint32_t)g.MP * 8u;
@@ -618,13 +613,12 @@ __device__ __forceinline__ void hm_col_emit(const DftMat& d, const ColAcc<EVEN>&
 }
 
 template <int S, bool EVEN, int MODE, int NLK>
-__global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restrict__ spec, Tables T, Geom g, ColDesc d) {
+__global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restrict__ spec, Tables T, Geom g, DftMat dm, ColDesc d) {
   constexpr int W = gcol_waves(S), TW = gcol_tiles(S, EVEN), NC = GC_COLS / W;
   extern __shared__ float4 glds[];
   __shared__ float s_red[W];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int nT = g.nT, M = g.M, ncols = g.nX * g.nY;
-  const DftMat dm = T.dmt;
   const Tiles tiles = hm_tiles(dm, wave, W);
   const int pitch = gcol_pitch(nT, S);
   float* rows = reinterpret_cast<float*>(glds);
@@ -632,9 +626,9 @@ __global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restri
   const int c0 = blockIdx.x * GC_COLS;
   const int t0 = lane * S;
   const float invN = 1.f / (float)nT;
-  constexpr bool spectral_in = MODE != COL_LOAD;
-  constexpr bool rewrite = (MODE == COL_NL || MODE == COL_TAPER || MODE == COL_LOAD || MODE == COL_FINAL_SRC);
-  constexpr bool FIN = (MODE == COL_FINAL || MODE == COL_FINAL_SRC);
+  constexpr bool spectral_in = MODE != COL_LOAD && MODE != COL_INJECT;
+  constexpr bool rewrite = (MODE == COL_NL || MODE == COL_TAPER || MODE == COL_LOAD || MODE == COL_INJECT);
+  constexpr bool FIN = MODE == COL_FINAL;
   constexpr bool tapered = (MODE == COL_NL || MODE == COL_TAPER || MODE == COL_MAXABS);
   const float* tt = tapered && d.taper ? (d.taper == 1 ? T.tapt_h : T.tapt_f) : nullptr;
   const LaneCol<S, 64, false, true> lc{lane, lane, t0, nT};
@@ -719,6 +713,11 @@ __global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restri
     return;
   } else {
     if constexpr (spectral_in) inverse(0);
+    if constexpr (MODE == COL_INJECT) {
+      bool any = false;
+      for (int c = c0; c < min(c0 + GC_COLS, ncols); ++c) any = any || column_has_source(d, c);
+      if (!any) return;
+    }
 #pragma unroll 1
     for (int i = 0; i < NC; ++i) {
       const int col = wave * NC + i, c = c0 + col;
@@ -739,6 +738,11 @@ __global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restri
         for (int o = 32; o > 0; o >>= 1) e2 += __shfl_xor(e2, o, 64);
         if (lane == 0 && d.ibefore) d.ibefore[c] = e2;
         wmax = fmaxf(wmax, mx);
+        wave_sync();
+      } else if constexpr (MODE == COL_INJECT) {
+        const bool src = column_has_source(d, c);
+#pragma unroll 1
+        for (int t = lane; t < nT; t += 64) uc[skew(t)] = src ? source_sample(d, c, nT, t) : 0.f;
         wave_sync();
       } else if constexpr (MODE == COL_STORE) {
         float* dst = d.rout + (long)c * nT;
@@ -805,7 +809,8 @@ __global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restri
         if (c < ncols) {
           float2* sc = spec + (long)c * g.MP;
           const float2* X = reinterpret_cast<const float2*>(rows + col * pitch);
-          for (int m = lane; m <= M; m += 64) sc[m] = X[m];
+          if (MODE == COL_INJECT && !column_has_source(d, c)) continue;
+          for (int m = lane; m <= M; m += 64) sc[m] = MODE == COL_INJECT ? cadd(sc[m], X[m]) : X[m];
         }
       }
     }

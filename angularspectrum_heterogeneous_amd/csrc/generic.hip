@@ -53,31 +53,31 @@ size_t line_lds(const DftMat& d) { return (size_t)d.Kp * 16 * sizeof(float4); }
 
 }  // namespace
 
-void gen_xfwd(float2* spec, const Tables& T, const Geom& g, hipStream_t s) {
-  const dim3 grid(g.nY * g.nfb), block(64 * line_waves(T.dmx));
-  const size_t lds = line_lds(T.dmx);
-  DISPATCH_TILES(T.dmx, hipLaunchKernelGGL((k_gx_fwd<EVEN, T_>), grid, block, lds, s, spec, T, g));
+void gen_xfwd(float2* spec, const Geom& g, const DftMat& d, hipStream_t s) {
+  const dim3 grid(g.nY * g.nfb), block(64 * line_waves(d));
+  const size_t lds = line_lds(d);
+  DISPATCH_TILES(d, hipLaunchKernelGGL((k_gx_fwd<EVEN, T_>), grid, block, lds, s, spec, g, d));
 }
 
-void gen_xinv(int epi, float2* spec, const Tables& T, const Geom& g, const EpiDesc& e, hipStream_t s) {
-  const dim3 grid(g.nY * g.nfb), block(64 * line_waves(T.dmx));
-  const size_t lds = line_lds(T.dmx);
-  if (epi == 2) DISPATCH_TILES(T.dmx, hipLaunchKernelGGL((k_gx_inv_sa<EVEN, T_>), grid, block, lds, s, spec, T, g, e));
-  else if (epi == 1) DISPATCH_TILES(T.dmx, hipLaunchKernelGGL((k_gx_inv<EVEN, T_, 1>), grid, block, lds, s, spec, T, g, e));
-  else DISPATCH_TILES(T.dmx, hipLaunchKernelGGL((k_gx_inv<EVEN, T_, 0>), grid, block, lds, s, spec, T, g, e));
+void gen_xinv(int epi, float2* spec, const Tables& T, const Geom& g, const DftMat& d, const EpiDesc& e, hipStream_t s) {
+  const dim3 grid(g.nY * g.nfb), block(64 * line_waves(d));
+  const size_t lds = line_lds(d);
+  if (epi == 2) DISPATCH_TILES(d, hipLaunchKernelGGL((k_gx_inv_sa<EVEN, T_>), grid, block, lds, s, spec, T, g, d, e));
+  else if (epi == 1) DISPATCH_TILES(d, hipLaunchKernelGGL((k_gx_inv<EVEN, T_, 1>), grid, block, lds, s, spec, T, g, d, e));
+  else DISPATCH_TILES(d, hipLaunchKernelGGL((k_gx_inv<EVEN, T_, 0>), grid, block, lds, s, spec, T, g, d, e));
 }
 
-void gen_ypass(float2* spec, const Tables& T, const Geom& g, const OpDesc& op, hipStream_t s) {
-  const dim3 grid(g.nX * g.nfb), block(64 * line_waves(T.dmy));
-  const size_t lds = line_lds(T.dmy);
-  if (op.precise) DISPATCH_TILES(T.dmy, hipLaunchKernelGGL((k_gy_pass<EVEN, T_, true>), grid, block, lds, s, spec, T, g, op));
-  else DISPATCH_TILES(T.dmy, hipLaunchKernelGGL((k_gy_pass<EVEN, T_, false>), grid, block, lds, s, spec, T, g, op));
+void gen_ypass(float2* spec, const Tables& T, const Geom& g, const DftMat& d, const OpDesc& op, hipStream_t s) {
+  const dim3 grid(g.nX * g.nfb), block(64 * line_waves(d));
+  const size_t lds = line_lds(d);
+  if (op.precise) DISPATCH_TILES(d, hipLaunchKernelGGL((k_gy_pass<EVEN, T_, true>), grid, block, lds, s, spec, T, g, d, op));
+  else DISPATCH_TILES(d, hipLaunchKernelGGL((k_gy_pass<EVEN, T_, false>), grid, block, lds, s, spec, T, g, d, op));
 }
 
-void gen_ypower(const float2* spec, const Tables& T, const Geom& g, double* acc, hipStream_t s) {
-  const dim3 grid(g.nX * g.nfb), block(64 * line_waves(T.dmy));
-  const size_t lds = line_lds(T.dmy);
-  DISPATCH_TILES(T.dmy, hipLaunchKernelGGL((k_gy_power<EVEN, T_>), grid, block, lds, s, spec, T, g, acc));
+void gen_ypower(const float2* spec, const Tables& T, const Geom& g, const DftMat& d, double* acc, hipStream_t s) {
+  const dim3 grid(g.nX * g.nfb), block(64 * line_waves(d));
+  const size_t lds = line_lds(d);
+  DISPATCH_TILES(d, hipLaunchKernelGGL((k_gy_power<EVEN, T_>), grid, block, lds, s, spec, T, g, d, acc));
 }
 
 void gen_ysa(float2* spec, const Tables& T, const Geom& g, const ScreenDesc& sd, hipStream_t s) {
@@ -90,11 +90,11 @@ int gen_column_blocks(int ncols) { return (ncols + GC_COLS - 1) / GC_COLS; }
 namespace {
 
 template <int S, int MODE, int NLK>
-void launch_gcol_SMN(float2* spec, const Tables& T, const Geom& g, const ColDesc& cd, hipStream_t s) {
+void launch_gcol_SMN(float2* spec, const Tables& T, const Geom& g, const DftMat& d, const ColDesc& cd, hipStream_t s) {
   const dim3 grid(gen_column_blocks(g.nX * g.nY)), block(64 * gcol_waves(S));
   const size_t lds = (size_t)GC_COLS * gcol_pitch(g.nT, S) * sizeof(float);
-  if (T.dmt.even) hipLaunchKernelGGL((k_gcolumn<S, true, MODE, NLK>), grid, block, lds, s, spec, T, g, cd);
-  else hipLaunchKernelGGL((k_gcolumn<S, false, MODE, NLK>), grid, block, lds, s, spec, T, g, cd);
+  if (d.even) hipLaunchKernelGGL((k_gcolumn<S, true, MODE, NLK>), grid, block, lds, s, spec, T, g, d, cd);
+  else hipLaunchKernelGGL((k_gcolumn<S, false, MODE, NLK>), grid, block, lds, s, spec, T, g, d, cd);
 }
 template <int S, int NLK>
 void launch_graw(const Tables& T, const Geom& g, const ColDesc& cd, hipStream_t s) {
@@ -102,20 +102,18 @@ void launch_graw(const Tables& T, const Geom& g, const ColDesc& cd, hipStream_t 
   hipLaunchKernelGGL((k_gcolumn_raw<S, NLK>), dim3(blocks), dim3(64 * GR_WPB), 0, s, T, g, cd);
 }
 template <int S>
-void launch_gcol_S(float2* spec, const Tables& T, const Geom& g, const ColDesc& cd, hipStream_t s) {
+void launch_gcol_S(float2* spec, const Tables& T, const Geom& g, const DftMat& d, const ColDesc& cd, hipStream_t s) {
   switch (cd.mode) {
-    case COL_LOAD: launch_gcol_SMN<S, COL_LOAD, NL_NONE>(spec, T, g, cd, s); break;
+    case COL_LOAD: launch_gcol_SMN<S, COL_LOAD, NL_NONE>(spec, T, g, d, cd, s); break;
     case COL_NL:  // (the march's updates; KT_MINMOD is an operator of its own)
-      if (cd.nl == NL_KT) launch_gcol_SMN<S, COL_NL, NL_KT>(spec, T, g, cd, s);
-      else if (cd.nl == NL_TVD) launch_gcol_SMN<S, COL_NL, NL_TVD>(spec, T, g, cd, s);
-      else launch_gcol_SMN<S, COL_NL, NL_RUSANOV>(spec, T, g, cd, s);
+      if (cd.nl == NL_KT) launch_gcol_SMN<S, COL_NL, NL_KT>(spec, T, g, d, cd, s);
+      else if (cd.nl == NL_TVD) launch_gcol_SMN<S, COL_NL, NL_TVD>(spec, T, g, d, cd, s);
+      else launch_gcol_SMN<S, COL_NL, NL_RUSANOV>(spec, T, g, d, cd, s);
       break;
-    case COL_TAPER: launch_gcol_SMN<S, COL_TAPER, NL_NONE>(spec, T, g, cd, s); break;
-    case COL_FINAL:
-      if (cd.n_src > 0 || cd.smask) launch_gcol_SMN<S, COL_FINAL_SRC, NL_NONE>(spec, T, g, cd, s);
-      else launch_gcol_SMN<S, COL_FINAL, NL_NONE>(spec, T, g, cd, s);
-      break;
-    case COL_STORE: launch_gcol_SMN<S, COL_STORE, NL_NONE>(spec, T, g, cd, s); break;
+    case COL_TAPER: launch_gcol_SMN<S, COL_TAPER, NL_NONE>(spec, T, g, d, cd, s); break;
+    case COL_FINAL: launch_gcol_SMN<S, COL_FINAL, NL_NONE>(spec, T, g, d, cd, s); break;
+    case COL_INJECT: launch_gcol_SMN<S, COL_INJECT, NL_NONE>(spec, T, g, d, cd, s); break;
+    case COL_STORE: launch_gcol_SMN<S, COL_STORE, NL_NONE>(spec, T, g, d, cd, s); break;
     case COL_RAWNL:
       switch (cd.nl) {
         case NL_KT: launch_graw<S, NL_KT>(T, g, cd, s); break;
@@ -125,21 +123,21 @@ void launch_gcol_S(float2* spec, const Tables& T, const Geom& g, const ColDesc& 
         default: launch_graw<S, NL_NONE>(T, g, cd, s); break;
       }
       break;
-    case COL_MAXABS: launch_gcol_SMN<S, COL_MAXABS, NL_NONE>(spec, T, g, cd, s); break;
-    case COL_TOF: launch_gcol_SMN<S, COL_TOF, NL_NONE>(spec, T, g, cd, s); break;
+    case COL_MAXABS: launch_gcol_SMN<S, COL_MAXABS, NL_NONE>(spec, T, g, d, cd, s); break;
+    case COL_TOF: launch_gcol_SMN<S, COL_TOF, NL_NONE>(spec, T, g, d, cd, s); break;
     default: break;
   }
 }
 
 }  // namespace
 
-void gen_column(float2* spec, const Tables& T, const Geom& g, const ColDesc& cd, hipStream_t s) {
+void gen_column(float2* spec, const Tables& T, const Geom& g, const DftMat& d, const ColDesc& cd, hipStream_t s) {
   // S real samples per lane, 64 S >= nT
-  if (g.nT <= 128) launch_gcol_S<2>(spec, T, g, cd, s);
-  else if (g.nT <= 256) launch_gcol_S<4>(spec, T, g, cd, s);
-  else if (g.nT <= 512) launch_gcol_S<8>(spec, T, g, cd, s);
-  else if (g.nT <= 1024) launch_gcol_S<16>(spec, T, g, cd, s);
-  else launch_gcol_S<32>(spec, T, g, cd, s);
+  if (g.nT <= 128) launch_gcol_S<2>(spec, T, g, d, cd, s);
+  else if (g.nT <= 256) launch_gcol_S<4>(spec, T, g, d, cd, s);
+  else if (g.nT <= 512) launch_gcol_S<8>(spec, T, g, d, cd, s);
+  else if (g.nT <= 1024) launch_gcol_S<16>(spec, T, g, d, cd, s);
+  else launch_gcol_S<32>(spec, T, g, d, cd, s);
 }
 
 }  // namespace ash

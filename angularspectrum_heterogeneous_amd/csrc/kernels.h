@@ -142,7 +142,6 @@ struct Tables {
   const float2* twy;     // [nY]
   const float2* twc;     // column-transform pass twiddles: forward passes, then inverse passes
   const float2* twgt;    // [nT] exp(-2 pi i k / nT): column packing
-  DftMat dmx, dmy, dmt;  // axes that run the general-size kernels
 };
 
 struct Geom {
@@ -693,10 +692,10 @@ enum ColMode : int {
   COL_LOAD = 0,    // real field in -> spectrum (+ I_before, max|p| of the input)
   COL_NL = 1,      // taper * nonlinear step
   COL_TAPER = 2,   // taper only
-  COL_FINAL = 3,   // sources + reductions (+ spectrum rewrite if a source was added)
+  COL_FINAL = 3,   // reductions (read only)
   COL_STORE = 4,   // spectrum -> real field
   COL_RAWNL = 5,   // real field in -> nonlinear step -> real field out (no FFT)
-  COL_FINAL_SRC = 6,  // COL_FINAL on a step that injects source slices
+  COL_INJECT = 6,  // source slices added to the spectrum (columns with a source only)
   COL_TOREAL = 7,  // spectrum -> taper -> real field (the learned step's input)
   COL_MAXABS = 8,  // spectrum -> taper -> per-block max|p| into ColDesc::partial (read only)
   COL_TOF = 9,     // spectrum -> time of flight of the column into ColDesc::tof (read only)
@@ -740,7 +739,7 @@ struct ColDesc {
   unsigned* stats;   // [max_rows+1] max|p| bits; COL_LOAD writes slot 0, COL_FINAL slot row+1
   double* ibefore;   // [nX*nY] previous-step intensity (FP64)
   int cax;           // index of the on-axis column (nX/2, nY/2)
-  // sources (COL_FINAL)
+  // sources (COL_INJECT)
   const float* src[4];
   int n_src;
   const unsigned char* smask;
@@ -752,9 +751,13 @@ struct ColDesc {
 // Tone burst of the bowl and sparse-array sources in FP64, rounded to float32 once:
 // p0 exp(-(1.05 tm w0 / (ncycles pi))^(2 dur)) sin(w0 tm), tm = t - delay
 // (ASS:1061-1064, ASS:1196-1200, validate_transcranial.py:307-309).
+// With the usual exponent 4 the envelope is exactly zero in FP64 past 5.23 of its scale
+// (exp(-746) underflows), so the exponential, power and sine are left out there: most
+// of a column's samples lie outside the burst.
 __device__ __forceinline__ float tone_burst(double tm, double w0, double ncyc, double cexp, double p0) {
-  const double env = exp(-pow(1.05 * tm * w0 / (ncyc * 3.14159265358979323846), cexp));
-  return (float)(env * sin(w0 * tm) * p0);
+  const double a = 1.05 * tm * w0 / (ncyc * 3.14159265358979323846);
+  if (cexp == 4.0 && (a * a) * (a * a) > 746.0) return 0.f;
+  return (float)(exp(-pow(a, cexp)) * sin(w0 * tm) * p0);
 }
 
 // Dense field of a sparse source: out[c][t] = mask[c] ? tone_burst(taxis[t] - delay[c]) : 0.
