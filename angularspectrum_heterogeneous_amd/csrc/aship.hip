@@ -154,6 +154,7 @@ struct ash_plan {
   double* ibefore = nullptr;
   int* d_row = nullptr;
   double* obl_acc = nullptr;  // [2] power-weighted obliquity sums of the current step
+  double2* obl_part = nullptr;  // [nX * nfb] their per-block parts (useNonlinearityObliquity)
   unsigned* red = nullptr;    // [RED_WORDS] max|p| partials, global max, sub-cycling cap counter
   Tables T{};
   std::vector<void*> allocs;
@@ -593,13 +594,13 @@ void xinv(ash_plan* p, int epi, const EpiDesc& e, hipStream_t s) {
 template <int L>
 void launch_ypower_L(ash_plan* p, hipStream_t s) {
   const dim3 grid(p->g.nX * p->g.nfb);
-  if (p->rvy) hipLaunchKernelGGL((k_ypower<L, 1>), grid, dim3(LNT), 0, s, p->spec, p->T, p->g, p->obl_acc);
-  else hipLaunchKernelGGL((k_ypower<L, 0>), grid, dim3(LNT), 0, s, p->spec, p->T, p->g, p->obl_acc);
+  if (p->rvy) hipLaunchKernelGGL((k_ypower<L, 1>), grid, dim3(LNT), 0, s, p->spec, p->T, p->g, p->obl_part);
+  else hipLaunchKernelGGL((k_ypower<L, 0>), grid, dim3(LNT), 0, s, p->spec, p->T, p->g, p->obl_part);
 }
 void ypower(ash_plan* p, hipStream_t s) {
   ProfScope ps(p, ASH_K_YPASS, s);
   if (p->gen_y) {
-    gen_ypower(p->spec, p->T, p->g, p->dmy, p->obl_acc, s);
+    gen_ypower(p->spec, p->T, p->g, p->dmy, p->obl_part, s);
     return;
   }
   DISPATCH_L(p->g.nY, launch_ypower_L<L>(p, s));
@@ -757,9 +758,9 @@ void nl_obliquity(ash_plan* p, ColDesc& cd, hipStream_t s) {
   c.mode = COL_TAPER;
   c.nl = NL_NONE;
   column(p, c, s);
-  hipLaunchKernelGGL(k_zero2, dim3(1), dim3(1), 0, s, p->obl_acc);
   xfwd(p, s);
   ypower(p, s);
+  hipLaunchKernelGGL(k_sum_pairs, dim3(1), dim3(1024), 0, s, p->obl_part, p->g.nX * p->g.nfb, p->obl_acc);
   EpiDesc e = epi_base(p);
   e.scale = 1.f / (float)p->g.nX;
   xinv(p, 2, e, s);  // fw = sa = 0: scale and DC/Nyquist projection only
@@ -768,14 +769,16 @@ void nl_obliquity(ash_plan* p, ColDesc& cd, hipStream_t s) {
 }
 
 // The composite march step (ASS:874-913) on the spectral state, leaving the
-// state after the last attenuation visit with epilogue `epi_last` fused.
-void enqueue_composite(ash_plan* p, double dz, int epi_last, const EpiDesc& elast, hipStream_t s) {
+// state after the last attenuation visit with epilogue `epi_last` fused.  `row`: the
+// device step counter that the nonlinear pass advances, or null.
+void enqueue_composite(ash_plan* p, double dz, int epi_last, const EpiDesc& elast, int* row, hipStream_t s) {
   EpiDesc e = epi_base(p);
   ColDesc cd = col_base(p);
   cd.dz = dz;
   cd.beta_tvd = (float)beta_tvd(p, dz);
   cd.nl = nl_kind(p);
   cd.subcycle = is_kt(cd.nl) ? p->d.subcycle : 0;  // only the KT update sub-cycles (ASS:842-859)
+  cd.row = row;
   if (p->d.useSplitStep) {
     // attenuation half + propagator half, merged (both diagonal in k-space)
     xfwd(p, s);
@@ -821,7 +824,7 @@ void enqueue_step(ash_plan* p, const ash_step_io* io, hipStream_t s) {
   EpiDesc el = epi_base(p);
   el.fw = p->d.useFreqWeightedBoundary;
   el.sa = p->d.useSuperAbsorbing;
-  enqueue_composite(p, io->dz, 2, el, s);
+  enqueue_composite(p, io->dz, 2, el, p->d_row, s);
   ScreenDesc sd{};
   sd.sa_strength = (float)p->d.superAbsorbingStrength;
   sd.inv2dy = (float)(1.0 / (2 * p->d.dY));
@@ -880,7 +883,6 @@ void enqueue_step(ash_plan* p, const ash_step_io* io, hipStream_t s) {
     ct.tofref = p->tofref;
     column(p, ct, s);
   }
-  hipLaunchKernelGGL(k_advance_row, dim3(1), dim3(1), 0, s, p->d_row);
 }
 
 int load_real(ash_plan* p, const float* in, uint32_t* stats, double* ib, hipStream_t s) {
@@ -975,6 +977,8 @@ int ash_plan_create(const ash_desc* desc, ash_plan** out) try {
       (e = dalloc((void**)&p->ibefore, (size_t)d.nX * d.nY * sizeof(double))) != hipSuccess ||
       (e = dalloc((void**)&p->d_row, 64)) != hipSuccess ||
       (e = dalloc((void**)&p->obl_acc, 64)) != hipSuccess ||
+      (d.useNonlinearityObliquity &&
+       (e = dalloc((void**)&p->obl_part, (size_t)d.nX * p->g.nfb * sizeof(double2))) != hipSuccess) ||
       (e = dalloc((void**)&p->red, RED_WORDS * sizeof(unsigned))) != hipSuccess)
     return fail(ASH_E_HIP, std::string("hipMalloc: ") + hipGetErrorString(e));
   // padding bins are read (masked) but never written: clear once
@@ -1062,7 +1066,7 @@ int ash_step(ash_plan* p, const ash_step_io* io, void* stream) try {
   if (rc) return rc;
   hipStream_t s = (hipStream_t)stream;
   if (io->row != p->host_row) {
-    hipLaunchKernelGGL(k_set_row, dim3(1), dim3(1), 0, s, p->d_row, io->row);
+    hipLaunchKernelGGL(k_set_row, dim3(1), dim3(1), 0, s, p->d_row, io->row - 1);
   }
   if (plain_step(p, io)) {
     const bool same = p->gexec && same_io(p->gkey, *io);
@@ -1243,7 +1247,7 @@ int ash_batch_step(ash_batch* b, ash_plan* const* plans, const ash_step_io* ios,
   hipStream_t s = (hipStream_t)stream;
   for (int i = 0; i < n; ++i)
     if (ios[i].row != plans[i]->host_row)
-      hipLaunchKernelGGL(k_set_row, dim3(1), dim3(1), 0, s, plans[i]->d_row, ios[i].row);
+      hipLaunchKernelGGL(k_set_row, dim3(1), dim3(1), 0, s, plans[i]->d_row, ios[i].row - 1);
   if (all_plain) {
     bool same = b->gexec && (int)b->plans.size() == n;
     for (int i = 0; same && i < n; ++i)
@@ -1319,7 +1323,7 @@ int ash_march_step(ash_plan* p, const float* in, float* out, void* stream) try {
   hipStream_t s = (hipStream_t)stream;
   load_real(p, in, nullptr, nullptr, s);
   EpiDesc e = epi_base(p);
-  enqueue_composite(p, p->dz, 0, e, s);
+  enqueue_composite(p, p->dz, 0, e, nullptr, s);
   store_real(p, out, s);
   p->loaded = true;
   return check_launch();
@@ -1600,7 +1604,7 @@ int ash_profile_step(ash_plan* p, const ash_step_io* io, int32_t n_iter, float* 
   p->prof_ev.clear();
   p->ev_next = 0;
   p->prof_on = true;
-  hipLaunchKernelGGL(k_set_row, dim3(1), dim3(1), 0, s, p->d_row, io->row);
+  hipLaunchKernelGGL(k_set_row, dim3(1), dim3(1), 0, s, p->d_row, io->row - 1);
   for (int it = 0; it < n_iter; ++it) enqueue_step(p, io, s);
   p->prof_on = false;
   p->host_row = io->row + n_iter;

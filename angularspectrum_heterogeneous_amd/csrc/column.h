@@ -568,6 +568,7 @@ __global__ __launch_bounds__(256) void k_column(float2* __restrict__ spec, Table
   const LaneCol<S, LPC, STRIDED, false> lc{ln, lane, t0, NT_};
   constexpr bool FIN = MODE == COL_FINAL;
   const int row = (FIN || MODE == COL_TOF) ? *d.row : 0;
+  if ((MODE == COL_NL || MODE == COL_TOREAL) && d.row && blockIdx.x == 0 && tid == 0) *d.row += 1;
   // Burgers coefficient, scaled by the beam obliquity when requested (ASS:934)
   const double Nn = d.nscale ? d.N * (d.nscale[0] / (d.nscale[1] + 1e-30)) : d.N;
   float wmax = 0.f;  // running max|p| of this lane's columns (stats, COL_MAXABS)

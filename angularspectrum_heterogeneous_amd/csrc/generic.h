@@ -425,10 +425,10 @@ __global__ __launch_bounds__(512) void k_gy_pass(float2* __restrict__ spec, Tabl
 }
 
 // Power-weighted obliquity sums of a (kx row, f block) tile (as k_ypower): forward
-// DFT along y, then acc[0] += sum P k/k_z, acc[1] += sum P over propagating modes.
+// DFT along y, then sum P k/k_z and sum P over propagating modes, a pair per block.
 template <bool EVEN, int T_>
 __global__ __launch_bounds__(512) void k_gy_power(const float2* __restrict__ spec, Tables T, Geom g, DftMat d,
-                                                  double* __restrict__ acc) {
+                                                  double2* __restrict__ part) {
   extern __shared__ float4 eo[];
   __shared__ double sred[2][8];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
@@ -450,11 +450,7 @@ __global__ __launch_bounds__(512) void k_gy_power(const float2* __restrict__ spe
     hm_emit<EVEN, false>(d, a[i], t.lo + i, lane, [&](int pos, float2 v) {
       const double ky = T.ky[pos];
       const double kz2 = kz2_of(km, kperp2(kx, ky));
-      if (km > 0.0 && kz2 > 0.0) {
-        const double P = (double)v.x * v.x + (double)v.y * v.y;
-        num += P * km / fmax(sqrt(kz2), km * 1e-6);
-        den += P;
-      }
+      if (km > 0.0 && kz2 > 0.0) obliquity_term(v, km, kz2, num, den);
     });
   }
   for (int o = 32; o > 0; o >>= 1) {
@@ -466,8 +462,7 @@ __global__ __launch_bounds__(512) void k_gy_power(const float2* __restrict__ spe
   if (tid == 0) {
     double s0 = 0.0, s1 = 0.0;
     for (int w = 0; w < W; ++w) { s0 += sred[0][w]; s1 += sred[1][w]; }
-    atomicAdd(acc, s0);
-    atomicAdd(acc + 1, s1);
+    part[blockIdx.x] = make_double2(s0, s1);
   }
 }
 
@@ -634,6 +629,7 @@ __global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restri
   const LaneCol<S, 64, false, true> lc{lane, lane, t0, nT};
   const int row = (FIN || MODE == COL_TOF) ? *d.row : 0;
   const double Nn = d.nscale ? d.N * (d.nscale[0] / (d.nscale[1] + 1e-30)) : d.N;
+  if (MODE == COL_NL && d.row && blockIdx.x == 0 && tid == 0) *d.row += 1;
   float wmax = 0.f;
   int nsub_global = 1;
   if constexpr (NLK != NL_NONE) {

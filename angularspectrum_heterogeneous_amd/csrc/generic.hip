@@ -74,10 +74,10 @@ void gen_ypass(float2* spec, const Tables& T, const Geom& g, const DftMat& d, co
   else DISPATCH_TILES(d, hipLaunchKernelGGL((k_gy_pass<EVEN, T_, false>), grid, block, lds, s, spec, T, g, d, op));
 }
 
-void gen_ypower(const float2* spec, const Tables& T, const Geom& g, const DftMat& d, double* acc, hipStream_t s) {
+void gen_ypower(const float2* spec, const Tables& T, const Geom& g, const DftMat& d, double2* part, hipStream_t s) {
   const dim3 grid(g.nX * g.nfb), block(64 * line_waves(d));
   const size_t lds = line_lds(d);
-  DISPATCH_TILES(d, hipLaunchKernelGGL((k_gy_power<EVEN, T_>), grid, block, lds, s, spec, T, g, d, acc));
+  DISPATCH_TILES(d, hipLaunchKernelGGL((k_gy_power<EVEN, T_>), grid, block, lds, s, spec, T, g, d, part));
 }
 
 void gen_ysa(float2* spec, const Tables& T, const Geom& g, const ScreenDesc& sd, hipStream_t s) {

@@ -14,7 +14,7 @@ void dft_matrix_fill(const DftMat& d, const float2* tw, float4* A, hipStream_t s
 void gen_xfwd(float2* spec, const Geom& g, const DftMat& d, hipStream_t s);
 void gen_xinv(int epi, float2* spec, const Tables& T, const Geom& g, const DftMat& d, const EpiDesc& e, hipStream_t s);
 void gen_ypass(float2* spec, const Tables& T, const Geom& g, const DftMat& d, const OpDesc& op, hipStream_t s);
-void gen_ypower(const float2* spec, const Tables& T, const Geom& g, const DftMat& d, double* acc, hipStream_t s);
+void gen_ypower(const float2* spec, const Tables& T, const Geom& g, const DftMat& d, double2* part, hipStream_t s);
 void gen_ysa(float2* spec, const Tables& T, const Geom& g, const ScreenDesc& sd, hipStream_t s);
 // Column pass cd.mode on nT outside the FFT set; its blocks (one partial each for COL_MAXABS).
 void gen_column(float2* spec, const Tables& T, const Geom& g, const DftMat& d, const ColDesc& cd, hipStream_t s);

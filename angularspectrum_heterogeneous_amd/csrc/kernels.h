@@ -733,7 +733,8 @@ struct ColDesc {
   const int32_t* cflag;  // when set, only columns with cflag[c] != 0 are processed
   const double* nscale;  // when set, N is scaled by nscale[0] / (nscale[1] + 1e-30) (beam obliquity)
   // reductions (COL_FINAL / COL_LOAD)
-  const int* row;    // device step counter; outputs go to row `*row`
+  int* row;          // device step counter: advanced by the step's first column pass (COL_NL,
+                     // COL_TOREAL) when set; outputs of the passes after it go to row `*row`
   int max_rows;
   float* pnp; float* ppp; float* pI; float* pIloss; float* pax;
   unsigned* stats;   // [max_rows+1] max|p| bits; COL_LOAD writes slot 0, COL_FINAL slot row+1
@@ -921,16 +922,54 @@ static __global__ __launch_bounds__(1024) void k_reduce_max(const unsigned* __re
     out[0] = r;
   }
 }
-static __global__ void k_zero2(double* a) { a[0] = 0.0; a[1] = 0.0; }
+
+// P k/k_z and P of one mode, added to (num, den); k^2 - kx^2 - ky^2 = kz2 > 0 and k_z =
+// max(sqrt(kz2), 1e-6 k).  1/k_z is the hardware's FP64 estimate with two Newton steps
+// (to the last bit or two) instead of a square root and a division.
+__device__ __forceinline__ void obliquity_term(float2 v, double km, double kz2, double& num, double& den) {
+  const double z = fmax(kz2, km * km * 1e-12);
+  double r = __builtin_amdgcn_rsq(z);
+  r *= 1.5 - 0.5 * z * r * r;
+  r *= 1.5 - 0.5 * z * r * r;
+  const double P = (double)v.x * v.x + (double)v.y * v.y;
+  num += P * (km * r);
+  den += P;
+}
+
+// Adds the n per-block pairs of the obliquity sums into acc[0..1], in a fixed order.
+// One block.  (Atomics of all blocks on one pair of doubles queued at the L2: at
+// 192x192x512 the 3264 blocks of k_ypower took 90 us, now 30 and 5 here.)
+static __global__ __launch_bounds__(1024) void k_sum_pairs(const double2* __restrict__ part, int n,
+                                                           double* __restrict__ acc) {
+  __shared__ double2 s_red[16];
+  double a = 0.0, b = 0.0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < n; i += 1024) {
+    const double2 v = part[i];
+    a += v.x;
+    b += v.y;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    a += __shfl_xor(a, o, 64);
+    b += __shfl_xor(b, o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = make_double2(a, b);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 16; ++w) { a += s_red[w].x; b += s_red[w].y; }
+    acc[0] = a;
+    acc[1] = b;
+  }
+}
 
 // y transform of one (kx row, f block) tile and the power-weighted obliquity
-// sums of its plane-wave content (ASS:630-643): acc[0] += sum P k/k_z and
-// acc[1] += sum P over the propagating modes, P = |F|^2, k = 2 pi f / c0,
-// k_z = max(sqrt(k^2 - kx^2 - ky^2), 1e-6 k); f = 0 and evanescent modes
-// weigh 0 (ASS:598-627).  The state is only read.
+// sums of its plane-wave content (ASS:630-643): sum P k/k_z and sum P over the
+// propagating modes, P = |F|^2, k = 2 pi f / c0, k_z = max(sqrt(k^2 - kx^2 - ky^2),
+// 1e-6 k); f = 0 and evanescent modes weigh 0 (ASS:598-627).  One pair per block, for
+// k_sum_pairs.  The state is only read.
 template <int L, int V>
 __global__ __launch_bounds__(LNT) void k_ypower(const float2* __restrict__ spec, Tables T, Geom g,
-                                                double* __restrict__ acc) {
+                                                double2* __restrict__ part) {
   __shared__ float2 tw[L];
   __shared__ float2 buf[L * LF];
   __shared__ double sred[2][LNT / 64];
@@ -957,12 +996,7 @@ __global__ __launch_bounds__(LNT) void k_ypower(const float2* __restrict__ spec,
     for (int pos = tid / LF; pos < L; pos += LNT / LF) {
       const double ky = T.ky[pos];
       const double kz2 = kz2_of(km, kperp2(kx, ky));
-      if (kz2 > 0.0) {
-        const float2 v = buf[LY::idx(line, pos)];
-        const double P = (double)v.x * v.x + (double)v.y * v.y;
-        num += P * km / fmax(sqrt(kz2), km * 1e-6);
-        den += P;
-      }
+      if (kz2 > 0.0) obliquity_term(buf[LY::idx(line, pos)], km, kz2, num, den);
     }
   }
   for (int o = 32; o > 0; o >>= 1) {
@@ -974,10 +1008,8 @@ __global__ __launch_bounds__(LNT) void k_ypower(const float2* __restrict__ spec,
   if (tid == 0) {
     double a = 0.0, b = 0.0;
     for (int w = 0; w < LNT / 64; ++w) { a += sred[0][w]; b += sred[1][w]; }
-    atomicAdd(acc, a);
-    atomicAdd(acc + 1, b);
+    part[blockIdx.x] = make_double2(a, b);
   }
 }
-static __global__ void k_advance_row(int* row) { *row += 1; }
 
 }  // namespace ash
