@@ -387,7 +387,8 @@ int build_tables(ash_plan* p) {
     p->allocs.push_back(a);
     p->ws_bytes += (int64_t)bytes;
     m->A = (const float4*)a;
-    dft_matrix_fill(*m, tw, (float4*)a, nullptr);
+    m->tw = tw;
+    dft_matrix_fill(*m, (float4*)a, nullptr);
     return ASH_OK;
   };
   if (p->gen_x && (rc = matrix(nX, false, p->T.twx, &p->dmx))) return rc;

@@ -14,6 +14,13 @@
 // table exp(-2 pi i k / n) at (j k) mod n, so every entry is exact to one rounding,
 // and lie in memory in the order in which the lanes load them (k_dft_matrix).
 //
+// A length n = p q with a small odd factor p runs a p-point DFT first (decimation in
+// frequency): X_{p k + r} is the q-point DFT over s of W_n^{s r} sum_m x_{s + q m}
+// W_p^{m r}, so the matrix is that of q and a p-th of the products remain.  The radix
+// stage happens where the tile is folded into LDS; the inverse half of the y pass,
+// whose input lies in the order p k + r, runs it last instead.  At 365 = 5 * 73 an x
+// sweep takes 115 us instead of 211, the y pass 285 instead of 485.
+//
 // Per element of a complex line that is 2n flops (odd n) or n (even n): at
 // 365x365x425 an x sweep does 20.7 GFLOP over 454 MB, so the matrix cores bound it
 // above n of about 200 and memory below.  There, against the direct sums through LDS
@@ -55,7 +62,7 @@ __device__ __forceinline__ int hm_col(const DftMat& d, int j) {
 // tile at a time).  Each order is the faster one for its kernels: an x sweep at
 // 365x365x425 takes 225 against 255 us, a column inverse there 323 against 408 us.
 template <bool EVEN>
-__global__ __launch_bounds__(256) void k_dft_matrix(DftMat d, const float2* __restrict__ tw, float4* __restrict__ out) {
+__global__ __launch_bounds__(256) void k_dft_matrix(DftMat d, float4* __restrict__ out) {
   const long tot = (long)d.R * (d.Kp / 8) * 64;
   for (long e = (long)blockIdx.x * 256 + threadIdx.x; e < tot; e += (long)gridDim.x * 256) {
     const int lane = (int)(e % 64);
@@ -66,7 +73,7 @@ __global__ __launch_bounds__(256) void k_dft_matrix(DftMat d, const float2* __re
     for (int q = 0; q < 2; ++q) {
       const int j = hm_pos<EVEN>(d, 8 * g + 4 * q + (lane >> 4));
       float2 w = make_float2(0.f, 0.f);
-      if (k < d.rows && j <= d.h) w = tw[(int)(((long)j * k) % d.n)];
+      if (k < d.rows && j <= d.h) w = d.tw[(int)(((long)j * k) % d.q) * d.p];
       v[2 * q] = w.x;
       v[2 * q + 1] = -w.y;
     }
@@ -88,11 +95,12 @@ struct LineAcc {
   f32x4 c[NP][2], s[NP][2];                // [parity][re, im]
 };
 
-// The row tiles of a wave: [lo, lo + cnt) of d.R, counts that differ by at most one.
+// The row tiles of a wave: [lo, lo + cnt) of n, counts that differ by at most one.  A
+// line has p R of them, tile t = row tile t % R of residue t / R.
 struct Tiles { int lo, cnt; };
-__device__ __forceinline__ Tiles hm_tiles(const DftMat& d, int wave, int W) {
-  const int lo = wave * d.R / W;
-  return {lo, (wave + 1) * d.R / W - lo};
+__device__ __forceinline__ Tiles hm_tiles(int n, int wave, int W) {
+  const int lo = wave * n / W;
+  return {lo, (wave + 1) * n / W - lo};
 }
 
 // Walks ng matrix column groups through a ring of U register buffers: use(q) consumes
@@ -165,10 +173,18 @@ __device__ __forceinline__ void hm_line_n(const float4* eo, const DftMat& d, int
         });
   }
 }
-// The wave's tiles, T_ or T_ - 1 of them (T_ = ceil(R / W)).
-template <bool EVEN, int T_>
+// The wave's tiles, T_ or T_ - 1 of them (T_ = ceil(p R / W)): together when they are
+// rows of one matrix product (p = 1), else one after the other.
+template <bool EVEN, int T_, bool RADIX>
 __device__ __forceinline__ void hm_line(const float4* eo, const DftMat& d, const Tiles& t, int lane, LineAcc<EVEN> (&a)[T_]) {
-  if (t.cnt == T_) hm_line_n<EVEN, T_>(eo, d, t.lo, lane, a);
+  if constexpr (RADIX) {
+#pragma unroll
+    for (int i = 0; i < T_; ++i)
+      if (i < t.cnt) {
+        const int r = (t.lo + i) / d.R;
+        hm_line_n<EVEN, 1>(eo + r * d.Kp * 16, d, t.lo + i - r * d.R, lane, a + i);
+      }
+  } else if (t.cnt == T_) hm_line_n<EVEN, T_>(eo, d, t.lo, lane, a);
   else if constexpr (T_ > 1) hm_line_n<EVEN, T_ - 1>(eo, d, t.lo, lane, a);
 }
 
@@ -190,32 +206,141 @@ __device__ __forceinline__ void hm_values(const LineAcc<EVEN>& a, int i, float2&
   Q = make_float2(cr - si, ci + sr);
 }
 
-// f(position, value) for every output of this lane in one tile
-template <bool EVEN, bool INV, class F>
-__device__ __forceinline__ void hm_emit(const DftMat& d, const LineAcc<EVEN>& a, int rt, int lane, F f) {
+// f(position, value) for every output of this lane in tile t: position(k, r) of output k
+// of residue r
+template <bool EVEN, bool INV, class Pos, class F>
+__device__ __forceinline__ void hm_emit_at(const DftMat& d, const LineAcc<EVEN>& a, int t, int lane, Pos position, F f) {
+  const int r = t / d.R, rt = t - r * d.R;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int k = 16 * rt + 4 * (lane >> 4) + i;
     float2 P, Q, P2, Q2;
     hm_values<EVEN>(a, i, P, Q, P2, Q2);
     if (k < d.rows) {
-      f(k, INV ? Q : P);
-      if (k > 0) f(d.n - k, INV ? P : Q);
+      f(position(k, r), INV ? Q : P);
+      if (k > 0) f(position(d.q - k, r), INV ? P : Q);
       if constexpr (EVEN) {
         const int k2 = d.h - k;
         if (k2 != k) {
-          f(k2, INV ? Q2 : P2);
-          if (k > 0) f(d.h + k, INV ? P2 : Q2);
+          f(position(k2, r), INV ? Q2 : P2);
+          if (k > 0) f(position(d.h + k, r), INV ? P2 : Q2);
         }
       }
     }
   }
 }
+template <bool EVEN, bool INV, class F>
+__device__ __forceinline__ void hm_emit(const DftMat& d, const LineAcc<EVEN>& a, int t, int lane, F f) {
+  hm_emit_at<EVEN, INV>(d, a, t, lane, [&](int k, int r) { return d.p * k + r; }, f);
+}
 
-// Folds a line tile into LDS; ld(position, line) reads one element.  The loads of
-// four rows are issued before the first is used.
-template <bool EVEN, class Ld>
+// cos and sin of 2 pi k / P, k = 1 .. P/2, as hi/lo pairs (fft_engine.h: constants
+// rounded to float would bias every transform the same way).
+template <int P> struct OddTrig;
+template <> struct OddTrig<3> {
+  static constexpr float ch[] = {-0.5f}, cl[] = {2.220446049250313e-16f};
+  static constexpr float sh[] = {0.8660253882408142f}, sl[] = {1.5543625053737742e-08f};
+};
+template <> struct OddTrig<5> {
+  static constexpr float ch[] = {0.30901700258255005f, -0.80901700258255f}, cl[] = {-8.207602597565256e-09f, 8.207602597565256e-09f};
+  static constexpr float sh[] = {0.9510565400123596f, 0.5877852439880371f}, sl[] = {-2.3717205976936384e-08f, 8.304436249773062e-09f};
+};
+template <> struct OddTrig<7> {
+  static constexpr float ch[] = {0.6234897971153259f, -0.22252093255519867f, -0.9009688496589661f}, cl[] = {4.743407444607328e-09f, -1.4011156679316628e-09f, -1.8243452970523322e-08f};
+  static constexpr float sh[] = {0.7818315029144287f, 0.9749279022216797f, 0.4338837265968323f}, sl[] = {-2.0446398352191864e-08f, 9.960143820819667e-09f, 1.252072578949992e-08f};
+};
+template <> struct OddTrig<9> {
+  static constexpr float ch[] = {0.7660444378852844f, 0.1736481785774231f, -0.5f, -0.9396926164627075f}, cl[] = {5.2336934786012534e-09f, -9.104926812497638e-10f, 2.220446049250313e-16f, -4.323200908373792e-09f};
+  static constexpr float sh[] = {0.6427876353263855f, 0.9848077297210693f, 0.8660253882408142f, 0.3420201539993286f}, sl[] = {-2.5639845802061245e-08f, 2.3291137907222037e-08f, 1.5543625053737742e-08f, -1.0673659289750503e-08f};
+};
+// P-point DFT in registers, P odd: with a_m = x_m + x_{P-m}, b_m = x_m - x_{P-m},
+// y_r = x_0 + sum cos(2 pi m r / P) a_m -+ i sum sin(2 pi m r / P) b_m, y_{P-r} its mirror.
+template <int P, bool INV>
+__device__ __forceinline__ void odd_dft(float2* x) {
+  using C = OddTrig<P>;
+  constexpr int H = P / 2;
+  float2 a[H], b[H];
+#pragma unroll
+  for (int m = 1; m <= H; ++m) {
+    a[m - 1] = cadd(x[m], x[P - m]);
+    b[m - 1] = csub(x[m], x[P - m]);
+  }
+  const float2 x0 = x[0];
+  float2 sum = x0;
+#pragma unroll
+  for (int m = 0; m < H; ++m) sum = cadd(sum, a[m]);
+#pragma unroll
+  for (int r = 1; r <= H; ++r) {
+    float2 A = x0, B = make_float2(0.f, 0.f);
+#pragma unroll
+    for (int m = 1; m <= H; ++m) {
+      const int j = (m * r) % P, jj = j > H ? P - j : j;
+      if (jj == 0) {
+        A = cadd(A, a[m - 1]);
+      } else {
+        const float ch = C::ch[jj - 1], cl = C::cl[jj - 1];
+        const float sh = j > H ? -C::sh[jj - 1] : C::sh[jj - 1], sl = j > H ? -C::sl[jj - 1] : C::sl[jj - 1];
+        A = make_float2(fmaf(a[m - 1].x, ch, fmaf(a[m - 1].x, cl, A.x)), fmaf(a[m - 1].y, ch, fmaf(a[m - 1].y, cl, A.y)));
+        B = make_float2(fmaf(b[m - 1].x, sh, fmaf(b[m - 1].x, sl, B.x)), fmaf(b[m - 1].y, sh, fmaf(b[m - 1].y, sl, B.y)));
+      }
+    }
+    const float2 u = make_float2(A.x + B.y, A.y - B.x), v = make_float2(A.x - B.y, A.y + B.x);
+    x[r] = INV ? v : u;
+    x[P - r] = INV ? u : v;
+  }
+  x[0] = sum;
+}
+// x_r *= W_n^{s r} (conjugated for the inverse), r = 1 .. P-1; s r < n
+template <int P, bool INV>
+__device__ __forceinline__ void odd_twiddle(float2* x, const float2* tw, int s) {
+#pragma unroll
+  for (int r = 1; r < P; ++r) {
+    float2 w = tw[s * r];
+    if (INV) w.y = -w.y;
+    x[r] = cmul(x[r], w);
+  }
+}
+
+// Folds a line tile into LDS (rows [residue r][matrix column][line]); ld(position, line)
+// reads one element.  All loads of a row (of four rows when p = 1) are issued before the
+// first is used.
+template <bool EVEN, bool INV, int P, class Ld>
+__device__ __forceinline__ void hm_fold_p(float4* eo, const DftMat& d, int tid, int nthr, Ld ld) {
+  const int line = tid & 15, step = nthr >> 4;
+  for (int rr = tid >> 4; rr < d.Kp; rr += step) {
+    const int j = hm_pos<EVEN>(d, rr);
+    const bool pair = j > 0 && 2 * j != d.q;
+    const int s0 = min(j, d.h), s1 = pair && j <= d.h ? d.q - j : s0;
+    float2 a[P], b[P];
+#pragma unroll
+    for (int m = 0; m < P; ++m) {
+      a[m] = ld(s0 + d.q * m, line);
+      b[m] = ld(s1 + d.q * m, line);
+    }
+    odd_dft<P, INV>(a);
+    odd_dft<P, INV>(b);
+    odd_twiddle<P, INV>(a, d.tw, s0);
+    odd_twiddle<P, INV>(b, d.tw, s1);
+#pragma unroll
+    for (int r = 0; r < P; ++r) {
+      float4 v = make_float4(a[r].x, a[r].y, 0.f, 0.f);
+      if (pair) v = make_float4(a[r].x + b[r].x, a[r].y + b[r].y, a[r].x - b[r].x, a[r].y - b[r].y);
+      if (j > d.h) v = make_float4(0.f, 0.f, 0.f, 0.f);  // matrix padding
+      eo[(r * d.Kp + rr) * 16 + line] = v;
+    }
+  }
+}
+template <bool EVEN, bool INV, bool RADIX, class Ld>
 __device__ __forceinline__ void hm_fold(float4* eo, const DftMat& d, int tid, int nthr, Ld ld) {
+  if constexpr (RADIX) {
+    switch (d.p) {
+      case 3: hm_fold_p<EVEN, INV, 3>(eo, d, tid, nthr, ld); break;
+      case 5: hm_fold_p<EVEN, INV, 5>(eo, d, tid, nthr, ld); break;
+      case 7: hm_fold_p<EVEN, INV, 7>(eo, d, tid, nthr, ld); break;
+      default: hm_fold_p<EVEN, INV, 9>(eo, d, tid, nthr, ld); break;
+    }
+    return;
+  }
   const int line = tid & 15, step = nthr >> 4;
   for (int r0 = tid >> 4; r0 < d.Kp; r0 += 4 * step) {
     float2 a[4], b[4];
@@ -239,35 +364,60 @@ __device__ __forceinline__ void hm_fold(float4* eo, const DftMat& d, int tid, in
   }
 }
 
+// The radix stage after the inverse q-point transforms z[r][s] (rows of 16 lines):
+// x_{s + q m} = sum_r W_p^{-m r} W_n^{-s r} z_r[s]; st(position, line, value) stores.
+template <int P, class St>
+__device__ __forceinline__ void hm_combine_p(const float2* z, const DftMat& d, int tid, int nthr, St st) {
+  const int line = tid & 15, step = nthr >> 4;
+  for (int s = tid >> 4; s < d.q; s += step) {
+    float2 x[P];
+#pragma unroll
+    for (int r = 0; r < P; ++r) x[r] = z[(r * d.q + s) * 16 + line];
+    odd_twiddle<P, true>(x, d.tw, s);
+    odd_dft<P, true>(x);
+#pragma unroll
+    for (int m = 0; m < P; ++m) st(s + d.q * m, line, x[m]);
+  }
+}
+template <class St>
+__device__ __forceinline__ void hm_combine(const float2* z, const DftMat& d, int tid, int nthr, St st) {
+  switch (d.p) {
+    case 3: hm_combine_p<3>(z, d, tid, nthr, st); break;
+    case 5: hm_combine_p<5>(z, d, tid, nthr, st); break;
+    case 7: hm_combine_p<7>(z, d, tid, nthr, st); break;
+    default: hm_combine_p<9>(z, d, tid, nthr, st); break;
+  }
+}
+
 // x-sweep, forward DFT along x.  Tile = (y, 16 f bins).  Padding lines past the last
 // bin are zero and stay zero, so no load or store is guarded.
-template <bool EVEN, int T_>
+template <bool EVEN, int T_, bool RADIX>
 __global__ __launch_bounds__(512) void k_gx_fwd(float2* __restrict__ spec, Geom g, DftMat d) {
   extern __shared__ float4 eo[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
   const int y = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
   const uint32_t sxb = (uint32_t)g.nY * g.MP * 8u;
   float2* base = spec + (long)y * g.MP + f0;
-  hm_fold<EVEN>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * sxb + line * 8u); });
+  hm_fold<EVEN, false, RADIX>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * sxb + line * 8u); });
   __syncthreads();
   const uint32_t lo = (lane & 15) * 8u;
-  const Tiles t = hm_tiles(d, wave, W);
+  const Tiles t = hm_tiles(d.p * d.R, wave, W);
   LineAcc<EVEN> a[T_];
-  hm_line<EVEN, T_>(eo, d, t, lane, a);
+  hm_line<EVEN, T_, RADIX>(eo, d, t, lane, a);
 #pragma unroll
   for (int i = 0; i < T_; ++i)
     if (i < t.cnt) hm_emit<EVEN, false>(d, a[i], t.lo + i, lane, [&](int pos, float2 v) { gst(base, pos * sxb + lo, v); });
 }
 
 // x-sweep, inverse DFT along x + the epilogues 0 and 1 of k_xfft_inv.
-template <bool EVEN, int T_, int EPI>
+template <bool EVEN, int T_, bool RADIX, int EPI>
 __global__ __launch_bounds__(512) void k_gx_inv(float2* __restrict__ spec, Tables T, Geom g, DftMat d, EpiDesc ep) {
   extern __shared__ float4 eo[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
   const int y = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
   const uint32_t sxb = (uint32_t)g.nY * g.MP * 8u;
   float2* base = spec + (long)y * g.MP + f0;
-  hm_fold<EVEN>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * sxb + line * 8u); });
+  hm_fold<EVEN, true, RADIX>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * sxb + line * 8u); });
   __syncthreads();
   const uint32_t lo = (lane & 15) * 8u;
   float ty = 1.f;
@@ -276,9 +426,9 @@ __global__ __launch_bounds__(512) void k_gx_inv(float2* __restrict__ spec, Table
     ty = ep.half ? T.tapy_h[y] : T.tapy_f[y];
     tx = ep.half ? T.tapx_h : T.tapx_f;
   }
-  const Tiles t = hm_tiles(d, wave, W);
+  const Tiles t = hm_tiles(d.p * d.R, wave, W);
   LineAcc<EVEN> a[T_];
-  hm_line<EVEN, T_>(eo, d, t, lane, a);
+  hm_line<EVEN, T_, RADIX>(eo, d, t, lane, a);
 #pragma unroll
   for (int i = 0; i < T_; ++i)
     if (i < t.cnt)
@@ -292,18 +442,18 @@ __global__ __launch_bounds__(512) void k_gx_inv(float2* __restrict__ spec, Table
 // projection, frequency-weighted mask and the SA x stencil on the masked values,
 // which pass through the tile's LDS (n * 16 float2 fit the folded tile) once every
 // wave holds its T row tiles in registers.
-template <bool EVEN, int T_>
+template <bool EVEN, int T_, bool RADIX>
 __global__ __launch_bounds__(512) void k_gx_inv_sa(float2* __restrict__ spec, Tables T, Geom g, DftMat d, EpiDesc ep) {
   extern __shared__ float4 eo[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
   const int y = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
   const uint32_t sxb = (uint32_t)g.nY * g.MP * 8u;
   float2* base = spec + (long)y * g.MP + f0;
-  hm_fold<EVEN>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * sxb + line * 8u); });
+  hm_fold<EVEN, true, RADIX>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * sxb + line * 8u); });
   __syncthreads();
-  const Tiles t = hm_tiles(d, wave, W);
+  const Tiles t = hm_tiles(d.p * d.R, wave, W);
   LineAcc<EVEN> a[T_];
-  hm_line<EVEN, T_>(eo, d, t, lane, a);
+  hm_line<EVEN, T_, RADIX>(eo, d, t, lane, a);
   __syncthreads();
   float2* b = reinterpret_cast<float2*>(eo);
   const float lgy = T.lgy[y];
@@ -364,18 +514,18 @@ __device__ __forceinline__ LineConst line_const(const Tables& T, const OpDesc& o
 // happen in registers, and only the folded rows return to LDS.  The operator is
 // evaluated at every position's own wavenumber (the grids are mirror images only up
 // to rounding, and one ulp decides a mode at the evanescent cutoff).
-template <bool EVEN, int T_, bool PRECISE>
+template <bool EVEN, int T_, bool RADIX, bool PRECISE>
 __global__ __launch_bounds__(512) void k_gy_pass(float2* __restrict__ spec, Tables T, Geom g, DftMat d, OpDesc op) {
   extern __shared__ float4 eo[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
   const int x = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
   const uint32_t syb = (uint32_t)g.MP * 8u;
   float2* base = spec + (long)x * g.nY * g.MP + f0;
-  hm_fold<EVEN>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * syb + line * 8u); });
+  hm_fold<EVEN, false, RADIX>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * syb + line * 8u); });
   __syncthreads();
-  const Tiles t = hm_tiles(d, wave, W);
+  const Tiles t = hm_tiles(d.p * d.R, wave, W);
   LineAcc<EVEN> a[T_];
-  hm_line<EVEN, T_>(eo, d, t, lane, a);
+  hm_line<EVEN, T_, RADIX>(eo, d, t, lane, a);
   __syncthreads();
   {
     const int line = lane & 15, m = f0 + line;
@@ -388,28 +538,29 @@ __global__ __launch_bounds__(512) void k_gy_pass(float2* __restrict__ spec, Tabl
       else o = visit_operator(op, kk, lc, m);
       return cmul(v, o);
     };
-    // folded row of position k from the values at k and n - k
-    auto put = [&](int k, float2 v, float2 vn, bool pair) {
-      v = apply(k, v);
+    // folded row of output k of residue r from the values at k and q - k
+    auto put = [&](int k, int r, float2 v, float2 vn, bool pair) {
+      v = apply(d.p * k + r, v);
       float4 e = make_float4(v.x, v.y, 0.f, 0.f);
       if (pair) {
-        vn = apply(d.n - k, vn);
+        vn = apply(d.p * (d.q - k) + r, vn);
         e = make_float4(v.x + vn.x, v.y + vn.y, v.x - vn.x, v.y - vn.y);
       }
-      eo[hm_col<EVEN>(d, k) * 16 + line] = e;
+      eo[(r * d.Kp + hm_col<EVEN>(d, k)) * 16 + line] = e;
     };
 #pragma unroll
     for (int i = 0; i < T_; ++i) {
       if (i < t.cnt) {
+        const int r = (t.lo + i) / d.R, rt = t.lo + i - r * d.R;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int k = 16 * (t.lo + i) + 4 * (lane >> 4) + q;
+          const int k = 16 * rt + 4 * (lane >> 4) + q;
           float2 P, Q, P2, Q2;
           hm_values<EVEN>(a[i], q, P, Q, P2, Q2);
           if (k < d.rows) {
-            put(k, P, Q, k > 0);
+            put(k, r, P, Q, k > 0);
             if constexpr (EVEN) {
-              if (d.h - k != k) put(d.h - k, P2, Q2, k > 0);
+              if (d.h - k != k) put(d.h - k, r, P2, Q2, k > 0);
             }
           }
         }
@@ -417,16 +568,28 @@ __global__ __launch_bounds__(512) void k_gy_pass(float2* __restrict__ spec, Tabl
     }
   }
   __syncthreads();
-  const uint32_t lo = (lane & 15) * 8u;
-  hm_line<EVEN, T_>(eo, d, t, lane, a);
+  hm_line<EVEN, T_, RADIX>(eo, d, t, lane, a);
+  if constexpr (!RADIX) {
+    const uint32_t lo = (lane & 15) * 8u;
+#pragma unroll
+    for (int i = 0; i < T_; ++i)
+      if (i < t.cnt) hm_emit<EVEN, true>(d, a[i], t.lo + i, lane, [&](int pos, float2 v) { gst(base, pos * syb + lo, v); });
+    return;
+  }
+  __syncthreads();
+  float2* z = reinterpret_cast<float2*>(eo);
 #pragma unroll
   for (int i = 0; i < T_; ++i)
-    if (i < t.cnt) hm_emit<EVEN, true>(d, a[i], t.lo + i, lane, [&](int pos, float2 v) { gst(base, pos * syb + lo, v); });
+    if (i < t.cnt)
+      hm_emit_at<EVEN, true>(d, a[i], t.lo + i, lane, [&](int k, int r) { return r * d.q + k; },
+                             [&](int pos, float2 v) { z[pos * 16 + (lane & 15)] = v; });
+  __syncthreads();
+  hm_combine(z, d, tid, blockDim.x, [&](int pos, int line, float2 v) { gst(base, pos * syb + line * 8u, v); });
 }
 
 // Power-weighted obliquity sums of a (kx row, f block) tile (as k_ypower): forward
 // DFT along y, then sum P k/k_z and sum P over propagating modes, a pair per block.
-template <bool EVEN, int T_>
+template <bool EVEN, int T_, bool RADIX>
 __global__ __launch_bounds__(512) void k_gy_power(const float2* __restrict__ spec, Tables T, Geom g, DftMat d,
                                                   double2* __restrict__ part) {
   extern __shared__ float4 eo[];
@@ -435,15 +598,15 @@ __global__ __launch_bounds__(512) void k_gy_power(const float2* __restrict__ spe
   const int x = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
   const uint32_t syb = (uint32_t)g.MP * 8u;
   const float2* base = spec + (long)x * g.nY * g.MP + f0;
-  hm_fold<EVEN>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * syb + line * 8u); });
+  hm_fold<EVEN, false, RADIX>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * syb + line * 8u); });
   __syncthreads();
   const int m = f0 + (lane & 15);
   const double km = m <= g.M ? T.ka[m] : 0.0;  // ka[0] = 0: the DC bin weighs nothing
   const double kx = T.kx[x];
   double num = 0.0, den = 0.0;
-  const Tiles t = hm_tiles(d, wave, W);
+  const Tiles t = hm_tiles(d.p * d.R, wave, W);
   LineAcc<EVEN> a[T_];
-  hm_line<EVEN, T_>(eo, d, t, lane, a);
+  hm_line<EVEN, T_, RADIX>(eo, d, t, lane, a);
 #pragma unroll
   for (int i = 0; i < T_; ++i) {
     if (i >= t.cnt) break;
@@ -614,7 +777,7 @@ __global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restri
   __shared__ float s_red[W];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int nT = g.nT, M = g.M, ncols = g.nX * g.nY;
-  const Tiles tiles = hm_tiles(dm, wave, W);
+  const Tiles tiles = hm_tiles(dm.R, wave, W);
   const int pitch = gcol_pitch(nT, S);
   float* rows = reinterpret_cast<float*>(glds);
   auto skew = [](int t) { return t + t / S; };

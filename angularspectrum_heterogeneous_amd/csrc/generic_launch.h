@@ -4,12 +4,12 @@
 
 namespace ash {
 
-// Shape of the DFT matrix of a line axis or the column axis of length n (A is null), and
-// the device memory it takes.
+// Shape of the DFT matrix of a line axis or the column axis of length n (A and tw are
+// null), and the device memory it takes.
 DftMat dft_matrix_shape(int n, bool columns);
 size_t dft_matrix_bytes(const DftMat& d);
-// Fills A (dft_matrix_bytes on the device) from the axis' full-length twiddle table.
-void dft_matrix_fill(const DftMat& d, const float2* tw, float4* A, hipStream_t s);
+// Fills A (dft_matrix_bytes on the device) from d.tw, the axis' full-length twiddle table.
+void dft_matrix_fill(const DftMat& d, float4* A, hipStream_t s);
 
 void gen_xfwd(float2* spec, const Geom& g, const DftMat& d, hipStream_t s);
 void gen_xinv(int epi, float2* spec, const Tables& T, const Geom& g, const DftMat& d, const EpiDesc& e, hipStream_t s);

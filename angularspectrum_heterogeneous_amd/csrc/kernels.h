@@ -109,13 +109,15 @@ __device__ __forceinline__ void gst(float2* base, uint32_t off, float2 v) {
 // ---------------------------------------------------------------------------
 // Per-plan constant tables (device memory, built on the host in FP64).
 // ---------------------------------------------------------------------------
-// DFT matrix of an axis outside the FFT set (generic.h): n = length, h = n / 2, `rows`
-// matrix rows in R tiles of 16, Kp matrix columns (multiple of 8) of which the first
-// Ke take the even input positions when n is even (all of them otherwise).  Entry
-// (row tile rt, column group g) starts at A + rt * rs + g * gs.
+// DFT matrix of an axis outside the FFT set (generic.h): length n = p q, p an odd radix
+// taken first (1, 3, 5, 7 or 9), the matrix that of the q-point DFT.  h = q / 2, `rows`
+// matrix rows in R tiles of 16, Kp matrix columns (multiple of 8) of which the first Ke
+// take the even input positions when q is even (all of them otherwise).  Entry (row
+// tile rt, column group g) starts at A + rt * rs + g * gs.
 struct DftMat {
   const float4* A;
-  int n, h, rows, R, Ke, Kp, even;
+  const float2* tw;  // [n] exp(-2 pi i k / n)
+  int n, p, q, h, rows, R, Ke, Kp, even;
   int rs, gs;
 };
 

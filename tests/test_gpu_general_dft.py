@@ -1,7 +1,8 @@
 """The matrix-core DFTs of the general-size kernels at the sizes where their tiling
 can go wrong: the smallest lengths, one position around every 16-row tile and 8-column
 group, even lengths whose quarter is on and off a tile edge, the last length of every
-tiles-per-wave and samples-per-lane class, and the longest lines and columns.
+tiles-per-wave and samples-per-lane class, lengths that take a radix stage first, and
+the longest lines and columns.
 
 Against the FP64 oracle, rel-L2.  A length-n line sums n/2 float32 products per output,
 relative rounding error at most 6e-8 sqrt(n/2) in the root mean square; an operator
@@ -21,7 +22,10 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(2, 3, 4), (3, 2, 5), (15, 16, 7), (17, 31, 15), (32, 33, 31), (30, 34, 32), (62, 63, 33), (66, 65, 62),
           (5, 6, 127), (6, 5, 128), (5, 4, 129), (4, 5, 255), (5, 6, 258), (6, 5, 511), (4, 3, 513), (3, 4, 1022),
           (4, 3, 1025), (3, 4, 1536), (5, 4, 2047), (126, 127, 9), (130, 129, 8), (254, 255, 6), (258, 257, 5),
-          (382, 385, 4), (511, 514, 4), (1000, 3, 16), (3, 1023, 17), (1024, 5, 8), (6, 1022, 8), (1023, 2, 6)]
+          (382, 385, 4), (511, 514, 4), (1000, 3, 16), (3, 1023, 17), (1024, 5, 8), (6, 1022, 8), (1023, 2, 6),
+          # lines that take a radix 3, 5, 7 or 9 first, odd and even quotients
+          (129, 132, 5), (135, 130, 6), (133, 140, 5), (252, 245, 4), (365, 366, 4), (385, 147, 5), (990, 7, 6),
+          (7, 1001, 5), (1008, 4, 6)]
 
 
 @pytest.mark.parametrize("shape", SHAPES)
