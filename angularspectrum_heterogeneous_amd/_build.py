@@ -10,7 +10,8 @@ import tempfile
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libaship.so")
-SOURCES = ["aship.hip", "generic.hip"]
+SOURCES = ["aship.hip", "generic.hip", "generic_columns_short.hip", "generic_columns_8.hip",
+           "generic_columns_16.hip", "generic_columns_32.hip"]
 
 # Packed-FP32 VALU forms are disabled for every HIP translation unit.
 HIPCC_FLAGS = [

@@ -19,7 +19,7 @@
 // W_p^{m r}, so the matrix is that of q and a p-th of the products remain.  The radix
 // stage happens where the tile is folded into LDS; the inverse half of the y pass,
 // whose input lies in the order p k + r, runs it last instead.  At 365 = 5 * 73 an x
-// sweep takes 115 us instead of 211, the y pass 285 instead of 485.
+// sweep takes 116 us instead of 211, the y pass 293 instead of 485.
 //
 // Per element of a complex line that is 2n flops (odd n) or n (even n): at
 // 365x365x425 an x sweep does 20.7 GFLOP over 454 MB, so the matrix cores bound it
@@ -73,7 +73,10 @@ __global__ __launch_bounds__(256) void k_dft_matrix(DftMat d, float4* __restrict
     for (int q = 0; q < 2; ++q) {
       const int j = hm_pos<EVEN>(d, 8 * g + 4 * q + (lane >> 4));
       float2 w = make_float2(0.f, 0.f);
-      if (k < d.rows && j <= d.h) w = d.tw[(int)(((long)j * k) % d.q) * d.p];
+      if (k < d.rows && j <= d.h) {
+        const float4 t = d.tw[(int)(((long)j * k) % d.q) * d.p];
+        w = make_float2(t.x, t.y);
+      }
       v[2 * q] = w.x;
       v[2 * q + 1] = -w.y;
     }
@@ -253,6 +256,14 @@ template <> struct OddTrig<9> {
   static constexpr float ch[] = {0.7660444378852844f, 0.1736481785774231f, -0.5f, -0.9396926164627075f}, cl[] = {5.2336934786012534e-09f, -9.104926812497638e-10f, 2.220446049250313e-16f, -4.323200908373792e-09f};
   static constexpr float sh[] = {0.6427876353263855f, 0.9848077297210693f, 0.8660253882408142f, 0.3420201539993286f}, sl[] = {-2.5639845802061245e-08f, 2.3291137907222037e-08f, 1.5543625053737742e-08f, -1.0673659289750503e-08f};
 };
+// 1/n as a hi/lo pair (rounded to float it would scale every sample by the same error in
+// every visit) and x times such a pair: the low product meets the high one before a
+// rounding, for added to a rounded sum it would be lost
+__device__ __forceinline__ float2 inverse_pair(int n) {
+  const float hi = 1.f / (float)n;
+  return make_float2(hi, fmaf(-hi, (float)n, 1.f) * hi);
+}
+__device__ __forceinline__ float by_pair(float x, float2 w) { return fmaf(x, w.x, x * w.y); }
 // P-point DFT in registers, P odd: with a_m = x_m + x_{P-m}, b_m = x_m - x_{P-m},
 // y_r = x_0 + sum cos(2 pi m r / P) a_m -+ i sum sin(2 pi m r / P) b_m, y_{P-r} its mirror.
 template <int P, bool INV>
@@ -278,10 +289,10 @@ __device__ __forceinline__ void odd_dft(float2* x) {
       if (jj == 0) {
         A = cadd(A, a[m - 1]);
       } else {
-        const float ch = C::ch[jj - 1], cl = C::cl[jj - 1];
-        const float sh = j > H ? -C::sh[jj - 1] : C::sh[jj - 1], sl = j > H ? -C::sl[jj - 1] : C::sl[jj - 1];
-        A = make_float2(fmaf(a[m - 1].x, ch, fmaf(a[m - 1].x, cl, A.x)), fmaf(a[m - 1].y, ch, fmaf(a[m - 1].y, cl, A.y)));
-        B = make_float2(fmaf(b[m - 1].x, sh, fmaf(b[m - 1].x, sl, B.x)), fmaf(b[m - 1].y, sh, fmaf(b[m - 1].y, sl, B.y)));
+        const float2 c = make_float2(C::ch[jj - 1], C::cl[jj - 1]);
+        const float2 s = j > H ? make_float2(-C::sh[jj - 1], -C::sl[jj - 1]) : make_float2(C::sh[jj - 1], C::sl[jj - 1]);
+        A = make_float2(A.x + by_pair(a[m - 1].x, c), A.y + by_pair(a[m - 1].y, c));
+        B = make_float2(B.x + by_pair(b[m - 1].x, s), B.y + by_pair(b[m - 1].y, s));
       }
     }
     const float2 u = make_float2(A.x + B.y, A.y - B.x), v = make_float2(A.x - B.y, A.y + B.x);
@@ -290,14 +301,31 @@ __device__ __forceinline__ void odd_dft(float2* x) {
   }
   x[0] = sum;
 }
-// x_r *= W_n^{s r} (conjugated for the inverse), r = 1 .. P-1; s r < n
+// x times W_n^k (conjugated for the inverse), k < n, with the twiddle as a hi/lo pair: one
+// rounded to float would scale the same element by the same error in every transform of
+// a march, where the entries of the matrix average out over a sum.
+template <bool INV>
+__device__ __forceinline__ float2 cmul_tw(float2 x, float4 w) {
+  if (INV) { w.y = -w.y; w.w = -w.w; }
+  return make_float2(fmaf(x.x, w.x, fmaf(-x.y, w.y, fmaf(x.x, w.z, -x.y * w.w))),
+                     fmaf(x.x, w.y, fmaf(x.y, w.x, fmaf(x.x, w.w, x.y * w.z))));
+}
+// x_r *= W_n^{s r}, r = 1 .. P-1; s r < n.  W_n^{(q-s) r} = W_p^r conj W_n^{s r}: the partner
+// q - s enters its P-point DFT one place further on and takes the conjugate twiddles, so
+// a folded pair reads one set (with two the line kernels hold 133 registers, three
+// waves a SIMD).
 template <int P, bool INV>
-__device__ __forceinline__ void odd_twiddle(float2* x, const float2* tw, int s) {
+__device__ __forceinline__ void odd_twiddle(float2* x, const float4* tw, int s) {
+#pragma unroll
+  for (int r = 1; r < P; ++r) x[r] = cmul_tw<INV>(x[r], tw[s * r]);
+}
+template <int P, bool INV>
+__device__ __forceinline__ void odd_twiddle_pair(float2* x, float2* partner, const float4* tw, int s) {
 #pragma unroll
   for (int r = 1; r < P; ++r) {
-    float2 w = tw[s * r];
-    if (INV) w.y = -w.y;
-    x[r] = cmul(x[r], w);
+    const float4 w = tw[s * r];
+    x[r] = cmul_tw<INV>(x[r], w);
+    partner[r] = cmul_tw<!INV>(partner[r], w);
   }
 }
 
@@ -315,12 +343,11 @@ __device__ __forceinline__ void hm_fold_p(float4* eo, const DftMat& d, int tid, 
 #pragma unroll
     for (int m = 0; m < P; ++m) {
       a[m] = ld(s0 + d.q * m, line);
-      b[m] = ld(s1 + d.q * m, line);
+      b[(m + 1) % P] = ld(s1 + d.q * m, line);
     }
     odd_dft<P, INV>(a);
     odd_dft<P, INV>(b);
-    odd_twiddle<P, INV>(a, d.tw, s0);
-    odd_twiddle<P, INV>(b, d.tw, s1);
+    odd_twiddle_pair<P, INV>(a, b, d.tw, s0);
 #pragma unroll
     for (int r = 0; r < P; ++r) {
       float4 v = make_float4(a[r].x, a[r].y, 0.f, 0.f);
@@ -536,7 +563,7 @@ __global__ __launch_bounds__(512) void k_gy_pass(float2* __restrict__ spec, Tabl
       float2 o;
       if constexpr (PRECISE) o = visit_operator_fp64(op, kk, lc, m);
       else o = visit_operator(op, kk, lc, m);
-      return cmul(v, o);
+      return cmul_tw<false>(v, make_float4(o.x, o.y, d.norm_lo * o.x, d.norm_lo * o.y));
     };
     // folded row of output k of residue r from the values at k and q - k
     auto put = [&](int k, int r, float2 v, float2 vn, bool pair) {
@@ -633,7 +660,7 @@ __global__ __launch_bounds__(512) void k_gy_power(const float2* __restrict__ spe
 // DC/Nyquist projection and an optional phase/amplitude screen.  Tile = (x, 16 f
 // bins); the rows handled (all with a screen, else the two boundary bands) sit in
 // LDS, ysa_rows * 128 bytes of it.
-__global__ __launch_bounds__(256) void k_gy_sa(float2* __restrict__ spec, Tables T, Geom g, ScreenDesc s) {
+static __global__ __launch_bounds__(256) void k_gy_sa(float2* __restrict__ spec, Tables T, Geom g, ScreenDesc s) {
   extern __shared__ float2 sbuf[];
   const int L = g.nY;
   const int tid = threadIdx.x, l = tid & 15;
@@ -696,8 +723,16 @@ __global__ __launch_bounds__(256) void k_gy_sa(float2* __restrict__ spec, Tables
 // change form.  Semantics of the transforms (ASS:664, :685): the inverse ignores the
 // imaginary parts of the DC bin and, for even nT, of the Nyquist bin; the forward
 // writes them as zero.
-// Per sample that is nT flops per transform (odd nT) or nT/2 (even): the matrix cores
-// bound the pass.  The row pitch is an odd multiple of 8 floats: the 16 columns x 4
+// nT = p q with an odd radix p goes through the p residues r of the bin (or the p
+// subsequences of the samples) as the lines do.  Residue 0 is the q-point transform of
+// real samples, residues r and p - r are mirror images, so 1 <= r <= p/2 are complex
+// q-point transforms and the others are not formed.  A row then holds the folded input
+// as float2[Kp] of residue 0 and float4[Kp] of each other, and the inverse's output as
+// q real and p/2 times q complex values before the radix stage.
+// Per sample that is nT flops per transform (odd nT) or nT/2 (even), a p-th of it after a
+// radix stage.  Without one the matrix cores bound the pass (96 TFLOP/s at nT = 1201);
+// with one the vector work between the products does (at 365x365x425 the taper pass
+// takes 374 us, 613 without the radix 5, of which the products are about 80).  The row pitch is an odd multiple of 8 floats: the 16 columns x 4
 // positions of an operand read fall in distinct banks.
 // ---------------------------------------------------------------------------
 constexpr int GC_COLS = 16;
@@ -706,11 +741,16 @@ constexpr int gcol_waves(int S) { return S == 2 ? 4 : 8; }
 constexpr int gcol_tiles(int S, bool even) {
   return ((even ? S + 1 : 2 * S) + gcol_waves(S) - 1) / gcol_waves(S);
 }
-// floats per row: nT/2 + 16 float2 (15 zeros stand under the matrix padding) and
-// nT + nT/S skewed samples
-__host__ __device__ inline int gcol_pitch(int nT, int S) {
-  const int x = 2 * (nT / 2 + 16), u = nT + nT / S + 2;
-  return ((x > u ? x : u) + 7) / 16 * 16 + 8;
+// and with a radix stage (p > 1; p/2 + 1 residues of R tiles), over all lengths that take one
+constexpr int gcol_radix_tiles(int S, bool even) {
+  return S == 32 ? (even ? 3 : 6) : S == 16 ? (even ? 2 : 3) : (even ? 1 : 2);
+}
+// floats per row: nT/2 + 16 float2 (15 zeros stand under the matrix padding; with a radix
+// p Kp float2 and the nT/2 + 1 bins) and nT + nT/S skewed samples
+__host__ __device__ inline int gcol_pitch(const DftMat& d, int S) {
+  const int x = d.p == 1 ? 2 * (d.n / 2 + 16) : 2 * d.p * d.Kp, b = 2 * (d.n / 2 + 1) + 2, u = d.n + d.n / S + 2;
+  const int m = x > b ? x : b;
+  return ((m > u ? m : u) + 7) / 16 * 16 + 8;
 }
 
 template <bool EVEN>
@@ -770,20 +810,277 @@ __device__ __forceinline__ void hm_col_emit(const DftMat& d, const ColAcc<EVEN>&
   }
 }
 
-template <int S, bool EVEN, int MODE, int NLK>
-__global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restrict__ spec, Tables T, Geom g, DftMat dm, ColDesc d) {
-  constexpr int W = gcol_waves(S), TW = gcol_tiles(S, EVEN), NC = GC_COLS / W;
+// --- radix stage of the columns (p = P) -----------------------------------------
+// offset of residue r in the folded row and of its q values before the inverse's radix
+// stage, in floats
+__device__ __forceinline__ int ct_fold_off(const DftMat& d, int r) { return r == 0 ? 0 : (4 * r - 2) * d.Kp; }
+__device__ __forceinline__ int ct_z_off(const DftMat& d, int r) { return r == 0 ? 0 : ((d.q + 1) & ~1) + (r - 1) * 2 * d.q; }
+
+// Bin m (0 <= m < n) of a real column's spectrum: stored up to n/2, mirrored past it.
+__device__ __forceinline__ float2 column_bin(const float2* sc, int m, const Geom& g, int sel, const float2* ref) {
+  const int i = m <= g.M ? m : g.nT - m;
+  float2 x = sc[i];
+  const bool real = i == 0 || i == g.nyq;
+  if (real) x.y = 0.f;
+  x = tof_bin(sel, i, x, g.nyq, ref);
+  if (real) x.y = 0.f;
+  return m <= g.M ? x : cconj(x);
+}
+
+// Spectrum -> folded row, for the inverse.
+template <bool EVEN, int P>
+__device__ __forceinline__ void ct_fold_bins(float* row, const float2* sc, const DftMat& d, const Geom& g, int sel,
+                                             const float2* ref, int lane) {
+  for (int rr = lane; rr < d.Kp; rr += 64) {
+    const int j = hm_pos<EVEN>(d, rr), jj = min(j, d.h);
+    const bool pad = j > d.h, pair = !pad && j > 0 && 2 * j != d.q;
+    float2 x[P / 2 + 1], y[P / 2 + 1];
+    x[0] = column_bin(sc, P * jj, g, sel, ref);
+#pragma unroll
+    for (int r = 1; r <= P / 2; ++r) {
+      x[r] = column_bin(sc, P * jj + r, g, sel, ref);
+      y[r] = column_bin(sc, pair ? P * (d.q - jj) + r : r, g, sel, ref);
+    }
+    const float f = pad ? 0.f : (j == 0 || 2 * P * j == d.n) ? 1.f : 2.f;
+    reinterpret_cast<float2*>(row)[rr] = pad ? make_float2(0.f, 0.f) : cscale(x[0], f);
+#pragma unroll
+    for (int r = 1; r <= P / 2; ++r) {
+      float4 v = make_float4(x[r].x, x[r].y, 0.f, 0.f);
+      if (pair) v = make_float4(x[r].x + y[r].x, x[r].y + y[r].y, x[r].x - y[r].x, x[r].y - y[r].y);
+      if (pad) v = make_float4(0.f, 0.f, 0.f, 0.f);
+      reinterpret_cast<float4*>(row + ct_fold_off(d, r))[rr] = v;
+    }
+  }
+}
+
+// The inverse's radix stage: x_{s + q m} = z_0[s] + 2 Re sum_{r <= P/2} W_P^{-m r} W_n^{-s r}
+// z_r[s], scaled and tapered, from the row's z values to its skewed samples (the wave
+// reads the row whole before it writes).
+template <int S, int P>
+__device__ __forceinline__ void ct_combine(float* row, const DftMat& d, float2 invN, const float* tt, int lane) {
+  using C = OddTrig<P>;
+  constexpr int H = P / 2, NI = (S + P - 1) / P;
+  float v[NI][P];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int s = lane + 64 * i;
+    if (s < d.q) {
+      const float z0 = row[s];
+      float2 y[H];
+      float sum = 0.f;
+#pragma unroll
+      for (int r = 1; r <= H; ++r) {
+        const float2 z = reinterpret_cast<const float2*>(row + ct_z_off(d, r))[s];
+        y[r - 1] = cmul_tw<true>(z, d.tw[s * r]);
+        sum += y[r - 1].x;
+      }
+      v[i][0] = fmaf(2.f, sum, z0);
+#pragma unroll
+      for (int m = 1; m <= H; ++m) {
+        float A = 0.f, B = 0.f;
+#pragma unroll
+        for (int r = 1; r <= H; ++r) {
+          const int j = (m * r) % P, jj = j > H ? P - j : j;
+          if (jj == 0) {
+            A += y[r - 1].x;
+          } else {
+            A += by_pair(y[r - 1].x, make_float2(C::ch[jj - 1], C::cl[jj - 1]));
+            const float b = by_pair(y[r - 1].y, make_float2(C::sh[jj - 1], C::sl[jj - 1]));
+            B += j > H ? -b : b;
+          }
+        }
+        v[i][m] = fmaf(2.f, A - B, z0);
+        v[i][P - m] = fmaf(2.f, A + B, z0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // one round's temporaries at a time
+  }
+  wave_sync();
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int s = lane + 64 * i;
+    if (s < d.q) {
+#pragma unroll
+      for (int m = 0; m < P; ++m) {
+        const int t = s + d.q * m;
+        float x = by_pair(v[i][m], invN);
+        if (tt) x *= tt[t];
+        row[t + t / S] = x;
+      }
+    }
+  }
+}
+
+// Samples -> folded row, for the forward transform: y_r[s] = W_n^{s r} sum_m u_{s + q m}
+// W_P^{m r}, r <= P/2, folded over s and q - s; this is the sum over m.
+template <int P>
+__device__ __forceinline__ void ct_sample_dft(const float* u, float2* y) {
+  using C = OddTrig<P>;
+  constexpr int H = P / 2;
+  float a[H], b[H], sum = u[0];
+#pragma unroll
+  for (int m = 1; m <= H; ++m) {
+    a[m - 1] = u[m] + u[P - m];
+    b[m - 1] = u[m] - u[P - m];
+    sum += a[m - 1];
+  }
+  y[0] = make_float2(sum, 0.f);
+#pragma unroll
+  for (int r = 1; r <= H; ++r) {
+    float A = u[0], B = 0.f;
+#pragma unroll
+    for (int m = 1; m <= H; ++m) {
+      const int j = (m * r) % P, jj = j > H ? P - j : j;
+      if (jj == 0) {
+        A += a[m - 1];
+      } else {
+        A += by_pair(a[m - 1], make_float2(C::ch[jj - 1], C::cl[jj - 1]));
+        const float w = by_pair(b[m - 1], make_float2(C::sh[jj - 1], C::sl[jj - 1]));
+        B += j > H ? -w : w;
+      }
+    }
+    y[r] = make_float2(A, -B);
+  }
+}
+// rounds of 64 matrix columns of a q-point transform, q <= 64 S / P
+constexpr int ct_rounds(int S, int P) {
+  int most = 0;
+  for (int q = 64 * S / P - 1; q <= 64 * S / P; ++q) {
+    const int h = q / 2;
+    const int kp = q % 2 ? (h + 8) / 8 * 8 : (h / 2 + 8) / 8 * 8 + ((h + 1) / 2 + 7) / 8 * 8;
+    if (kp > most) most = kp;
+  }
+  return (most + 63) / 64;
+}
+template <int S, bool EVEN, int P>
+__device__ __forceinline__ void ct_fold_samples(float* row, const DftMat& d, int lane) {
+  constexpr int H = P / 2, NF = ct_rounds(S, P);
+  float2 e0[NF];  // residue 0
+  float4 v[NF][H];
+#pragma unroll
+  for (int i = 0; i < NF; ++i) {
+    const int rr = lane + 64 * i;
+    if (rr < d.Kp) {
+      const int j = hm_pos<EVEN>(d, rr), jj = min(j, d.h);
+      const bool pad = j > d.h, pair = !pad && j > 0 && 2 * j != d.q;
+      const int s1 = pair ? d.q - jj : jj;
+      float a[P], b[P];
+#pragma unroll
+      for (int m = 0; m < P; ++m) {
+        const int t0 = jj + d.q * m, t1 = s1 + d.q * m;
+        a[m] = row[t0 + t0 / S];
+        b[(m + 1) % P] = row[t1 + t1 / S];
+      }
+      float2 x[H + 1], y[H + 1];
+      ct_sample_dft<P>(a, x);
+      ct_sample_dft<P>(b, y);
+#pragma unroll
+      for (int r = 1; r <= H; ++r) {
+        const float4 w = d.tw[jj * r];
+        x[r] = cmul_tw<false>(x[r], w);
+        y[r] = cmul_tw<true>(y[r], w);
+      }
+      e0[i] = make_float2(pad ? 0.f : pair ? x[0].x + y[0].x : x[0].x, pair ? x[0].x - y[0].x : 0.f);
+#pragma unroll
+      for (int r = 1; r <= H; ++r) {
+        float4 w = make_float4(x[r].x, x[r].y, 0.f, 0.f);
+        if (pair) w = make_float4(x[r].x + y[r].x, x[r].y + y[r].y, x[r].x - y[r].x, x[r].y - y[r].y);
+        if (pad) w = make_float4(0.f, 0.f, 0.f, 0.f);
+        v[i][r - 1] = w;
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // one round's temporaries at a time
+  }
+  wave_sync();
+#pragma unroll
+  for (int i = 0; i < NF; ++i) {
+    const int rr = lane + 64 * i;
+    if (rr < d.Kp) {
+      reinterpret_cast<float2*>(row)[rr] = e0[i];
+#pragma unroll
+      for (int r = 1; r <= H; ++r) reinterpret_cast<float4*>(row + ct_fold_off(d, r))[rr] = v[i][r - 1];
+    }
+  }
+}
+
+// One row tile of residue r of the folded column `row`.
+template <bool EVEN>
+__device__ __forceinline__ void ct_tile(const DftMat& d, int r, int rt, int lane, const float* row, LineAcc<EVEN>& a) {
+  constexpr int U = 4;
+#pragma unroll
+  for (int p = 0; p < LineAcc<EVEN>::NP; ++p) {
+    const int gp = p == 0 ? 0 : d.Ke / 8, ng = (p == 0 ? d.Ke : d.Kp - d.Ke) / 8;
+    const float4* ap = d.A + (long)rt * d.rs + gp * d.gs + lane;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) a.c[p][q] = a.s[p][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float4 w[U];
+    if (r == 0) {
+      const float2* bp = reinterpret_cast<const float2*>(row) + gp * 8 + (lane >> 4);
+      float2 b[U][2];
+      hm_ring<U>(
+          ng,
+          [&](int q, int g) {
+            w[q] = ap[g * d.gs];
+            b[q][0] = bp[g * 8];
+            b[q][1] = bp[g * 8 + 4];
+          },
+          [&](int q) {
+            a.c[p][0] = mfma4(w[q].x, b[q][0].x, a.c[p][0]);
+            a.s[p][0] = mfma4(w[q].y, b[q][0].y, a.s[p][0]);
+            a.c[p][0] = mfma4(w[q].z, b[q][1].x, a.c[p][0]);
+            a.s[p][0] = mfma4(w[q].w, b[q][1].y, a.s[p][0]);
+          });
+    } else {
+      const float4* bp = reinterpret_cast<const float4*>(row + ct_fold_off(d, r)) + gp * 8 + (lane >> 4);
+      float4 b[U][2];
+      hm_ring<U>(
+          ng,
+          [&](int q, int g) {
+            w[q] = ap[g * d.gs];
+            b[q][0] = bp[g * 8];
+            b[q][1] = bp[g * 8 + 4];
+          },
+          [&](int q) {
+            a.c[p][0] = mfma4(w[q].x, b[q][0].x, a.c[p][0]);
+            a.c[p][1] = mfma4(w[q].x, b[q][0].y, a.c[p][1]);
+            a.s[p][0] = mfma4(w[q].y, b[q][0].z, a.s[p][0]);
+            a.s[p][1] = mfma4(w[q].y, b[q][0].w, a.s[p][1]);
+            a.c[p][0] = mfma4(w[q].z, b[q][1].x, a.c[p][0]);
+            a.c[p][1] = mfma4(w[q].z, b[q][1].y, a.c[p][1]);
+            a.s[p][0] = mfma4(w[q].w, b[q][1].z, a.s[p][0]);
+            a.s[p][1] = mfma4(w[q].w, b[q][1].w, a.s[p][1]);
+          });
+    }
+  }
+}
+
+// CALL with P = d.p
+#define CT_DISPATCH(d, CALL)                        \
+  switch ((d).p) {                                  \
+    case 3: { constexpr int P = 3; CALL; } break;   \
+    case 5: { constexpr int P = 5; CALL; } break;   \
+    case 7: { constexpr int P = 7; CALL; } break;   \
+    default: { constexpr int P = 9; CALL; } break;  \
+  }
+
+// two blocks per CU and more for up to 1024 samples (four waves per SIMD); the FP64 tone
+// burst and the longest rows take what they need
+constexpr int gcol_waves_per_simd(int S, bool radix, int mode) { return radix && S <= 16 && mode != COL_INJECT && mode != COL_TOF ? 4 : 1; }
+
+template <int S, bool EVEN, bool RADIX, int MODE, int NLK>
+__global__ __launch_bounds__(64 * gcol_waves(S), gcol_waves_per_simd(S, RADIX, MODE)) void k_gcolumn(float2* __restrict__ spec, Tables T, Geom g, DftMat dm, ColDesc d) {
+  constexpr int W = gcol_waves(S), TW = RADIX ? gcol_radix_tiles(S, EVEN) : gcol_tiles(S, EVEN), NC = GC_COLS / W;
   extern __shared__ float4 glds[];
   __shared__ float s_red[W];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int nT = g.nT, M = g.M, ncols = g.nX * g.nY;
-  const Tiles tiles = hm_tiles(dm.R, wave, W);
-  const int pitch = gcol_pitch(nT, S);
+  const Tiles tiles = hm_tiles(RADIX ? (dm.p / 2 + 1) * dm.R : dm.R, wave, W);
+  const int pitch = gcol_pitch(dm, S);
   float* rows = reinterpret_cast<float*>(glds);
   auto skew = [](int t) { return t + t / S; };
   const int c0 = blockIdx.x * GC_COLS;
   const int t0 = lane * S;
-  const float invN = 1.f / (float)nT;
+  const float2 invN = inverse_pair(nT);
   constexpr bool spectral_in = MODE != COL_LOAD && MODE != COL_INJECT;
   constexpr bool rewrite = (MODE == COL_NL || MODE == COL_TAPER || MODE == COL_LOAD || MODE == COL_INJECT);
   constexpr bool FIN = MODE == COL_FINAL;
@@ -810,6 +1107,10 @@ __global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restri
       const int col = wave * NC + i, c = c0 + col;
       if (c < ncols) {
         const float2* sc = spec + (long)c * g.MP;
+        if constexpr (RADIX) {
+          CT_DISPATCH(dm, (ct_fold_bins<EVEN, P>(rows + col * pitch, sc, dm, g, sel, d.tofref, lane)));
+          continue;
+        }
         float2* X = reinterpret_cast<float2*>(rows + col * pitch);
 #pragma unroll 4
         for (int m = lane; m < M + 16; m += 64) {
@@ -824,20 +1125,45 @@ __global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restri
       }
     }
     __syncthreads();
-    ColAcc<EVEN> a[TW];
-    const float2* xc = reinterpret_cast<const float2*>(rows + (lane & 15) * pitch);
-    hm_col<EVEN, TW>(dm, tiles, lane, xc, a);
-    __syncthreads();
     float* uc = rows + (lane & 15) * pitch;
+    if constexpr (RADIX) {
+      LineAcc<EVEN> a[TW];
 #pragma unroll
-    for (int i = 0; i < TW; ++i)
+      for (int i = 0; i < TW; ++i)
+        if (i < tiles.cnt) {
+          const int r = (tiles.lo + i) / dm.R;
+          ct_tile<EVEN>(dm, r, tiles.lo + i - r * dm.R, lane, uc, a[i]);
+        }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < TW; ++i)
+        if (i < tiles.cnt) {
+          const int r = (tiles.lo + i) / dm.R;
+          float* z = uc + ct_z_off(dm, r);
+          hm_emit_at<EVEN, true>(dm, a[i], tiles.lo + i, lane, [](int k, int) { return k; }, [&](int k, float2 v) {
+            if (r == 0) z[k] = v.x - v.y;
+            else reinterpret_cast<float2*>(z)[k] = v;
+          });
+        }
+      __syncthreads();
+#pragma unroll 1
+      for (int i = 0; i < NC; ++i)
+        CT_DISPATCH(dm, (ct_combine<S, P>(rows + (wave * NC + i) * pitch, dm, invN, tapered ? tt : nullptr, lane)));
+      wave_sync();  // (each wave reads on only its own columns)
+      return;
+    }
+    ColAcc<EVEN> a[RADIX ? 1 : TW];
+    if constexpr (!RADIX) hm_col<EVEN, TW>(dm, tiles, lane, reinterpret_cast<const float2*>(uc), a);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < (RADIX ? 0 : TW); ++i)
       if (i < tiles.cnt)
         hm_col_emit<EVEN>(dm, a[i], tiles.lo + i, lane, [&](int t, float C, float Sn) {
-          float v = (C - Sn) * invN;
+          float v = by_pair(C - Sn, invN);
           if (tapered && tt) v *= tt[t];
           uc[skew(t)] = v;
           if (t > 0 && 2 * t != nT) {
-            float w = (C + Sn) * invN;
+            float w = by_pair(C + Sn, invN);
             if (tapered && tt) w *= tt[nT - t];
             uc[skew(nT - t)] = w;
           }
@@ -926,7 +1252,9 @@ __global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restri
           wave_sync();
         }
       }
-      if constexpr (rewrite) {
+      if constexpr (rewrite && RADIX) {
+        CT_DISPATCH(dm, (ct_fold_samples<S, EVEN, P>(uc, dm, lane)));
+      } else if constexpr (rewrite) {
         // U -> E (the row is read whole before it is written)
         constexpr int NF = S / 2 + 1;  // positions 0 .. M + 15 <= 32 S + 15, 64 per round
         float2 e[NF];
@@ -950,17 +1278,37 @@ __global__ __launch_bounds__(64 * gcol_waves(S)) void k_gcolumn(float2* __restri
     }
     if constexpr (rewrite) {
       __syncthreads();
-      ColAcc<EVEN> a[TW];
-      const float2* ec = reinterpret_cast<const float2*>(rows + (lane & 15) * pitch);
-      hm_col<EVEN, TW>(dm, tiles, lane, ec, a);
-      __syncthreads();
-      float2* xc = reinterpret_cast<float2*>(rows + (lane & 15) * pitch);
+      float* ec = rows + (lane & 15) * pitch;
+      float2* xc = reinterpret_cast<float2*>(ec);
+      if constexpr (RADIX) {
+        LineAcc<EVEN> a[TW];
 #pragma unroll
-      for (int i = 0; i < TW; ++i)
-        if (i < tiles.cnt)
-          hm_col_emit<EVEN>(dm, a[i], tiles.lo + i, lane, [&](int m, float C, float Sn) {
-            xc[m] = make_float2(C, (m == 0 || m == g.nyq) ? 0.f : -Sn);
-          });
+        for (int i = 0; i < TW; ++i)
+          if (i < tiles.cnt) {
+            const int r = (tiles.lo + i) / dm.R;
+            ct_tile<EVEN>(dm, r, tiles.lo + i - r * dm.R, lane, ec, a[i]);
+          }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TW; ++i)
+          if (i < tiles.cnt)
+            hm_emit<EVEN, false>(dm, a[i], tiles.lo + i, lane, [&](int m, float2 v) {
+              // (past nT/2: the mirrored bin, of another residue; residue 0 forms it itself)
+              if (m == 0 || m == g.nyq) v.y = 0.f;
+              if (m <= M) xc[m] = v;
+              else if (tiles.lo + i >= dm.R) xc[nT - m] = cconj(v);
+            });
+      } else {
+        ColAcc<EVEN> a[TW];
+        hm_col<EVEN, TW>(dm, tiles, lane, xc, a);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TW; ++i)
+          if (i < tiles.cnt)
+            hm_col_emit<EVEN>(dm, a[i], tiles.lo + i, lane, [&](int m, float C, float Sn) {
+              xc[m] = make_float2(C, (m == 0 || m == g.nyq) ? 0.f : -Sn);
+            });
+      }
       __syncthreads();
 #pragma unroll
       for (int i = 0; i < NC; ++i) {

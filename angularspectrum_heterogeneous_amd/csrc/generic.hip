@@ -34,15 +34,19 @@ size_t line_lds(const DftMat& d) { return (size_t)d.p * d.Kp * 16 * sizeof(float
 
 DftMat dft_matrix_shape(int n, bool columns) {
   DftMat d = matrix_of(n, 1);
-  if (!columns && n >= 128) {
-    // the radix that leaves the fewest products, if that is at most 0.6 of them (shorter
-    // lines are bound by memory already, and a small gain is lost to the radix stage)
+  if (n > (columns ? 256 : 128)) {
+    // the radix that leaves the fewest products, if that is at most 0.6 of them (a small
+    // gain is lost to the radix stage).  Shorter lines are bound by memory already;
+    // shorter columns by the launch and the stages between the products: the KT pass at
+    // 64x64x189 takes 15.5 us without a radix and 17.4 with one, at 128x128x300 56.6 and
+    // 47.6, at 128x128x801 257 and 105, at 128x128x1995 1254 and 449.
     auto products = [](const DftMat& m) { return m.p * m.R * m.Kp; };
     DftMat best = d;
     for (int p : {3, 5, 7, 9}) {
       if (n % p) continue;
       const DftMat m = matrix_of(n, p);
-      if (products(m) < products(best) && line_tiles(m) <= (m.even ? 3 : 4) && line_lds(m) <= 160 * 1024) best = m;
+      const bool fits = columns || (line_tiles(m) <= (m.even ? 3 : 4) && line_lds(m) <= 160 * 1024);
+      if (products(m) < products(best) && fits) best = m;
     }
     if (10 * products(best) <= 6 * products(d)) d = best;
   }
@@ -121,57 +125,13 @@ void gen_ysa(float2* spec, const Tables& T, const Geom& g, const ScreenDesc& sd,
 
 int gen_column_blocks(int ncols) { return (ncols + GC_COLS - 1) / GC_COLS; }
 
-namespace {
-
-template <int S, int MODE, int NLK>
-void launch_gcol_SMN(float2* spec, const Tables& T, const Geom& g, const DftMat& d, const ColDesc& cd, hipStream_t s) {
-  const dim3 grid(gen_column_blocks(g.nX * g.nY)), block(64 * gcol_waves(S));
-  const size_t lds = (size_t)GC_COLS * gcol_pitch(g.nT, S) * sizeof(float);
-  if (d.even) hipLaunchKernelGGL((k_gcolumn<S, true, MODE, NLK>), grid, block, lds, s, spec, T, g, d, cd);
-  else hipLaunchKernelGGL((k_gcolumn<S, false, MODE, NLK>), grid, block, lds, s, spec, T, g, d, cd);
-}
-template <int S, int NLK>
-void launch_graw(const Tables& T, const Geom& g, const ColDesc& cd, hipStream_t s) {
-  const int blocks = std::min((g.nX * g.nY + GR_WPB - 1) / GR_WPB, 2048);
-  hipLaunchKernelGGL((k_gcolumn_raw<S, NLK>), dim3(blocks), dim3(64 * GR_WPB), 0, s, T, g, cd);
-}
-template <int S>
-void launch_gcol_S(float2* spec, const Tables& T, const Geom& g, const DftMat& d, const ColDesc& cd, hipStream_t s) {
-  switch (cd.mode) {
-    case COL_LOAD: launch_gcol_SMN<S, COL_LOAD, NL_NONE>(spec, T, g, d, cd, s); break;
-    case COL_NL:  // (the march's updates; KT_MINMOD is an operator of its own)
-      if (cd.nl == NL_KT) launch_gcol_SMN<S, COL_NL, NL_KT>(spec, T, g, d, cd, s);
-      else if (cd.nl == NL_TVD) launch_gcol_SMN<S, COL_NL, NL_TVD>(spec, T, g, d, cd, s);
-      else launch_gcol_SMN<S, COL_NL, NL_RUSANOV>(spec, T, g, d, cd, s);
-      break;
-    case COL_TAPER: launch_gcol_SMN<S, COL_TAPER, NL_NONE>(spec, T, g, d, cd, s); break;
-    case COL_FINAL: launch_gcol_SMN<S, COL_FINAL, NL_NONE>(spec, T, g, d, cd, s); break;
-    case COL_INJECT: launch_gcol_SMN<S, COL_INJECT, NL_NONE>(spec, T, g, d, cd, s); break;
-    case COL_STORE: launch_gcol_SMN<S, COL_STORE, NL_NONE>(spec, T, g, d, cd, s); break;
-    case COL_RAWNL:
-      switch (cd.nl) {
-        case NL_KT: launch_graw<S, NL_KT>(T, g, cd, s); break;
-        case NL_KT_MINMOD: launch_graw<S, NL_KT_MINMOD>(T, g, cd, s); break;
-        case NL_RUSANOV: launch_graw<S, NL_RUSANOV>(T, g, cd, s); break;
-        case NL_TVD: launch_graw<S, NL_TVD>(T, g, cd, s); break;
-        default: launch_graw<S, NL_NONE>(T, g, cd, s); break;
-      }
-      break;
-    case COL_MAXABS: launch_gcol_SMN<S, COL_MAXABS, NL_NONE>(spec, T, g, d, cd, s); break;
-    case COL_TOF: launch_gcol_SMN<S, COL_TOF, NL_NONE>(spec, T, g, d, cd, s); break;
-    default: break;
-  }
-}
-
-}  // namespace
-
 void gen_column(float2* spec, const Tables& T, const Geom& g, const DftMat& d, const ColDesc& cd, hipStream_t s) {
   // S real samples per lane, 64 S >= nT
-  if (g.nT <= 128) launch_gcol_S<2>(spec, T, g, d, cd, s);
-  else if (g.nT <= 256) launch_gcol_S<4>(spec, T, g, d, cd, s);
-  else if (g.nT <= 512) launch_gcol_S<8>(spec, T, g, d, cd, s);
-  else if (g.nT <= 1024) launch_gcol_S<16>(spec, T, g, d, cd, s);
-  else launch_gcol_S<32>(spec, T, g, d, cd, s);
+  if (g.nT <= 128) gen_column_S<2>(spec, T, g, d, cd, s);
+  else if (g.nT <= 256) gen_column_S<4>(spec, T, g, d, cd, s);
+  else if (g.nT <= 512) gen_column_S<8>(spec, T, g, d, cd, s);
+  else if (g.nT <= 1024) gen_column_S<16>(spec, T, g, d, cd, s);
+  else gen_column_S<32>(spec, T, g, d, cd, s);
 }
 
 }  // namespace ash

@@ -19,5 +19,7 @@ void gen_ysa(float2* spec, const Tables& T, const Geom& g, const ScreenDesc& sd,
 // Column pass cd.mode on nT outside the FFT set; its blocks (one partial each for COL_MAXABS).
 void gen_column(float2* spec, const Tables& T, const Geom& g, const DftMat& d, const ColDesc& cd, hipStream_t s);
 int gen_column_blocks(int ncols);
+template <int S>
+void gen_column_S(float2* spec, const Tables& T, const Geom& g, const DftMat& d, const ColDesc& cd, hipStream_t s);
 
 }  // namespace ash

@@ -116,9 +116,10 @@ __device__ __forceinline__ void gst(float2* base, uint32_t off, float2 v) {
 // tile rt, column group g) starts at A + rt * rs + g * gs.
 struct DftMat {
   const float4* A;
-  const float2* tw;  // [n] exp(-2 pi i k / n)
+  const float4* tw;  // [n] exp(-2 pi i k / n): (x, y) rounded to float32, and what that left out
   int n, p, q, h, rows, R, Ke, Kp, even;
   int rs, gs;
+  float norm_lo;  // y axis: what float32 left out of the visits' 1/(nX nY), relative
 };
 
 struct Tables {

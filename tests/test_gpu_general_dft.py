@@ -25,7 +25,11 @@ SHAPES = [(2, 3, 4), (3, 2, 5), (15, 16, 7), (17, 31, 15), (32, 33, 31), (30, 34
           (382, 385, 4), (511, 514, 4), (1000, 3, 16), (3, 1023, 17), (1024, 5, 8), (6, 1022, 8), (1023, 2, 6),
           # lines that take a radix 3, 5, 7 or 9 first, odd and even quotients
           (129, 132, 5), (135, 130, 6), (133, 140, 5), (252, 245, 4), (365, 366, 4), (385, 147, 5), (990, 7, 6),
-          (7, 1001, 5), (1008, 4, 6)]
+          (7, 1001, 5), (1008, 4, 6),
+          # and columns (with 16 columns to a block, some blocks partly filled)
+          (5, 4, 129), (4, 5, 130), (3, 7, 133), (5, 5, 135), (6, 5, 189), (7, 5, 252), (5, 7, 300), (4, 5, 301),
+          (5, 9, 425), (4, 4, 510), (3, 5, 513), (5, 4, 801), (4, 5, 1010), (3, 6, 1022), (5, 4, 1035), (4, 5, 1200),
+          (3, 7, 1995), (4, 4, 2043), (5, 4, 2044), (4, 5, 2045), (3, 4, 2046)]
 
 
 @pytest.mark.parametrize("shape", SHAPES)
