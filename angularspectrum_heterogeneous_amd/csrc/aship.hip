@@ -544,8 +544,8 @@ struct ProfScope {
 template <int L>
 void launch_xfwd_L(ash_plan* p, hipStream_t s) {
   const dim3 grid(p->g.nY * p->g.nfb);
-  if (p->rvx) hipLaunchKernelGGL((k_xfft_fwd<L, 1>), grid, dim3(LNT), 0, s, p->spec, p->T, p->g);
-  else hipLaunchKernelGGL((k_xfft_fwd<L, 0>), grid, dim3(LNT), 0, s, p->spec, p->T, p->g);
+  if (p->rvx) hipLaunchKernelGGL((k_xfft_fwd<L, 1>), grid, dim3(xline_threads<L>()), 0, s, p->spec, p->T, p->g);
+  else hipLaunchKernelGGL((k_xfft_fwd<L, 0>), grid, dim3(xline_threads<L>()), 0, s, p->spec, p->T, p->g);
 }
 template <int L>
 void launch_ypass_L(ash_plan* p, const OpDesc& op, hipStream_t s) {
@@ -558,8 +558,8 @@ void launch_ypass_L(ash_plan* p, const OpDesc& op, hipStream_t s) {
 template <int L, int EPI>
 void launch_xinv_L(ash_plan* p, const EpiDesc& e, hipStream_t s) {
   const dim3 grid(p->g.nY * p->g.nfb);
-  if (p->rvx) hipLaunchKernelGGL((k_xfft_inv<L, EPI, 1>), grid, dim3(LNT), 0, s, p->spec, p->T, p->g, e);
-  else hipLaunchKernelGGL((k_xfft_inv<L, EPI, 0>), grid, dim3(LNT), 0, s, p->spec, p->T, p->g, e);
+  if (p->rvx) hipLaunchKernelGGL((k_xfft_inv<L, EPI, 1>), grid, dim3(xline_threads<L>()), 0, s, p->spec, p->T, p->g, e);
+  else hipLaunchKernelGGL((k_xfft_inv<L, EPI, 0>), grid, dim3(xline_threads<L>()), 0, s, p->spec, p->T, p->g, e);
 }
 template <int L>
 void launch_ysa_L(ash_plan* p, const ScreenDesc& sd, hipStream_t s) {

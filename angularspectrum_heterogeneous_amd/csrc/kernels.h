@@ -305,11 +305,17 @@ __device__ __forceinline__ float2 visit_operator(const OpDesc& op, double kk, co
   return make_float2(amp * c, amp * s);
 }
 
+// threads of an x-sweep block: 512 at 384 points, whose tiles hold a CU to three blocks
+// (384x384x1024: forward 264 -> 249 us, inverse 289 -> 265; 384 threads gain nothing,
+// 640 to 1024 nothing more)
+template <int L> constexpr int xline_threads() { return L == 384 ? 512 : LNT; }
+
 // ---------------------------------------------------------------------------
 // x-sweep, forward FFT along x.  Tile = (y, f-block).
 // ---------------------------------------------------------------------------
 template <int L, int V>
-__global__ __launch_bounds__(LNT) void k_xfft_fwd(float2* __restrict__ spec, Tables T, Geom g) {
+__global__ __launch_bounds__((xline_threads<L>())) void k_xfft_fwd(float2* __restrict__ spec, Tables T, Geom g) {
+  constexpr int NTX = xline_threads<L>();
   __shared__ float2 tw[L];
   __shared__ float2 buf[L * LF];
   const int tid = threadIdx.x;
@@ -318,7 +324,7 @@ __global__ __launch_bounds__(LNT) void k_xfft_fwd(float2* __restrict__ spec, Tab
   const uint32_t sxb = (uint32_t)g.nY * g.MP * 8u;  // x stride in bytes
   float2* base = spec + (long)y * g.MP + f0;
   const int nvalid = min(LF, g.M + 1 - f0);
-  load_tw<L>(tw, T.twx, tid, LNT);
+  load_tw<L>(tw, T.twx, tid, NTX);
   __syncthreads();
   using LY = Lay<L, LF, 0, true>;
   auto ld = [&](int line, int pos) -> float2 {
@@ -327,16 +333,17 @@ __global__ __launch_bounds__(LNT) void k_xfft_fwd(float2* __restrict__ spec, Tab
   auto st = [&](int line, int pos, float2 v) {
     if (line < nvalid) gst(base, pos * sxb + line * 8u, v);
   };
-  fft_run<L, false, LNT, LF, LY, V>(buf, tw, tid, ld, st);
+  fft_run<L, false, NTX, LF, LY, V>(buf, tw, tid, ld, st);
 }
 
 // f bins per y-pass tile: 8 for the 384-point line, whose 16-bin tile (78 KB of
 // LDS with the operator table) would hold the CU to two blocks
 template <int L> constexpr int ypass_lines() { return L == 384 ? 8 : LF; }
 // threads of a y-pass block: 512 for the 256-point 8*8*4 order, whose every pass
-// has 512 or more butterflies per tile (twice the waves per CU in the same LDS),
-// else LNT
-template <int L, int V> constexpr int ypass_threads() { return (L == 256 && V == 1) ? 512 : LNT; }
+// has 512 or more butterflies per tile (twice the waves per CU in the same LDS), and
+// for the 384-point line (384x384x1024: 332 -> 306 us; 192 and 384 threads 348 and 381;
+// 16-bin tiles 338 at best), else LNT
+template <int L, int V> constexpr int ypass_threads() { return (L == 256 && V == 1) || L == 384 ? 512 : LNT; }
 
 // ---------------------------------------------------------------------------
 // y-pass: forward FFT along y, multiply by the visit operator, inverse FFT.
@@ -467,7 +474,8 @@ struct EpiDesc {
 };
 
 template <int L, int EPI, int V>
-__global__ __launch_bounds__(LNT) void k_xfft_inv(float2* __restrict__ spec, Tables T, Geom g, EpiDesc e) {
+__global__ __launch_bounds__((xline_threads<L>())) void k_xfft_inv(float2* __restrict__ spec, Tables T, Geom g, EpiDesc e) {
+  constexpr int NTX = xline_threads<L>();
   __shared__ float2 tw[L];
   __shared__ float2 buf[L * LF];
   const int tid = threadIdx.x;
@@ -476,7 +484,7 @@ __global__ __launch_bounds__(LNT) void k_xfft_inv(float2* __restrict__ spec, Tab
   const uint32_t sxb = (uint32_t)g.nY * g.MP * 8u;  // x stride in bytes
   float2* base = spec + (long)y * g.MP + f0;
   const int nvalid = min(LF, g.M + 1 - f0);
-  load_tw<L>(tw, T.twx, tid, LNT);
+  load_tw<L>(tw, T.twx, tid, NTX);
   __syncthreads();
   using LY = Lay<L, LF, 0, true>;
   auto ld = [&](int line, int pos) -> float2 {
@@ -494,13 +502,13 @@ __global__ __launch_bounds__(LNT) void k_xfft_inv(float2* __restrict__ spec, Tab
     // butterflies of that pass), so the stores wait on no load
     using PL = PassR<L, Radix<L, V>::NP - 1, true, V>;
     constexpr int RL = PL::R, NBL = PL::NB, TOTL = NBL * LF;
-    constexpr bool TPRE = EPI == 1 && TOTL % LNT == 0;
-    float tf[TPRE ? (TOTL / LNT) * RL : 1];
+    constexpr bool TPRE = EPI == 1 && TOTL % NTX == 0;
+    float tf[TPRE ? (TOTL / NTX) * RL : 1];
     if constexpr (TPRE) {
 #pragma unroll
-      for (int q = 0; q < TOTL / LNT; ++q) {
+      for (int q = 0; q < TOTL / NTX; ++q) {
         int line, j;
-        LY::template map<NBL>(tid + q * LNT, line, j);
+        LY::template map<NBL>(tid + q * NTX, line, j);
 #pragma unroll
         for (int r = 0; r < RL; ++r) tf[q * RL + r] = tx[out_pos<L, Radix<L, V>::NP - 1, true, V>(j, r)] * ty;
       }
@@ -511,7 +519,7 @@ __global__ __launch_bounds__(LNT) void k_xfft_inv(float2* __restrict__ spec, Tab
       else if constexpr (EPI == 1) v = cscale(v, tx[pos] * ty);
       if (line < nvalid) gst(base, pos * sxb + line * 8u, v);
     };
-    fft_run<L, true, LNT, LF, LY, V>(buf, tw, tid, ld, st);
+    fft_run<L, true, NTX, LF, LY, V>(buf, tw, tid, ld, st);
   } else {
     // the inverse transform's last pass stores into LDS with the scale, the
     // DC/Nyquist projection and the frequency-weighted mask already applied,
@@ -522,7 +530,7 @@ __global__ __launch_bounds__(LNT) void k_xfft_inv(float2* __restrict__ spec, Tab
     __shared__ float slgx[TLDS ? L : 1], swx[TLDS ? L : 1];
     __shared__ float sfwe[LF];
     if constexpr (TLDS) {
-      for (int i = tid; i < L; i += LNT) {
+      for (int i = tid; i < L; i += NTX) {
         slgx[i] = T.lgx[i];
         swx[i] = T.sa_wx[i];
       }
@@ -539,17 +547,17 @@ __global__ __launch_bounds__(LNT) void k_xfft_inv(float2* __restrict__ spec, Tab
       if (e.fw) v = cscale(v, exp2f(sfwe[line] * (lgx[pos] + lgy)));
       buf[LY::idx(line, pos)] = v;
     };
-    fft_run<L, true, LNT, LF, LY, V>(buf, tw, tid, ld, st_lds);
+    fft_run<L, true, NTX, LF, LY, V>(buf, tw, tid, ld, st_lds);
     __syncthreads();
     // element e -> (line, pos), line fastest: coalesced 128-byte rows; the
-    // line of a thread is fixed (LNT is a multiple of LF)
-    constexpr int PER = (L * LF) / LNT;
+    // line of a thread is fixed (NTX is a multiple of LF)
+    constexpr int PER = (L * LF) / NTX;
     const int line = tid % LF;
     const float cw = T.sa_cw[min(f0 + line, g.MP - 1)];
     float2 res[PER];
 #pragma unroll
     for (int q = 0; q < PER; ++q) {
-      const int pos = (tid + q * LNT) / LF;
+      const int pos = (tid + q * NTX) / LF;
       float2 v = buf[LY::idx(line, pos)];
       if (e.sa) {
         const float w = wx[pos];
@@ -568,7 +576,7 @@ __global__ __launch_bounds__(LNT) void k_xfft_inv(float2* __restrict__ spec, Tab
     }
     if (line < nvalid) {
 #pragma unroll
-      for (int q = 0; q < PER; ++q) gst(base, ((tid + q * LNT) / LF) * sxb + line * 8u, res[q]);
+      for (int q = 0; q < PER; ++q) gst(base, ((tid + q * NTX) / LF) * sxb + line * 8u, res[q]);
     }
   }
 }
