@@ -357,8 +357,10 @@ __device__ __forceinline__ void hm_fold_p(float4* eo, const DftMat& d, int tid, 
     }
   }
 }
-template <bool EVEN, bool INV, bool RADIX, class Ld>
-__device__ __forceinline__ void hm_fold(float4* eo, const DftMat& d, int tid, int nthr, Ld ld) {
+// (`between` runs once, while the first rows' loads are in flight, when there is no radix)
+struct HmNothing { __device__ void operator()() const {} };
+template <bool EVEN, bool INV, bool RADIX, class Ld, class Fn = HmNothing>
+__device__ __forceinline__ void hm_fold(float4* eo, const DftMat& d, int tid, int nthr, Ld ld, Fn between = Fn()) {
   if constexpr (RADIX) {
     switch (d.p) {
       case 3: hm_fold_p<EVEN, INV, 3>(eo, d, tid, nthr, ld); break;
@@ -369,14 +371,19 @@ __device__ __forceinline__ void hm_fold(float4* eo, const DftMat& d, int tid, in
     return;
   }
   const int line = tid & 15, step = nthr >> 4;
-  for (int r0 = tid >> 4; r0 < d.Kp; r0 += 4 * step) {
-    float2 a[4], b[4];
+  float2 a[4], b[4];
+  auto load = [&](int r0) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int j = min(hm_pos<EVEN>(d, min(r0 + q * step, d.Kp - 1)), d.h);
       a[q] = ld(j, line);
       b[q] = ld(j == 0 ? 0 : d.n - j, line);
     }
+  };
+  load(tid >> 4);
+  between();
+  for (int r0 = tid >> 4; r0 < d.Kp; r0 += 4 * step) {
+    if (r0 != tid >> 4) load(r0);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const int r = r0 + q * step;
@@ -541,28 +548,49 @@ __device__ __forceinline__ LineConst line_const(const Tables& T, const OpDesc& o
 // happen in registers, and only the folded rows return to LDS.  The operator is
 // evaluated at every position's own wavenumber (the grids are mirror images only up
 // to rounding, and one ulp decides a mode at the evanescent cutoff).
-template <bool EVEN, int T_, bool RADIX, bool PRECISE>
+//
+// TABLE: all threads first evaluate the operator into LDS, while the line is on its way.
+// For one or two row tiles (n up to 126 even, 63 odd), where two or three of the four
+// waves have none and a lane evaluated 8 (odd n) or 16 positions one after the other:
+// 51x51x101 8.7 -> 6.7 us, 128x96x801 51.5 -> 44.2.  With four tiles it gains nothing
+// (120x101x301 25.1, 24.5 us), with three the LDS costs more (164 points: 61.9, 74.6).
+template <bool EVEN, int T_, bool RADIX, bool PRECISE, bool TABLE = false>
 __global__ __launch_bounds__(512) void k_gy_pass(float2* __restrict__ spec, Tables T, Geom g, DftMat d, OpDesc op) {
+  static_assert(!TABLE || (T_ == 1 && !RADIX));
   extern __shared__ float4 eo[];
+  float2* opt = reinterpret_cast<float2*>(eo + d.Kp * 16);  // TABLE: [position][line]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
   const int x = blockIdx.x / g.nfb, f0 = (blockIdx.x % g.nfb) * LF;
   const uint32_t syb = (uint32_t)g.MP * 8u;
   float2* base = spec + (long)x * g.nY * g.MP + f0;
-  hm_fold<EVEN, false, RADIX>(eo, d, tid, blockDim.x, [&](int pos, int line) { return gld(base, pos * syb + line * 8u); });
+  const int line = tid & 15, m = f0 + line;  // (blockDim.x is a multiple of 16)
+  const double kx = T.kx[x];
+  auto visit_at = [&](const LineConst& lc, int pos) {
+    const double kk = kperp2(kx, T.ky[pos]);
+    if constexpr (PRECISE) return visit_operator_fp64(op, kk, lc, m);
+    else return visit_operator(op, kk, lc, m);
+  };
+  auto ld = [&](int pos, int l) { return gld(base, pos * syb + l * 8u); };
+  if constexpr (TABLE) {
+    hm_fold<EVEN, false, RADIX>(eo, d, tid, blockDim.x, ld, [&] {
+      const LineConst lc = line_const(T, op, m);
+      for (int pos = tid >> 4; pos < d.n; pos += blockDim.x >> 4) opt[pos * 16 + line] = visit_at(lc, pos);
+    });
+  } else {
+    hm_fold<EVEN, false, RADIX>(eo, d, tid, blockDim.x, ld);
+  }
   __syncthreads();
   const Tiles t = hm_tiles(d.p * d.R, wave, W);
   LineAcc<EVEN> a[T_];
   hm_line<EVEN, T_, RADIX>(eo, d, t, lane, a);
   __syncthreads();
   {
-    const int line = lane & 15, m = f0 + line;
-    const LineConst lc = line_const(T, op, m);
-    const double kx = T.kx[x];
+    LineConst lc;
+    if constexpr (!TABLE) lc = line_const(T, op, m);
     auto apply = [&](int pos, float2 v) {
-      const double kk = kperp2(kx, T.ky[pos]);
       float2 o;
-      if constexpr (PRECISE) o = visit_operator_fp64(op, kk, lc, m);
-      else o = visit_operator(op, kk, lc, m);
+      if constexpr (TABLE) o = opt[pos * 16 + line];
+      else o = visit_at(lc, pos);
       return cmul_tw<false>(v, make_float4(o.x, o.y, d.norm_lo * o.x, d.norm_lo * o.y));
     };
     // folded row of output k of residue r from the values at k and q - k

@@ -108,6 +108,14 @@ void gen_xinv(int epi, float2* spec, const Tables& T, const Geom& g, const DftMa
 void gen_ypass(float2* spec, const Tables& T, const Geom& g, const DftMat& d, const OpDesc& op, hipStream_t s) {
   const dim3 grid(g.nX * g.nfb), block(64 * line_waves(d));
   const size_t lds = line_lds(d);
+  if (d.p == 1 && d.R <= 2) {  // the operator from a table in LDS (see k_gy_pass)
+    auto launch = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, block, lds + (size_t)d.n * 16 * sizeof(float2), s, spec, T, g, d, op);
+    };
+    if (op.precise) d.even ? launch(k_gy_pass<true, 1, false, true, true>) : launch(k_gy_pass<false, 1, false, true, true>);
+    else d.even ? launch(k_gy_pass<true, 1, false, false, true>) : launch(k_gy_pass<false, 1, false, false, true>);
+    return;
+  }
   if (op.precise) DISPATCH_TILES(d, hipLaunchKernelGGL((k_gy_pass<EVEN, T_, RADIX, true>), grid, block, lds, s, spec, T, g, d, op));
   else DISPATCH_TILES(d, hipLaunchKernelGGL((k_gy_pass<EVEN, T_, RADIX, false>), grid, block, lds, s, spec, T, g, d, op));
 }

@@ -26,6 +26,11 @@ SHAPES = [(2, 3, 4), (3, 2, 5), (15, 16, 7), (17, 31, 15), (32, 33, 31), (30, 34
           # lines that take a radix 3, 5, 7 or 9 first, odd and even quotients
           (129, 132, 5), (135, 130, 6), (133, 140, 5), (252, 245, 4), (365, 366, 4), (385, 147, 5), (990, 7, 6),
           (7, 1001, 5), (1008, 4, 6),
+          # y passes that take the operator from a table: one and two row tiles, and the
+          # first length past them
+          (5, 60, 9), (3, 62, 6), (3, 64, 5), (7, 124, 18), (5, 126, 6), (4, 61, 33),
+          # y passes with a power-of-two or 3 2^k line: one x row a block up to 768 pairs, else two
+          (46, 64, 1024), (48, 64, 1024), (2, 384, 256), (2, 192, 512), (6, 128, 256),
           # and columns (with 16 columns to a block, some blocks partly filled)
           (5, 4, 129), (4, 5, 130), (3, 7, 133), (5, 5, 135), (6, 5, 189), (7, 5, 252), (5, 7, 300), (4, 5, 301),
           (5, 9, 425), (4, 4, 510), (3, 5, 513), (5, 4, 801), (4, 5, 1010), (3, 6, 1022), (5, 4, 1035), (4, 5, 1200),
