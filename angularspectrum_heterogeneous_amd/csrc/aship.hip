@@ -549,7 +549,11 @@ void launch_xfwd_L(ash_plan* p, hipStream_t s) {
 }
 template <int L>
 void launch_ypass_L(ash_plan* p, const OpDesc& op, hipStream_t s) {
-  const dim3 grid((p->g.nX / 2) * (p->g.MP / ypass_lines<L>()));  // one block per (x row pair, f group)
+  // one block per (x row pair, f group); up to three of them a CU, one per row: the chip
+  // is latency bound there (a step at 64x64x256 85.5 -> 80.6 us, 128x128x256 181.9 ->
+  // 177.2, but 128x128x512, of 1088 pairs, 211 -> 216)
+  const int pairs = (p->g.nX / 2) * (p->g.MP / ypass_lines<L>());
+  const dim3 grid(pairs <= 768 ? 2 * pairs : pairs);
   // the FP64-operator reference runs with the default radix order
   if (op.precise) hipLaunchKernelGGL((k_ypass<L, true, 0>), grid, dim3(ypass_threads<L, 0>()), 0, s, p->spec, p->T, p->g, op);
   else if (p->rvy) hipLaunchKernelGGL((k_ypass<L, false, 1>), grid, dim3(ypass_threads<L, 1>()), 0, s, p->spec, p->T, p->g, op);

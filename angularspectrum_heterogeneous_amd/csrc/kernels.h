@@ -355,7 +355,7 @@ template <int L, int V> constexpr int ypass_threads() { return (L == 256 && V ==
 // positions y and nY-1-y the same ky^2.  The operator depends on (kx, ky)
 // only through kk = kx^2 + ky^2, so one block evaluates it once per
 // (|ky| index, f bin) into an LDS table and applies it to both rows: a
-// quarter of one evaluation per element.
+// quarter of one evaluation per element.  (On small grids a block takes one row.)
 template <int L, bool PRECISE, int V>
 __global__ __launch_bounds__((ypass_threads<L, V>())) void k_ypass(float2* __restrict__ spec, Tables T, Geom g, OpDesc op) {
   constexpr int H = L / 2;
@@ -367,7 +367,9 @@ __global__ __launch_bounds__((ypass_threads<L, V>())) void k_ypass(float2* __res
   __shared__ LineConst slc[LFY];
   const int tid = threadIdx.x;
   const int nfb = g.MP / LFY;
-  const int ip = blockIdx.x / nfb, fb = blockIdx.x % nfb;
+  const int bx = blockIdx.x / nfb, fb = blockIdx.x % nfb;
+  const int rows = (int)gridDim.x > g.nX / 2 * nfb ? 1 : 2;  // x rows of this block
+  const int ip = min(bx, g.nX - 1 - bx);  // the operator's row: the lower of the pair
   const int f0 = fb * LFY;
   const uint32_t syb = (uint32_t)g.MP * 8u;  // y stride in bytes
   // lines past the Nyquist bin (padding, f > M) are transformed like the others
@@ -414,7 +416,7 @@ __global__ __launch_bounds__((ypass_threads<L, V>())) void k_ypass(float2* __res
       }
     }
   };
-  prefetch(ip);
+  prefetch(bx);
   {
     const double kx = T.kx[ip];
     // entry e = tid + NTY k is on line e % LF = myline
@@ -428,13 +430,13 @@ __global__ __launch_bounds__((ypass_threads<L, V>())) void k_ypass(float2* __res
   }
   // the table is read after the barriers of the forward transform
 #pragma unroll 1
-  for (int h = 0; h < 2; ++h) {
+  for (int h = 0; h < rows; ++h) {
     // an opaque copy of the thread index per row: without it the compiler
     // keeps every thread-dependent LDS address and twiddle of both transforms
     // live across the rows (~70 more VGPRs, one block fewer per CU)
     int t = tid;
     asm volatile("" : "+v"(t));
-    const int x = h == 0 ? ip : g.nX - 1 - ip;
+    const int x = h == 0 ? bx : g.nX - 1 - bx;
     float2* base = spec + (long)x * g.nY * g.MP + f0;
     int k = 0;  // the first pass asks for its elements in prefetch order
     auto ld = [&](int line, int pos) -> float2 {
@@ -445,7 +447,7 @@ __global__ __launch_bounds__((ypass_threads<L, V>())) void k_ypass(float2* __res
     // pass 0 stores to LDS only after its barrier, which follows every read of
     // the previous row's last pass
     fft_run<L, false, NTY, LFY, LY, V>(buf, tw, t, ld, st_lds);
-    if (h == 0) prefetch(g.nX - 1 - ip);
+    if (h + 1 < rows) prefetch(g.nX - 1 - bx);
     auto ld_op = [&](int line, int pos) -> float2 {
       const int i = pos < H ? pos : L - 1 - pos;
       return cmul(buf[LY::idx(line, pos)], opt[i * LFY + line]);
