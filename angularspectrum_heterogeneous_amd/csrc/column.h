@@ -360,7 +360,8 @@ __device__ __forceinline__ void column_realspace(float (&u)[S], const LaneCol<S,
         }
       }
     }
-    if (MODE == COL_RAWNL && live) L.store(d.rout + (long)c * L.nT, u);
+    // (a bounded column's caller stores it)
+    if (MODE == COL_RAWNL && !BOUNDED && live) L.store(d.rout + (long)c * L.nT, u);
   } else if constexpr (FIN) {
     // (padding samples of a bounded lane are zero: they add nothing to e2 but are
     // kept out of the extrema)

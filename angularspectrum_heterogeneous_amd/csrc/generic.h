@@ -1369,13 +1369,16 @@ __global__ __launch_bounds__(64 * gcol_waves(S), gcol_waves_per_simd(S, RADIX, M
 }
 
 // Nonlinear update of real columns of any length (COL_RAWNL, no transform): one wave
-// per column, lane ln holds the S contiguous samples from S ln.
+// per column, lane ln holds the S contiguous samples from S ln.  Columns pass through
+// LDS, so that memory sees whole rows (128x96x801: 72 -> 17-25 us, KT 55).
 constexpr int GR_WPB = 4;
 template <int S, int NLK>
 __global__ __launch_bounds__(64 * GR_WPB) void k_gcolumn_raw(Tables T, Geom g, ColDesc d) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int nT = g.nT, ncols = g.nX * g.nY, t0 = lane * S;
   const LaneCol<S, 64, false, true> lc{lane, lane, t0, nT};
+  __shared__ float rows[GR_WPB][64 * (S + 1)];  // sample t at t + t/S: a lane's samples start in its own bank
+  float* row = rows[wave];
   const double Nn = d.nscale ? d.N * (d.nscale[0] / (d.nscale[1] + 1e-30)) : d.N;
   float wmax = 0.f;
   int nsub_global = 1;
@@ -1392,8 +1395,26 @@ __global__ __launch_bounds__(64 * GR_WPB) void k_gcolumn_raw(Tables T, Geom g, C
     const float* src = d.rin + (long)c * nT;
     float u[S];
 #pragma unroll
-    for (int i = 0; i < S; ++i) u[i] = (t0 + i < nT) ? src[t0 + i] : 0.f;
+    for (int i = 0; i < S; ++i) {
+      const int t = lane + 64 * i;
+      u[i] = t < nT ? src[t] : 0.f;
+    }
+#pragma unroll
+    for (int i = 0; i < S; ++i) row[lane + 64 * i + (lane + 64 * i) / S] = u[i];
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < S; ++i) u[i] = row[t0 + i + lane];
     column_realspace<S, 64, false, true, COL_RAWNL, NLK>(u, lc, d, T, c, true, ncols, 0, Nn, nsub_global, wmax);
+    float* dst = d.rout + (long)c * nT;
+#pragma unroll
+    for (int i = 0; i < S; ++i) row[t0 + i + lane] = u[i];
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < S; ++i) {
+      const int t = lane + 64 * i;
+      if (t < nT) dst[t] = row[t + t / S];
+    }
+    wave_sync();
   }
 }
 

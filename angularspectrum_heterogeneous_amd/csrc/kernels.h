@@ -912,7 +912,15 @@ static __global__ __launch_bounds__(256) void k_absmax_cols(const float* __restr
   const long c1 = c0 + ABSMAX_COLS < ncols ? c0 + ABSMAX_COLS : ncols;
   const long e0 = c0 * nT, e1 = c1 * nT;
   unsigned m = 0u;
-  for (long e = e0 + threadIdx.x; e < e1; e += 256) m = max(m, __float_as_uint(fabsf(u[e])));
+  long e = e0 + threadIdx.x;
+  for (; e + 7 * 256 < e1; e += 8 * 256) {  // eight loads in flight (128x96x801: 50 us with one, 12 so)
+    float v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) v[q] = u[e + q * 256];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) m = max(m, __float_as_uint(fabsf(v[q])));
+  }
+  for (; e < e1; e += 256) m = max(m, __float_as_uint(fabsf(u[e])));
   for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned)__shfl_xor((int)m, o, 64));
   if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = m;
   __syncthreads();

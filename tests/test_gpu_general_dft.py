@@ -88,3 +88,22 @@ def test_general_columns_do_not_mix():
     keep[1, 2] = False
     assert np.array_equal(got[keep], want[keep])
     assert rel_l2(want, u) < 2e-6
+
+
+@pytest.mark.parametrize("nT", [7, 63, 65, 129, 257, 300, 513, 801, 1025, 2047])
+def test_raw_columns_move_through_lds_whole(nT):
+    """The nonlinear step of real columns around every samples-per-lane class: against the
+    oracle (the operator tests' 1e-6: a few float32 operations a sample), in place, and the
+    peak of the field to the last bit."""
+    from angularspectrum_heterogeneous_amd import _lib
+    shape = (5, 27, nT)  # 135 columns: three blocks of the peak, the last partly filled
+    p = _params(shape)
+    N, dz = p.beta / (2 * p.c0 ** 3 * p.rho0), 3.08e-4
+    plan = _plan(shape, p, dz)
+    u = _field(shape, p0=3e6)
+    got = plan.nonlinear_step(_dev(u), _lib.NL_RUSANOV, dz)
+    assert rel_l2(got.cpu().numpy(), O.rusanov_flux_standard(u.astype(np.float64), N, dz, p.dT)) < 1e-6
+    x = _dev(u)
+    plan.nonlinear_step(x, _lib.NL_RUSANOV, dz, out=x)
+    assert np.array_equal(x.cpu().numpy(), got.cpu().numpy())
+    assert plan.max_abs(_dev(u)) == float(np.abs(u).max())
