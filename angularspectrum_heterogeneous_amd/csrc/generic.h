@@ -24,9 +24,9 @@
 // Per element of a complex line that is 2n flops (odd n) or n (even n): at
 // 365x365x425 an x sweep does 20.7 GFLOP over 454 MB, so the matrix cores bound it
 // above n of about 200 and memory below.  There, against the direct sums through LDS
-// (a vector fma and two LDS reads per term): x sweep 2217 -> 293 us, y pass 5145 ->
-// 541 us, KT column pass 5736 -> 743 us; at 193x193x1201 the KT column pass 17.7 ->
-// 2.4 ms.
+// (a vector fma and two LDS reads per term): x sweep 2217 -> 211 us, y pass 5145 ->
+// 485 us before the radix, KT column pass 5736 -> 613 us and 451 with it; at
+// 193x193x1201, whose 1201 is prime, the KT column pass 17.7 -> 1.42 ms.
 #pragma once
 #include "column.h"
 
@@ -760,8 +760,9 @@ static __global__ __launch_bounds__(256) void k_gy_sa(float2* __restrict__ spec,
 // Per sample that is nT flops per transform (odd nT) or nT/2 (even), a p-th of it after a
 // radix stage.  Without one the matrix cores bound the pass (96 TFLOP/s at nT = 1201);
 // with one the vector work between the products does (at 365x365x425 the taper pass
-// takes 374 us, 613 without the radix 5, of which the products are about 80).  The row pitch is an odd multiple of 8 floats: the 16 columns x 4
-// positions of an operand read fall in distinct banks.
+// takes 363 us, 613 without the radix 5, of which the products are about 80).  The row
+// pitch is an odd multiple of 8 floats: the 16 columns x 4 positions of an operand read
+// fall in distinct banks.
 // ---------------------------------------------------------------------------
 constexpr int GC_COLS = 16;
 constexpr int gcol_waves(int S) { return S == 2 ? 4 : 8; }
